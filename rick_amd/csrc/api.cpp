@@ -192,6 +192,7 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
     const uint64_t nb = (uint64_t)g.planes * g.tiles_u * g.tiles_v;
     if (nb >= (1ull << 31)) return set_error(RICK_ERR_INVALID, "too many grid tiles");
     g.nb = (uint32_t)nb;
+    g.cshift = counter_shift(g.nb);
     g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task : 4096u;
     g.ntable = kTableOversample * d.w_support;
     // ~64-128 KB of grid per zero task measured best (LOFAR-like grid).
@@ -456,14 +457,14 @@ int rick_plan_image(rick_plan p, unsigned int n, unsigned int F, unsigned int P,
         return RICK_OK;
     }
     // Sparse grid: tiles of empty buckets are left unwritten; the row FFT
-    // reads only occupied tiles (bucket counts) and treats the rest as zero.
+    // reads only occupied tiles (bucket offsets) and treats the rest as zero.
     // (A row of more than 256 tiles exceeds the row FFT's occupancy table;
     // such grids are cleared densely instead.)
     const bool sparse = p->geom.nx / p->geom.tu <= 256;
     RICK_HIP(launch_grid(p->geom, p->work, p->d.precision, p->table_d, n, F, P, uu, vv, ww, vr,
                          vi, wt, grid, 0, s, &p->timing, !sparse));
     RICK_HIP(launch_image_chain(p->fft, p->d.precision, grid, norm, s, &p->timing,
-                                sparse ? &p->geom : nullptr, sparse ? p->work.counts : nullptr,
+                                sparse ? &p->geom : nullptr, sparse ? p->work.offsets : nullptr,
                                 sparse ? p->work.rowlive : nullptr, p->phase, re, im));
     return RICK_OK;
 }
@@ -620,7 +621,7 @@ int rick_batch_run(rick_batch b, void *stream)
                          &p->timing, !sparse, b->jobs_d, b->njobs));
     const double norm = 1.0 / (double)((double)p->geom.nx * (double)p->geom.ny);
     RICK_HIP(launch_image_chain(p->fft, p->d.precision, b->grid, norm, s, &p->timing,
-                                sparse ? &p->geom : nullptr, sparse ? p->work.counts : nullptr,
+                                sparse ? &p->geom : nullptr, sparse ? p->work.offsets : nullptr,
                                 sparse ? p->work.rowlive : nullptr, p->phase, nullptr, nullptr,
                                 b->pjobs_d, b->njobs));
     return RICK_OK;

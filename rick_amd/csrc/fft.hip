@@ -353,17 +353,22 @@ constexpr int lds_elems(int L, bool rows)
 // Occupancy flags per workgroup: G rows x (L/32) tiles of >= 32 cells.
 constexpr int oc_bytes(int L) { return lines_per_wg(L) * (L / 32 > 0 ? L / 32 : 1); }
 
-// Occupancy of a sparse grid: counts of the gridder bucket (plane, tile row,
-// tile column), zero where the tile was never written, and rows[plane * ny +
-// v], non-zero iff grid row v of the plane holds a non-zero cell.  The row
+// Occupancy of a sparse grid: record offsets of the gridder buckets (plane,
+// tile row, tile column), a bucket's offset equal to the next one's where the
+// tile was never written, and rows[plane * ny + v], non-zero iff grid row v of the plane holds a non-zero cell.  The row
 // transform skips the other rows (writes nothing) and later column passes
 // read them as zero.
 struct Occupancy {
-    const uint32_t *counts;
+    const uint32_t *offsets;
     const unsigned char *rows;
     int tv, tiles_u, tiles_v, ny;
     int tu_shift;   // log2 of the tile width (a power of two)
 };
+
+__device__ __forceinline__ bool tile_occupied(const Occupancy &oc, size_t bucket)
+{
+    return oc.offsets[bucket] != oc.offsets[bucket + 1];
+}
 
 // Row flags of the grid for the column kernels (null: dense input).
 struct ColOcc {
@@ -385,7 +390,7 @@ __device__ __forceinline__ void col_rowlive(const ColOcc &co, int plane, int row
 }
 
 // Rows: workgroup w handles rows w*G .. w*G+G-1 of the planes*ny rows.
-// MASK (one row per workgroup, bucket counts of at most 64 tiles per row):
+// MASK (one row per workgroup, at most 64 tiles per row):
 // the row's tile occupancy is a bit mask in scalar registers, so the test of
 // each loaded element compiles to a shift and a select.
 template <typename T, int L, int E, bool MASK>
@@ -419,13 +424,13 @@ k_fft_rows(int rows_total, const C2<T> *__restrict__ tw, const C2<T> *gin, C2<T>
         // table or barrier is needed.  A row without a non-zero cell is zero
         // and is neither computed nor written.
         if (oc.rows && !oc.rows[row0]) return;
-        // Every wave reads the row's (at most 64) tile counts, one per lane;
-        // the ballot is the occupancy bit mask.
+        // Every wave tests the row's (at most 64) tiles, one per lane; the
+        // ballot is the occupancy bit mask.
         const int plane = (int)(row0 / oc.ny), v = (int)(row0 % oc.ny);
         const int t = threadIdx.x & 63;
         const bool occd =
             t < oc.tiles_u &&
-            oc.counts[((size_t)plane * oc.tiles_v + v / oc.tv) * oc.tiles_u + t] != 0;
+            tile_occupied(oc, ((size_t)plane * oc.tiles_v + v / oc.tv) * oc.tiles_u + t);
         ln.occ_mask = __ballot(occd);
         ln.occ_mask_on = true;
         ln.occ_shift = oc.tu_shift;
@@ -436,14 +441,14 @@ k_fft_rows(int rows_total, const C2<T> *__restrict__ tw, const C2<T> *gin, C2<T>
         for (int g = threadIdx.x; g < ln.nvalid; g += NT) live |= oc.rows[row0 + g];
         if (!__syncthreads_or(live)) return;
     }
-    if (!MASK && oc.counts) {
+    if (!MASK && oc.offsets) {
         for (int i = threadIdx.x; i < G * oc.tiles_u && oc.tiles_u <= MAXT; i += NT) {
             const int g = i / oc.tiles_u, t = i % oc.tiles_u;
             const size_t row = row0 + g;
             unsigned char live = 0;
             if (g < ln.nvalid && (oc.rows == nullptr || oc.rows[row])) {
                 const int plane = (int)(row / oc.ny), v = (int)(row % oc.ny);
-                live = oc.counts[((size_t)plane * oc.tiles_v + v / oc.tv) * oc.tiles_u + t] != 0;
+                live = tile_occupied(oc, ((size_t)plane * oc.tiles_v + v / oc.tv) * oc.tiles_u + t);
             }
             occ[i] = live;
         }
@@ -709,7 +714,7 @@ hipError_t launch_rows(int L, int rows_total, const C2<T> *tw, const C2<T> *in, 
         constexpr int G = lines_per_wg(LL);                                                \
         constexpr int E = row_values<T>();                                                 \
         if constexpr (G == 1) {                                                            \
-            if (oc.counts && oc.tiles_u <= 64) {                                           \
+            if (oc.offsets && oc.tiles_u <= 64) {                                           \
                 hipLaunchKernelGGL((k_fft_rows<T, LL, E, true>), dim3(rows_total),         \
                                    dim3(LL / E), 0, s, rows_total, tw, in, out, scale, oc); \
                 return hipGetLastError();                                                  \
@@ -843,7 +848,7 @@ hipError_t image_chain_impl(const FftPlan &p, void *grid_v, double scale_d, hipS
     const CT *twy = static_cast<const CT *>(p.tw_y);
     const int nx = p.nx, ny = p.ny, planes = p.planes;
     ColOcc co{};
-    if (oc.counts && oc.rows) {
+    if (oc.offsets && oc.rows) {
         co.rows = oc.rows;
         co.ny = ny;
     }
@@ -901,7 +906,7 @@ hipError_t launch_fft(const FftPlan &p, int precision, const void *in, void *out
 
 hipError_t launch_image_chain(const FftPlan &p, int precision, void *grid, double scale,
                               hipStream_t s, Timing *tm, const GridGeom *occ_geom,
-                              const uint32_t *occ_counts, const unsigned char *occ_rows,
+                              const uint32_t *occ_offsets, const unsigned char *occ_rows,
                               const PhaseGeom &pg,
                               double *re, double *im, const PhaseJob *jobs, int njobs)
 {
@@ -909,10 +914,10 @@ hipError_t launch_image_chain(const FftPlan &p, int precision, void *grid, doubl
     if (tm == nullptr) tm = &off;
     Occupancy oc{};
     if (occ_geom) {
-        if (!occ_counts || p.nx / occ_geom->tu > 256 || occ_geom->tu <= 0 ||
+        if (!occ_offsets || p.nx / occ_geom->tu > 256 || occ_geom->tu <= 0 ||
             (occ_geom->tu & (occ_geom->tu - 1)) != 0)
             return hipErrorInvalidValue;
-        oc.counts = occ_counts;
+        oc.offsets = occ_offsets;
         oc.rows = occ_rows;
         oc.tu_shift = __builtin_ctz((unsigned)occ_geom->tu);
         oc.tv = occ_geom->tv;

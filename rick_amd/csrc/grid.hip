@@ -73,6 +73,16 @@ constexpr uint32_t kSplitTask = 3u;           // task.w of a split bucket's task
 constexpr int kTileThreads = 512;
 constexpr int kLdsBytes = 160 * 1024;         // LDS per CU
 constexpr uint32_t kPersistSlots = 64;        // task slots per resident workgroup to persist
+// Device-scope atomics on one 128-byte line are performed one after the other,
+// and neighbouring buckets are the ones hit together: with packed counters the
+// scatter's returning atomics took two thirds of its time.  A bucket's counters
+// are 2^6 words apart while all of them fit 2^21 words (8 MB), closer in larger
+// grids, where the traffic spreads over more buckets.  Scatter, packed against
+// spread: 516 k rows on 512^2 x 8 planes 47 -> 19 us, 3 M rows on 2048^2 x 12
+// 213 -> 118 us, 7.7 M rows of 16 channels on 4096^2 x 32 428 -> 368 us; 2^5
+// words and 2^20 in all measured 20 / 119 / 382 us, 2^3 words 22 / 154 / 389 us.
+constexpr int kCounterShiftMax = 6;
+constexpr uint64_t kCounterWords = 1u << 21;
 constexpr int kPadU = 8;  // LDS row padding (elements): rows shift by 8 banks
 
 struct RecF64 {
@@ -197,6 +207,13 @@ __device__ __forceinline__ int row_keys(const GridGeom &g, const Foot &f, uint32
     return n;
 }
 
+// A bucket's counters (histogram and scatter cursor) lie 2^g.cshift words
+// apart, see counter_shift().
+__device__ __forceinline__ size_t counter_at(const GridGeom &g, uint32_t b)
+{
+    return (size_t)b << g.cshift;
+}
+
 // LDS open-addressing hash set of 2^HB bucket keys with at most kMaxProbe
 // probes: returns the key's slot, or kEmpty when none was free on its path.
 template <int HB>
@@ -283,7 +300,7 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
                 const int nk = row_keys(g, f, keys);
                 for (int q = 0; q < nk; ++q) {
                     const uint32_t h = hinsert_peek<kBinHashBits>(hkey, keys[q]);
-                    if (h == kEmpty) atomicAdd(&counts[keys[q]], 1u);
+                    if (h == kEmpty) atomicAdd(&counts[counter_at(g, keys[q])], 1u);
                     else atomicAdd(&hcnt[h], 1u);
                 }
             }
@@ -292,7 +309,7 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
     __syncthreads();
     for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) {
         const uint32_t c = hcnt[i];
-        if (c) atomicAdd(&counts[hkey[i]], c);
+        if (c) atomicAdd(&counts[counter_at(g, hkey[i])], c);
     }
 }
 
@@ -339,7 +356,7 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k < nv) {
-            c[k] = counts[b0 + k];
+            c[k] = counts[counter_at(g, b0 + k)];
             r += c[k];
             sp += c[k] > g.rmax ? 1u : 0u;
             ne += c[k] > 0 ? 1u : 0u;
@@ -426,7 +443,7 @@ k_scan_down(GridGeom g, const uint32_t *__restrict__ counts,
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k < nv) {
-            c[k] = counts[b0 + k];
+            c[k] = counts[counter_at(g, b0 + k)];
             v[0] += c[k];
             v[2] += c[k] > g.rmax ? 1u : 0u;
         }
@@ -454,7 +471,7 @@ k_scan_down(GridGeom g, const uint32_t *__restrict__ counts,
     for (int k = 0; k < nv; ++k) {
         const uint32_t b = b0 + k;
         offsets[b] = ro;
-        cursor[b] = ro;
+        cursor[counter_at(g, b)] = ro;
         if (c[k] == 0) {
             // Every zrun-th bucket of a run of empty ones starts a zero task.
             if (zero && run % g.zrun == 0) {
@@ -731,7 +748,7 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
     for (int t = 0; t < kSlotsPerThread; ++t) {
         const int i = threadIdx.x + t * kScatterThreads;
         const uint32_t c = hcnt[i];
-        got[t] = c ? atomicAdd(&cursor[hkey[i]], c) : 0u;
+        got[t] = c ? atomicAdd(&cursor[counter_at(g, hkey[i])], c) : 0u;
     }
 #pragma unroll
     for (int t = 0; t < kSlotsPerThread; ++t) hbase[threadIdx.x + t * kScatterThreads] = got[t];
@@ -743,7 +760,7 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
             if (q < nk[k]) {
                 const uint32_t it = item[k][q];
                 const uint32_t pos = (it & kDirect)
-                                         ? atomicAdd(&cursor[it & ~kDirect], 1u)
+                                         ? atomicAdd(&cursor[counter_at(g, it & ~kDirect)], 1u)
                                          : hbase[it & (kHashSlots - 1)] + (it >> kHashBits);
                 typename RecOf<PREC>::type r;
                 r.pu = pu[k];
@@ -1257,6 +1274,13 @@ void capacities(const GridGeom &g, uint32_t max_points, uint32_t *rec_cap, uint3
 
 }  // namespace
 
+int counter_shift(uint32_t nb)
+{
+    int shift = 0;
+    while (shift < kCounterShiftMax && ((uint64_t)nb << (shift + 1)) <= kCounterWords) ++shift;
+    return shift;
+}
+
 uint32_t batch_row_align() { return (uint32_t)kBinRows; }
 
 const char *grid_launch_limit(const GridGeom &g, uint32_t max_points)
@@ -1281,9 +1305,9 @@ size_t grid_work_bytes(const GridGeom &g, uint32_t max_points, int precision)
     capacities(g, max_points, &rec_cap, &split_cap, &task_cap, &nscan);
     const size_t rs = precision == RICK_FP64 ? sizeof(RecF64) : sizeof(RecF32);
     size_t b = 0;
-    b += align_up(sizeof(uint32_t) * g.nb, 256);           // counts
+    b += align_up((sizeof(uint32_t) * g.nb) << g.cshift, 256);   // counts
     b += align_up((size_t)g.planes * g.ny, 256);           // rowlive (after the counts)
-    b += align_up(sizeof(uint32_t) * g.nb, 256);           // cursor
+    b += align_up((sizeof(uint32_t) * g.nb) << g.cshift, 256);   // cursor
     b += align_up(sizeof(uint32_t) * (g.nb + 1), 256);     // offsets
     b += align_up(sizeof(uint32_t) * kScanQ * nscan, 256); // blocksum
     b += align_up(sizeof(uint4) * task_cap, 256);          // tasks
@@ -1309,9 +1333,9 @@ void grid_work_carve(const GridGeom &g, uint32_t max_points, int precision, void
         p += align_up(bytes, 256);
         return q;
     };
-    w->counts = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * g.nb));
+    w->counts = reinterpret_cast<uint32_t *>(take((sizeof(uint32_t) * g.nb) << g.cshift));
     w->rowlive = reinterpret_cast<unsigned char *>(take((size_t)g.planes * g.ny));
-    w->cursor = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * g.nb));
+    w->cursor = reinterpret_cast<uint32_t *>(take((sizeof(uint32_t) * g.nb) << g.cshift));
     w->offsets = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * (g.nb + 1)));
     w->blocksum = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * kScanQ * nscan));
     w->tasks = reinterpret_cast<uint4 *>(take(sizeof(uint4) * task_cap));

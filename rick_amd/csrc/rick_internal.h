@@ -108,6 +108,7 @@ struct GridGeom {
     int tu_shift, tv_shift; // log2(tu), log2(tv)
     int tiles_u, tiles_v;   // tiles per axis
     uint32_t nb;            // buckets = planes*tiles_u*tiles_v
+    int cshift;             // log2 words between consecutive buckets' counters
     uint32_t rmax;          // rows per task
     int ntable;
     double cmax;            // largest per-cell convolution weight (a bound)
@@ -129,8 +130,8 @@ inline double exact_inverse(double d)
 
 // Workspace of the binned gridder, carved out of one device allocation.
 struct GridWork {
-    uint32_t *counts;       // [nb]  records per bucket
-    uint32_t *cursor;       // [nb]  scatter cursor (starts at the bucket offset)
+    uint32_t *counts;       // [nb << cshift] records per bucket
+    uint32_t *cursor;       // [nb << cshift] scatter cursor (starts at the bucket offset)
     uint32_t *offsets;      // [nb+1] exclusive scan of counts
     uint32_t *blocksum;     // [5*nscan] per scan block: records, accumulation tasks, split,
                             //   non-empty, zero tasks
@@ -166,6 +167,8 @@ struct BatchJob {
     int plane0, planes;     // the job's planes in the group's plane stack
     double dw, inv_dw;      // inv_dw: exact_inverse(dw)
 };
+// log2 of the words between the counters of consecutive buckets.
+int counter_shift(uint32_t nb);
 // Rows per block of the count kernel: batch jobs start at multiples of it.
 uint32_t batch_row_align();
 
@@ -241,8 +244,9 @@ hipError_t launch_phase(const PhaseGeom &p, int precision, const void *gridss, d
                         double *im, int accumulate, hipStream_t s, Timing *tm);
 
 // Image chain after gridding, in place on grid (clobbered) and without
-// scratch: row FFT reading only the tiles whose gridder bucket count
-// (occ_counts, geometry occ_geom; null: dense grid) is non-zero and skipping
+// scratch: row FFT reading only the tiles whose gridder bucket holds records
+// (occ_offsets, the scan of the bucket counts, geometry occ_geom; null: dense
+// grid) and skipping
 // grid rows whose flag in occ_rows (planes*ny, written by the tile kernel) is
 // zero, column FFT whose last pass is fused with the phase correction and plane sum
 // into the images (overwritten).  Scales by `scale` (1/(Nx*Ny)).
@@ -257,7 +261,7 @@ struct PhaseJob {
 };
 hipError_t launch_image_chain(const FftPlan &p, int precision, void *grid, double scale,
                               hipStream_t s, Timing *tm, const GridGeom *occ_geom,
-                              const uint32_t *occ_counts, const unsigned char *occ_rows,
+                              const uint32_t *occ_offsets, const unsigned char *occ_rows,
                               const PhaseGeom &pg, double *re, double *im,
                               const PhaseJob *jobs = nullptr,
                               int njobs = 0);
