@@ -162,8 +162,8 @@ int rick_plan_phase(rick_plan plan, const void *gridss, double *image_real,
  * recorded work and returns, per stage, the summed kernel time (ms) and the
  * number of launches since the previous query, then resets. */
 enum {
-    RICK_STAGE_COUNT_ROWS = 0, /* bucket histogram (incl. clearing it)        */
-    RICK_STAGE_SCAN = 1,       /* bucket / task offsets                        */
+    RICK_STAGE_COUNT_ROWS = 0, /* bucket histogram                             */
+    RICK_STAGE_SCAN = 1,       /* bucket / task offsets, clearing the counters */
     RICK_STAGE_SCATTER = 2,    /* per-row channel sums -> sorted records       */
     RICK_STAGE_ZERO = 3,       /* reserved: empty tiles are cleared by zero    */
                                /* tasks inside stage 4                         */
@@ -172,7 +172,8 @@ enum {
     RICK_STAGE_FFT_COLS_B = 6, /* column FFT four-step B                       */
     RICK_STAGE_FFT_ROWS = 7,   /* row FFT (+ 1/(Nx*Ny))                         */
     RICK_STAGE_PHASE = 8,      /* phase correction + plane sum                 */
-    RICK_STAGE_ZERO_SPLIT = 9, /* clear tiles of split buckets                 */
+    RICK_STAGE_ZERO_SPLIT = 9, /* reserved: split buckets' tiles are cleared   */
+                               /* inside stage 2                               */
     RICK_STAGE_COUNT = 10
 };
 int rick_plan_profile(rick_plan plan, int enable);

@@ -13,14 +13,14 @@
 //                histogram: device-scope atomics are slow on this chip (its
 //                eight L2 slices are not coherent with each other), and 16384
 //                consecutive rows touch a few thousand distinct buckets.
-//   k_scan_*     multi-block exclusive scans of the histogram -> bucket
-//                offsets, the task list (a task is <= rmax records of one
+//   k_scan_*     exclusive scans of the histogram -> bucket offsets, the task list (a task is <= rmax records of one
 //                bucket, or a zero task), the list of split buckets.
 //   k_scatter    forms per row S = sum_{f,p} fl32(weight*vis) (NaN real parts
 //                skipped, w-stacking.cu:517) and writes a record {pos_u,
 //                pos_v, S} to each of its buckets; slots come from one
 //                returning global atomic per distinct key per 2048-row block.
-//   k_zero_split clears the tiles of split buckets (overwrite mode).
+//                Its last workgroups clear the tiles of split buckets
+//                (overwrite mode).
 //   k_tile       one workgroup per task: accumulates its records into an FP64
 //                LDS tile (one lane per record, LDS atomics), then writes
 //                the tile once with plain, coalesced stores; tasks of split
@@ -39,6 +39,7 @@
 // rounding order (identical when F*P == 1).
 #include "rick_internal.h"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -59,17 +60,16 @@ constexpr int kRowsPerBlock = kScatterThreads * kRowsPerThread;
 constexpr int kHashBits = 12;
 constexpr int kHashSlots = 1 << kHashBits;
 constexpr uint32_t kDirect = 0x80000000u;     // item flag: key without a hash slot
-// Count: 16384-row blocks, 8192-slot hash with bounded probing, overflow ->
-// direct global atomic.
+// Count: blocks of 1, 4 or 16 rows per thread (count_rows_per_thread) with a
+// hash of half as many slots as rows (at least 2048) and bounded probing;
+// overflow -> direct global atomic.
 constexpr int kBinThreads = 1024;
-constexpr int kBinRowsPerThread = 16;
-constexpr int kBinRows = kBinThreads * kBinRowsPerThread;
+constexpr int kBinRows = kBinThreads * 16;    // largest count block; batch jobs start at multiples
 static_assert(kBinRows % kRowsPerBlock == 0, "a scatter block must not span two batch jobs");
-constexpr int kBinHashBits = 13;
-constexpr int kBinSlots = 1 << kBinHashBits;
 constexpr int kMaxProbe = 32;
 constexpr uint32_t kZeroTask = 2u;            // task.w of a zero task
 constexpr uint32_t kSplitTask = 3u;           // task.w of a split bucket's task: 3 + split slot
+constexpr uint32_t kZeroBlocks = 64;          // scatter workgroups clearing split buckets' tiles
 constexpr int kTileThreads = 512;
 constexpr int kLdsBytes = 160 * 1024;         // LDS per CU
 constexpr uint32_t kPersistSlots = 64;        // task slots per resident workgroup to persist
@@ -246,27 +246,22 @@ __device__ __forceinline__ uint32_t hinsert_peek(uint32_t *hkey, uint32_t key)
     return kEmpty;
 }
 
-__global__ void k_fill_u32(uint32_t *p, uint32_t n, uint32_t v)
-{
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
 // 8 waves per SIMD: two 1024-thread blocks per CU (their hash tables take
 // 64 KB of LDS each), which needs the SGPR count held to the 8-wave budget.
-template <bool BATCH>
+template <bool BATCH, int RPT, int HB>
 __global__ void __launch_bounds__(kBinThreads, 8)
 k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
         const double *__restrict__ vv_all, const double *__restrict__ ww_all,
         uint32_t *__restrict__ counts, const BatchJob *__restrict__ jobs, int njobs)
 {
-    __shared__ uint32_t hkey[kBinSlots], hcnt[kBinSlots];
-    for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) {
+    constexpr int SLOTS = 1 << HB;
+    __shared__ uint32_t hkey[SLOTS], hcnt[SLOTS];
+    for (int i = threadIdx.x; i < SLOTS; i += kBinThreads) {
         hkey[i] = kEmpty;
         hcnt[i] = 0;
     }
     __syncthreads();
-    const BlockRows br = block_rows(g, blockIdx.x * (uint32_t)kBinRows, n_all, uu_all, vv_all,
+    const BlockRows br = block_rows(g, blockIdx.x * (uint32_t)(kBinThreads * RPT), n_all, uu_all, vv_all,
                                     ww_all, nullptr, nullptr, nullptr, BATCH ? jobs : nullptr,
                                     njobs);
     const auto *__restrict__ uu = as_global(br.uu);
@@ -276,9 +271,9 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
     // A thread's rows are taken kCountBatch at a time, all their coordinates
     // requested before any is hashed: one memory round trip per batch rather
     // than one per row.
-    constexpr int kCountBatch = 4;
-    static_assert(kBinRowsPerThread % kCountBatch == 0, "row batches per thread");
-    for (int k0 = 0; k0 < kBinRowsPerThread; k0 += kCountBatch) {
+    constexpr int kCountBatch = RPT < 4 ? RPT : 4;
+    static_assert(RPT % kCountBatch == 0, "row batches per thread");
+    for (int k0 = 0; k0 < RPT; k0 += kCountBatch) {
         double u[kCountBatch], v[kCountBatch], w[kCountBatch];
 #pragma unroll
         for (int j = 0; j < kCountBatch; ++j) {
@@ -299,7 +294,7 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
                 uint32_t keys[4];
                 const int nk = row_keys(g, f, keys);
                 for (int q = 0; q < nk; ++q) {
-                    const uint32_t h = hinsert_peek<kBinHashBits>(hkey, keys[q]);
+                    const uint32_t h = hinsert_peek<HB>(hkey, keys[q]);
                     if (h == kEmpty) atomicAdd(&counts[counter_at(g, keys[q])], 1u);
                     else atomicAdd(&hcnt[h], 1u);
                 }
@@ -307,15 +302,15 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < kBinSlots; i += kBinThreads) {
+    for (int i = threadIdx.x; i < SLOTS; i += kBinThreads) {
         const uint32_t c = hcnt[i];
         if (c) atomicAdd(&counts[counter_at(g, hkey[i])], c);
     }
 }
 
-// Scan of the histogram in three kernels: per-block sums, a single-block scan
-// of those, and the per-block downsweep that emits offsets and tasks.  Five
-// quantities are scanned: records, accumulation tasks, split buckets,
+// Scan of the histogram: grids of up to 1024 buckets in one workgroup, larger
+// ones in two kernels, per-block sums and the downsweep that emits offsets and
+// tasks.  Five quantities are scanned: records, accumulation tasks, split buckets,
 // non-empty buckets, zero tasks.  The task array holds the accumulation
 // tasks first and the zero tasks after them; the tile kernel interleaves the
 // two evenly over its workgroups.
@@ -383,90 +378,89 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
     }
 }
 
-constexpr int kTopThreads = 1024;
-
-__global__ void __launch_bounds__(kTopThreads)
-k_scan_top(GridGeom g, uint32_t *__restrict__ blocksum, uint32_t nscan,
-           uint32_t *__restrict__ offsets, uint32_t *__restrict__ meta)
-{
-    __shared__ uint32_t s[kScanQ][kTopThreads];
-    uint32_t carry[kScanQ] = {0, 0, 0, 0, 0};
-    for (uint32_t c0 = 0; c0 < nscan; c0 += kTopThreads) {
-        const uint32_t i = c0 + threadIdx.x;
-        uint32_t v[kScanQ];
-#pragma unroll
-        for (int a = 0; a < kScanQ; ++a) {
-            v[a] = i < nscan ? blocksum[a * nscan + i] : 0u;
-            s[a][threadIdx.x] = v[a];
-        }
-        __syncthreads();
-        for (int d = 1; d < kTopThreads; d <<= 1) {
-            uint32_t add[kScanQ] = {0, 0, 0, 0, 0};
-            if ((int)threadIdx.x >= d)
-#pragma unroll
-                for (int a = 0; a < kScanQ; ++a) add[a] = s[a][threadIdx.x - d];
-            __syncthreads();
-#pragma unroll
-            for (int a = 0; a < kScanQ; ++a) s[a][threadIdx.x] += add[a];
-            __syncthreads();
-        }
-#pragma unroll
-        for (int a = 0; a < kScanQ; ++a) {
-            if (i < nscan) blocksum[a * nscan + i] = carry[a] + s[a][threadIdx.x] - v[a];
-            carry[a] += s[a][kTopThreads - 1];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        offsets[g.nb] = carry[0];
-        meta[0] = carry[0];             // records
-        meta[1] = carry[1] + carry[4];  // tasks (accumulation + zero)
-        meta[2] = carry[2];             // split buckets
-        meta[3] = carry[3];             // non-empty buckets
-        meta[4] = carry[1];             // accumulation tasks (stored first)
-        meta[5] = 0;                    // next task for the tile kernel's workgroups
-        meta[6] = meta[7] = 0;          // largest |S| of the call (FP32 split buckets)
-    }
-}
-
+// Offsets, cursors, tasks and split list of 1024 buckets per workgroup.  The
+// counters it has read and the row flags are cleared on the way: the counters
+// for the next call's count, the flags for this call's tile kernel.  With nscan == 1
+// this is the whole scan; otherwise each workgroup sums the block sums before
+// it (and all of them, for the totals) itself, which for at most a few
+// thousand blocks is less than a launch between the two kernels costs.
 __global__ void __launch_bounds__(kThreads)
-k_scan_down(GridGeom g, const uint32_t *__restrict__ counts,
-            const uint32_t *__restrict__ blockoff, uint32_t nscan, uint32_t *__restrict__ offsets,
-            uint32_t *__restrict__ cursor, uint4 *__restrict__ tasks, uint32_t task_cap,
-            uint32_t *__restrict__ split_list, uint32_t split_cap, const uint32_t *__restrict__ meta,
-            int zero)
+k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restrict__ blocksum,
+            uint32_t nscan, uint32_t *__restrict__ offsets, uint32_t *__restrict__ cursor,
+            uint4 *__restrict__ tasks, uint32_t task_cap, uint32_t *__restrict__ split_list,
+            uint32_t split_cap, uint32_t *__restrict__ meta, uint32_t *__restrict__ rowlive,
+            uint32_t rowlive_words, int zero)
 {
-    __shared__ uint32_t s[4][kThreads];
-    uint32_t c[4] = {0, 0, 0, 0}, v[4] = {0, 0, 0, 0};
-    const uint32_t b0 = blockIdx.x * kScanBlock + threadIdx.x * 4;
+    constexpr int NT = kThreads, NW = NT / 64;
+    __shared__ uint32_t wtot[kScanQ][NW];       // wave totals
+    __shared__ uint32_t before[kScanQ], total[kScanQ];
+    // Split buckets of this block, whose tasks the whole workgroup writes.
+    __shared__ uint4 big[4 * NT];               // bucket, first record, records, first task
+    __shared__ uint32_t bigtag[4 * NT], nbig;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t i = blockIdx.x * NT + threadIdx.x; i < rowlive_words; i += gridDim.x * NT)
+        rowlive[i] = 0u;
+    uint32_t c[4] = {0, 0, 0, 0}, v[kScanQ] = {0, 0, 0, 0, 0};
+    const uint32_t b0 = blockIdx.x * (4 * NT) + threadIdx.x * 4;
     const int nv = b0 >= g.nb ? 0 : (int)min(4u, g.nb - b0);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         if (k < nv) {
             c[k] = counts[counter_at(g, b0 + k)];
+            counts[counter_at(g, b0 + k)] = 0u;
             v[0] += c[k];
             v[2] += c[k] > g.rmax ? 1u : 0u;
+            v[3] += c[k] > 0 ? 1u : 0u;
         }
     }
-    group_tasks(c, nv, g.rmax, zero, g.zrun, v[1], v[3]);
+    group_tasks(c, nv, g.rmax, zero, g.zrun, v[1], v[4]);
+    // Inclusive scan in the wave, then over the wave totals.
+    uint32_t x[kScanQ];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) s[a][threadIdx.x] = v[a];
-    __syncthreads();
-    for (int d = 1; d < kThreads; d <<= 1) {
-        uint32_t add[4] = {0, 0, 0, 0};
-        if ((int)threadIdx.x >= d)
-#pragma unroll
-            for (int a = 0; a < 4; ++a) add[a] = s[a][threadIdx.x - d];
-        __syncthreads();
-#pragma unroll
-        for (int a = 0; a < 4; ++a) s[a][threadIdx.x] += add[a];
-        __syncthreads();
+    for (int a = 0; a < kScanQ; ++a) {
+        x[a] = v[a];
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x[a], d);
+            if (lane >= d) x[a] += y;
+        }
+        if (lane == 63) wtot[a][wave] = x[a];
     }
-    uint32_t ro = blockoff[blockIdx.x] + s[0][threadIdx.x] - v[0];
-    uint32_t to = blockoff[nscan + blockIdx.x] + s[1][threadIdx.x] - v[1];
-    uint32_t so = blockoff[2 * nscan + blockIdx.x] + s[2][threadIdx.x] - v[2];
-    // Zero tasks follow all accumulation tasks (meta[4] of them).
-    uint32_t zo = meta[4] + blockoff[4 * nscan + blockIdx.x] + s[3][threadIdx.x] - v[3];
+    if (threadIdx.x == 0) nbig = 0u;
+    if (threadIdx.x < kScanQ) before[threadIdx.x] = total[threadIdx.x] = 0u;
+    __syncthreads();
+    if (nscan > 1) {
+#pragma unroll
+        for (int a = 0; a < kScanQ; ++a) {
+            uint32_t pre = 0, all = 0;
+            for (uint32_t i = threadIdx.x; i < nscan; i += NT) {
+                const uint32_t y = blocksum[a * nscan + i];
+                all += y;
+                if (i < blockIdx.x) pre += y;
+            }
+            for (int d = 32; d > 0; d >>= 1) {
+                pre += __shfl_xor(pre, d);
+                all += __shfl_xor(all, d);
+            }
+            if (lane == 0) {
+                atomicAdd(&before[a], pre);
+                atomicAdd(&total[a], all);
+            }
+        }
+    } else if (threadIdx.x < kScanQ) {
+        uint32_t all = 0;
+        for (int i = 0; i < NW; ++i) all += wtot[threadIdx.x][i];
+        total[threadIdx.x] = all;
+    }
+    __syncthreads();
+    uint32_t ex[kScanQ];
+#pragma unroll
+    for (int a = 0; a < kScanQ; ++a) {
+        ex[a] = before[a] + x[a] - v[a];
+        for (int i = 0; i < wave; ++i) ex[a] += wtot[a][i];
+    }
+    uint32_t ro = ex[0], to = ex[1], so = ex[2];
+    // Zero tasks follow all accumulation tasks.
+    uint32_t zo = total[1] + ex[4];
     int run = 0;
     for (int k = 0; k < nv; ++k) {
         const uint32_t b = b0 + k;
@@ -484,17 +478,39 @@ k_scan_down(GridGeom g, const uint32_t *__restrict__ counts,
         } else {
             run = 0;
             const uint32_t nt = ntasks_of(c[k], g.rmax);
-            // Tasks of a split bucket carry its slot in split_list (always
-            // below split_cap: a split bucket holds more than rmax records).
-            const uint32_t tag = nt > 1 ? (so < split_cap ? kSplitTask + so : 1u) : 0u;
-            for (uint32_t q = 0; q < nt; ++q) {
-                const uint32_t r0 = ro + q * g.rmax, r1 = min(r0 + g.rmax, ro + c[k]);
-                if (to + q < task_cap) tasks[to + q] = make_uint4(b, r0, r1, tag);
+            if (nt == 1) {
+                if (to < task_cap) tasks[to] = make_uint4(b, ro, ro + c[k], 0u);
+            } else {
+                // Tasks of a split bucket carry its slot in split_list (always
+                // below split_cap: a split bucket holds more than rmax records).
+                const uint32_t i = atomicAdd(&nbig, 1u);
+                big[i] = make_uint4(b, ro, c[k], to);
+                bigtag[i] = so < split_cap ? kSplitTask + so : 1u;
+                if (so < split_cap) split_list[so++] = b;
             }
-            if (nt > 1 && so < split_cap) split_list[so++] = b;
             to += nt;
         }
         ro += c[k];
+    }
+    __syncthreads();
+    // One wave per split bucket.
+    for (uint32_t i = wave; i < nbig; i += NW) {
+        const uint4 e = big[i];
+        const uint32_t nt = ntasks_of(e.z, g.rmax);
+        for (uint32_t q = lane; q < nt; q += 64) {
+            const uint32_t r0 = e.y + q * g.rmax, r1 = min(r0 + g.rmax, e.y + e.z);
+            if (e.w + q < task_cap) tasks[e.w + q] = make_uint4(e.x, r0, r1, bigtag[i]);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        offsets[g.nb] = total[0];
+        meta[0] = total[0];             // records
+        meta[1] = total[1] + total[4];  // tasks (accumulation + zero)
+        meta[2] = total[2];             // split buckets
+        meta[3] = total[3];             // non-empty buckets
+        meta[4] = total[1];             // accumulation tasks (stored first)
+        meta[5] = 0;                    // next task for the tile kernel's workgroups
+        meta[6] = meta[7] = 0;          // largest |S| of the call (FP32 split buckets)
     }
 }
 
@@ -574,6 +590,31 @@ __device__ __forceinline__ void wave_row_sums(uint32_t r0, uint32_t n, uint32_t 
     }
 }
 
+// Clears the tiles of buckets that several tasks accumulate into atomically:
+// the split buckets first, first + stride, ... (one workgroup each).
+template <typename T2>
+__device__ __forceinline__ void zero_split_tiles(const GridGeom &g, uint32_t first, uint32_t stride,
+                                                 uint32_t nsplit,
+                                                 const uint32_t *__restrict__ split_list,
+                                                 T2 *__restrict__ grid)
+{
+    const uint32_t per_plane = (uint32_t)g.tiles_u * (uint32_t)g.tiles_v;
+    T2 z;
+    z.x = z.y = 0;
+    for (uint32_t i = first; i < nsplit; i += stride) {
+        const uint32_t b = split_list[i];
+        const int w = (int)(b / per_plane), rem = (int)(b % per_plane);
+        const int tv = rem / g.tiles_u, tu = rem % g.tiles_u;
+        const int j0 = tu * g.tu, k0 = tv * g.tv;
+        const int nj = min(g.tu, g.nx - j0), nk = min(g.tv, g.ny - k0);
+        for (int idx = threadIdx.x; idx < nk << g.tu_shift; idx += blockDim.x) {
+            const int kk = idx >> g.tu_shift, jj = idx & (g.tu - 1);
+            if (jj < nj)
+                grid[((size_t)w * g.ny + (size_t)(k0 + kk)) * (size_t)g.nx + (size_t)(j0 + jj)] = z;
+        }
+    }
+}
+
 // VMODE: 0 = per-row scalar reads, 1 = per-row 16-byte reads (F*P a multiple
 // of 4), 2 or 4 = wave-cooperative reads with VMODE lanes per row (F*P = 8 or
 // 16); 16-byte modes need 16-byte aligned visibility arrays.
@@ -584,8 +625,17 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
           const float *__restrict__ vr_all, const float *__restrict__ vi_all,
           const float *__restrict__ wt_all, uint32_t *__restrict__ cursor,
           typename RecOf<PREC>::type *__restrict__ rec, uint32_t *__restrict__ meta,
-          const BatchJob *__restrict__ jobs, int njobs)
+          const BatchJob *__restrict__ jobs, int njobs, uint32_t row_blocks,
+          const uint32_t *__restrict__ split_list, void *grid)
 {
+    // Workgroups past the row blocks clear the tiles of split buckets, which
+    // the tile kernel's tasks add to (a launch of its own took 4-9 us).
+    if (blockIdx.x >= row_blocks) {
+        using T2 = typename std::conditional<PREC == RICK_FP64, double2, float2>::type;
+        zero_split_tiles<T2>(g, blockIdx.x - row_blocks, gridDim.x - row_blocks, meta[2],
+                             split_list, static_cast<T2 *>(grid));
+        return;
+    }
     const BlockRows br = block_rows(g, blockIdx.x * kRowsPerBlock, n_all, uu_all, vv_all, ww_all,
                                     vr_all, vi_all, wt_all, BATCH ? jobs : nullptr, njobs);
     const double *__restrict__ uu = br.uu;
@@ -777,29 +827,6 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
         }
     }
 }
-
-// Clears the tiles of buckets that several tasks accumulate into atomically.
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-k_zero_split(GridGeom g, const uint32_t *__restrict__ split_list, const uint32_t *__restrict__ meta,
-             T *__restrict__ grid)
-{
-    if (blockIdx.x >= meta[2]) return;
-    const uint32_t b = split_list[blockIdx.x];
-    const uint32_t per_plane = (uint32_t)g.tiles_u * (uint32_t)g.tiles_v;
-    const int w = (int)(b / per_plane), rem = (int)(b % per_plane);
-    const int tv = rem / g.tiles_u, tu = rem % g.tiles_u;
-    const int j0 = tu * g.tu, k0 = tv * g.tv;
-    const int nj = min(g.tu, g.nx - j0), nk = min(g.tv, g.ny - k0);
-    for (int idx = threadIdx.x; idx < nk * g.tu; idx += kThreads) {
-        const int kk = idx / g.tu, jj = idx % g.tu;
-        if (jj >= nj) continue;
-        const size_t c = ((size_t)w * g.ny + (size_t)(k0 + kk)) * (size_t)g.nx + (size_t)(j0 + jj);
-        grid[2 * c] = T(0);
-        grid[2 * c + 1] = T(0);
-    }
-}
-
 
 // FP32 split buckets (several tasks add into one tile) accumulate in one
 // 64-bit fixed-point tile per bucket with integer atomics, so the sum does not
@@ -1274,6 +1301,17 @@ void capacities(const GridGeom &g, uint32_t max_points, uint32_t *rec_cap, uint3
 
 }  // namespace
 
+// Rows per thread of the count kernel.  Larger blocks send fewer atomics to
+// the histogram (7.7 M rows: 254 / 114 / 69 us at 1 / 4 / 16 rows a thread; 3 M
+// rows: 102 / 47 / 42 us), but a launch that does not fill the chip takes as
+// long as one thread's rows (50 k rows: 7 / 12 / 34 us; 516 k: 13 / 13 / 33;
+// 1 M: 28 / 18 / 37; 1.5 M: 38 / 24 / 37).
+int count_rows_per_thread(uint32_t n)
+{
+    if (n >= 160u * 16 * kBinThreads) return 16;
+    return n >= 128u * 4 * kBinThreads ? 4 : 1;
+}
+
 int counter_shift(uint32_t nb)
 {
     int shift = 0;
@@ -1289,7 +1327,7 @@ const char *grid_launch_limit(const GridGeom &g, uint32_t max_points)
     capacities(g, max_points, &rec_cap, &split_cap, &task_cap, &nscan);
     // A launch holds fewer than 2^32 threads.  Persistent tile launches are
     // capped at the resident workgroups; the others take one workgroup per
-    // task slot, and k_zero_split one per split-bucket slot.
+    // task slot.
     constexpr uint64_t kMaxThreads = 1ull << 32;
     if (!tile_persistent(g.tu, g.tv) && (uint64_t)task_cap * kTileThreads >= kMaxThreads)
         return "too many gridding tasks for one tile launch (fewer tiles or rows per "
@@ -1365,36 +1403,45 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
     Timing off;
     if (tm == nullptr) tm = &off;
     const uint32_t nblk = (n + kRowsPerBlock - 1) / kRowsPerBlock;
-    const uint32_t cblk = (n + kBinRows - 1) / kBinRows;
-    // The counts and the row flags that follow them are cleared together.
-    const uint32_t fill_words =
-        (uint32_t)((reinterpret_cast<const char *>(w.rowlive) - reinterpret_cast<const char *>(w.counts) +
-                    align_up((size_t)g.planes * g.ny, 256)) / sizeof(uint32_t));
-    const uint32_t fill_blocks = min((fill_words + 255u) / 256u, 4096u);
+    const int rpt = count_rows_per_thread(n);
+    const uint32_t cblk = (uint32_t)(((uint64_t)n + (uint64_t)rpt * kBinThreads - 1) /
+                                     ((uint64_t)rpt * kBinThreads));
     // Overwrite of a dense grid: runs of empty buckets get zero tasks.
     const int zero = (!accumulate && clear_empty) ? 1 : 0;
     // Overwrite of a sparse grid: the tile kernel flags the rows it writes
     // non-zero cells to, for the image chain.
     unsigned char *rowlive = (!accumulate && !clear_empty) ? w.rowlive : nullptr;
     tm->begin(RICK_STAGE_COUNT_ROWS, s);
-    hipLaunchKernelGGL(k_fill_u32, dim3(fill_blocks), dim3(256), 0, s, w.counts, fill_words, 0u);
     if (n > 0) {
-        if (jobs)
-            hipLaunchKernelGGL(k_count<true>, dim3(cblk), dim3(kBinThreads), 0, s, g, n, uu, vv,
-                               ww, w.counts, jobs, njobs);
-        else
-            hipLaunchKernelGGL(k_count<false>, dim3(cblk), dim3(kBinThreads), 0, s, g, n, uu, vv,
-                               ww, w.counts, jobs, njobs);
+#define RICK_COUNT(BT, R, HB)                                                                 \
+    hipLaunchKernelGGL((k_count<BT, R, HB>), dim3(cblk), dim3(kBinThreads), 0, s, g, n, uu, vv, \
+                       ww, w.counts, jobs, njobs)
+        if (jobs) {
+            if (rpt == 16) RICK_COUNT(true, 16, 13);
+            else if (rpt == 4) RICK_COUNT(true, 4, 12);
+            else RICK_COUNT(true, 1, 11);
+        } else {
+            if (rpt == 16) RICK_COUNT(false, 16, 13);
+            else if (rpt == 4) RICK_COUNT(false, 4, 12);
+            else RICK_COUNT(false, 1, 11);
+        }
+#undef RICK_COUNT
     }
     tm->end(RICK_STAGE_COUNT_ROWS, s);
     tm->begin(RICK_STAGE_SCAN, s);
-    hipLaunchKernelGGL(k_scan_reduce, dim3(w.nscan), dim3(kThreads), 0, s, g, w.counts,
-                       w.blocksum, w.nscan, zero);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kTopThreads), 0, s, g, w.blocksum, w.nscan,
-                       w.offsets, w.meta);
-    hipLaunchKernelGGL(k_scan_down, dim3(w.nscan), dim3(kThreads), 0, s, g, w.counts,
-                       w.blocksum, w.nscan, w.offsets, w.cursor, w.tasks, w.task_cap,
-                       w.split_list, w.split_cap, w.meta, zero);
+    const uint32_t rl_words = (uint32_t)(align_up((size_t)g.planes * g.ny, 256) / sizeof(uint32_t));
+    uint32_t *rl = reinterpret_cast<uint32_t *>(w.rowlive);
+    if (w.nscan == 1) {
+        hipLaunchKernelGGL(k_scan_down, dim3(1), dim3(kThreads), 0, s, g, w.counts, w.blocksum,
+                           1u, w.offsets, w.cursor, w.tasks, w.task_cap, w.split_list,
+                           w.split_cap, w.meta, rl, rl_words, zero);
+    } else {
+        hipLaunchKernelGGL(k_scan_reduce, dim3(w.nscan), dim3(kThreads), 0, s, g, w.counts,
+                           w.blocksum, w.nscan, zero);
+        hipLaunchKernelGGL(k_scan_down, dim3(w.nscan), dim3(kThreads), 0, s, g,
+                           w.counts, w.blocksum, w.nscan, w.offsets, w.cursor, w.tasks,
+                           w.task_cap, w.split_list, w.split_cap, w.meta, rl, rl_words, zero);
+    }
     tm->end(RICK_STAGE_SCAN, s);
     tm->begin(RICK_STAGE_SCATTER, s);
     if (n > 0) {
@@ -1403,17 +1450,19 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
                           ((reinterpret_cast<uintptr_t>(vr) | reinterpret_cast<uintptr_t>(vi)) &
                            15u) == 0u;   // batch: vr = vi = null, the caller checked the jobs
         const int mode = !vec4 ? 0 : FP == 8u ? 2 : FP == 16u ? 4 : 1;
+        // Overwritten grids: the split buckets' tiles start at zero (FP32: for
+        // the non-finite fallback; its finite sums go through integer tiles).
+        const uint32_t zblk = accumulate ? 0u : std::min(w.split_cap, kZeroBlocks);
+#define RICK_SCATTER_LAUNCH(PR, VM, BT)                                                       \
+    hipLaunchKernelGGL((k_scatter<PR, VM, BT>), dim3(nblk + zblk), dim3(kScatterThreads), 0,  \
+                       s, g, n, F, P, uu, vv, ww, vr, vi, wt, w.cursor,                       \
+                       static_cast<typename RecOf<PR>::type *>(w.records), w.meta, jobs,      \
+                       njobs, nblk, w.split_list, grid)
 #define RICK_SCATTER(PR, VM)                                                                  \
     if (jobs)                                                                                 \
-        hipLaunchKernelGGL((k_scatter<PR, VM, true>), dim3(nblk), dim3(kScatterThreads), 0, s, \
-                           g, n, F, P, uu, vv, ww, vr, vi, wt, w.cursor,                      \
-                           static_cast<typename RecOf<PR>::type *>(w.records), w.meta, jobs,  \
-                           njobs);                                                            \
+        RICK_SCATTER_LAUNCH(PR, VM, true);                                                    \
     else                                                                                      \
-        hipLaunchKernelGGL((k_scatter<PR, VM, false>), dim3(nblk), dim3(kScatterThreads), 0,  \
-                           s, g, n, F, P, uu, vv, ww, vr, vi, wt, w.cursor,                   \
-                           static_cast<typename RecOf<PR>::type *>(w.records), w.meta, jobs,  \
-                           njobs)
+        RICK_SCATTER_LAUNCH(PR, VM, false)
 #define RICK_SCATTER_MODES(PR)                                                                \
     switch (mode) {                                                                           \
     case 4: RICK_SCATTER(PR, 4); break;                                                       \
@@ -1428,25 +1477,11 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
         }
 #undef RICK_SCATTER_MODES
 #undef RICK_SCATTER
+#undef RICK_SCATTER_LAUNCH
     }
     tm->end(RICK_STAGE_SCATTER, s);
-    if (precision == RICK_FP64) {
-        if (!accumulate) {
-            tm->begin(RICK_STAGE_ZERO_SPLIT, s);
-            hipLaunchKernelGGL(k_zero_split<double>, dim3(w.split_cap), dim3(kThreads), 0, s, g,
-                               w.split_list, w.meta, static_cast<double *>(grid));
-            tm->end(RICK_STAGE_ZERO_SPLIT, s);
-        }
+    if (precision == RICK_FP64)
         return launch_tile<RICK_FP64>(g, w, table_d, grid, accumulate, rowlive, s, tm);
-    }
-    // FP32: split buckets accumulate in integer fixed point (order-independent);
-    // their grid tiles are cleared for the non-finite fallback.
-    if (!accumulate) {
-        tm->begin(RICK_STAGE_ZERO_SPLIT, s);
-        hipLaunchKernelGGL(k_zero_split<float>, dim3(w.split_cap), dim3(kThreads), 0, s, g,
-                           w.split_list, w.meta, static_cast<float *>(grid));
-        tm->end(RICK_STAGE_ZERO_SPLIT, s);
-    }
     return launch_tile<RICK_FP32>(g, w, table_d, grid, accumulate, rowlive, s, tm);
 }
 

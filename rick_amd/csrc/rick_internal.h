@@ -130,7 +130,7 @@ inline double exact_inverse(double d)
 
 // Workspace of the binned gridder, carved out of one device allocation.
 struct GridWork {
-    uint32_t *counts;       // [nb << cshift] records per bucket
+    uint32_t *counts;       // [nb << cshift] records per bucket; zero between calls
     uint32_t *cursor;       // [nb << cshift] scatter cursor (starts at the bucket offset)
     uint32_t *offsets;      // [nb+1] exclusive scan of counts
     uint32_t *blocksum;     // [5*nscan] per scan block: records, accumulation tasks, split,
@@ -142,8 +142,7 @@ struct GridWork {
                             //   tile kernel's next task slot (persistent workgroups)
     void *records;          // [rec_cap] sorted row records
     // [planes*ny] per grid row of each plane: non-zero iff the tile kernel
-    // wrote a non-zero cell to it (sparse overwrite only; cleared with the
-    // counts, whose allocation it directly follows).
+    // wrote a non-zero cell to it (sparse overwrite only; cleared by the scan).
     unsigned char *rowlive;
     // FP32 only: per split slot, the count of its tasks done and its 64-bit
     // fixed-point accumulator tile (re then im, tu*tv each); both are zero

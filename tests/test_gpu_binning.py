@@ -1,0 +1,46 @@
+"""The gridder's binning at the sizes where its launches change: blocks of 1,
+4 or 16 rows per thread, one scan workgroup or two scan kernels, split buckets
+spread over the scan's waves.  FP64 against the CPU oracle at the suite's
+1e-12 (only the order of the sums differs)."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import rel_l2
+from oracle import oracle as O
+import rick_amd
+from rick_amd import FP64, Plan
+
+pytestmark = pytest.mark.gpu
+
+
+def make_rows(n, seed, hot):
+    rng = np.random.default_rng(seed)
+    uu, vv, ww = (rng.uniform(0.0, 1.0, n) for _ in range(3))
+    k = int(n * hot)
+    uu[:k], vv[:k], ww[:k] = (rng.uniform(0.5, 0.51, k) for _ in range(3))
+    vr, vi = (rng.normal(size=n).astype(np.float32) for _ in range(2))
+    return uu, vv, ww, vr, vi, rng.uniform(0.5, 1.5, n).astype(np.float32)
+
+
+# Tiles are 64 x 64: 256^2 grids hold 16 buckets a plane, so 64 planes are the
+# last grid of one scan workgroup (1024 buckets) and 65 the first of two.
+@pytest.mark.parametrize("n,planes,rows_per_task", [
+    (1, 4, 0), (1023, 64, 3), (1025, 65, 3), (524287, 64, 300), (524289, 65, 300),
+    (2621439, 4, 4096), (2621443, 80, 4096)])
+def test_binning_launch_edges_match_oracle(n, planes, rows_per_task):
+    nx = 256
+    print(f"case n={n} planes={planes} rows_per_task={rows_per_task}", flush=True)
+    plan = Plan(nx, nx, planes, kernel=rick_amd.KAISERBESSEL, support=7, precision=FP64,
+                max_points=n, tile=(64, 64), rows_per_task=rows_per_task)
+    # Twice in a row with other rows, then fewer: the counters start clean each time.
+    for seed, m in ((1, n), (2, n), (3, (n + 1) // 2)):
+        rows = make_rows(m, seed, 0.3)
+        ref = O.wstack(O.KAISERBESSEL, planes, *rows, 1, 1, 1.0 / nx, 1.0 / planes, 7, nx, nx,
+                       threads=8)
+        out = plan.new_grid()
+        out.fill_(float("nan"))
+        plan.grid(*[torch.from_numpy(a).to("cuda") for a in rows], 1, 1, out=out)
+        got = out.cpu().numpy()
+        assert np.isfinite(got).all()
+        assert rel_l2(got, ref) <= 1e-12
