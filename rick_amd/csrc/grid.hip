@@ -310,31 +310,51 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
 
 // Scan of the histogram: grids of up to 1024 buckets in one workgroup, larger
 // ones in two kernels, per-block sums and the downsweep that emits offsets and
-// tasks.  Five quantities are scanned: records, accumulation tasks, split buckets,
-// non-empty buckets, zero tasks.  The task array holds the accumulation
-// tasks first and the zero tasks after them; the tile kernel interleaves the
-// two evenly over its workgroups.
-constexpr int kScanQ = 5;
-// Tasks of a bucket with c > 0 records.
+// tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
+// the accumulation tasks of three lengths.  The task array holds the long tasks
+// first (more than g.rmax / 2 records), then the middle ones (more than
+// g.rmax / 8), then the short ones, so that no long task starts when the others
+// are done, and the zero tasks last; the tile kernel interleaves accumulation
+// and zero tasks evenly over its workgroups.
+constexpr int kLengths = 3;
+enum { kQRecords, kQSplit, kQNonEmpty, kQZero, kQTasks, kScanQ = kQTasks + kLengths };
+
+// Tasks of a bucket with c > 0 records: equal parts of at most rmax records.
 __device__ __forceinline__ uint32_t ntasks_of(uint32_t c, uint32_t rmax)
 {
     return (c + rmax - 1) / rmax;
 }
 
-// Tasks of a scan thread's 4 consecutive buckets (nv of them exist): those of
-// the non-empty ones, plus, when the grid is overwritten (zero != 0), one zero
-// task per g.zrun consecutive empty ones.
-__device__ __forceinline__ void group_tasks(const uint32_t *c, int nv, uint32_t rmax, int zero,
-                                            int zrun, uint32_t &real, uint32_t &zeros)
+// Length class of the tasks of a bucket with c > 0 records (the parts of a
+// split bucket hold more than rmax / 2 each).
+__device__ __forceinline__ int length_class(uint32_t c, uint32_t rmax)
 {
-    real = zeros = 0;
+    return c > rmax / 2 ? 0 : c > rmax / 8 ? 1 : 2;
+}
+
+// What a scan thread's 4 consecutive buckets (nv of them exist) add: the
+// non-empty ones their records and tasks, and, when the grid is overwritten
+// (zero != 0), one zero task per zrun consecutive empty ones.
+__device__ __forceinline__ void group_sums(const uint32_t *c, int nv, uint32_t rmax, int zero,
+                                           int zrun, uint32_t *v)
+{
+#pragma unroll
+    for (int a = 0; a < kScanQ; ++a) v[a] = 0;
     int run = 0;  // length of the current run of empty buckets
-    for (int k = 0; k < nv; ++k) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (k >= nv) break;
         if (c[k]) {
-            real += ntasks_of(c[k], rmax);
+            v[kQRecords] += c[k];
+            v[kQSplit] += c[k] > rmax ? 1u : 0u;
+            v[kQNonEmpty] += 1u;
+            const uint32_t nt = c[k] > rmax ? ntasks_of(c[k], rmax) : 1u;
+            const int len = length_class(c[k], rmax);
+#pragma unroll
+            for (int q = 0; q < kLengths; ++q) v[kQTasks + q] += q == len ? nt : 0u;
             run = 0;
         } else {
-            if (zero && run % zrun == 0) ++zeros;
+            if (zero && run % zrun == 0) ++v[kQZero];
             ++run;
         }
     }
@@ -345,25 +365,15 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
               uint32_t nscan, int zero)
 {
     __shared__ uint32_t s[kScanQ][kThreads];
-    uint32_t r = 0, sp = 0, ne = 0, c[4] = {0, 0, 0, 0};
+    uint32_t c[4] = {0, 0, 0, 0}, v[kScanQ];
     const uint32_t b0 = blockIdx.x * kScanBlock + threadIdx.x * 4;
     const int nv = b0 >= g.nb ? 0 : (int)min(4u, g.nb - b0);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        if (k < nv) {
-            c[k] = counts[counter_at(g, b0 + k)];
-            r += c[k];
-            sp += c[k] > g.rmax ? 1u : 0u;
-            ne += c[k] > 0 ? 1u : 0u;
-        }
-    }
-    uint32_t tr, tz;
-    group_tasks(c, nv, g.rmax, zero, g.zrun, tr, tz);
-    s[0][threadIdx.x] = r;
-    s[1][threadIdx.x] = tr;
-    s[2][threadIdx.x] = sp;
-    s[3][threadIdx.x] = ne;
-    s[4][threadIdx.x] = tz;
+    for (int k = 0; k < 4; ++k)
+        if (k < nv) c[k] = counts[counter_at(g, b0 + k)];
+    group_sums(c, nv, g.rmax, zero, g.zrun, v);
+#pragma unroll
+    for (int a = 0; a < kScanQ; ++a) s[a][threadIdx.x] = v[a];
     __syncthreads();
     for (int d = kThreads / 2; d > 0; d >>= 1) {
         if ((int)threadIdx.x < d) {
@@ -400,7 +410,7 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (uint32_t i = blockIdx.x * NT + threadIdx.x; i < rowlive_words; i += gridDim.x * NT)
         rowlive[i] = 0u;
-    uint32_t c[4] = {0, 0, 0, 0}, v[kScanQ] = {0, 0, 0, 0, 0};
+    uint32_t c[4] = {0, 0, 0, 0}, v[kScanQ];
     const uint32_t b0 = blockIdx.x * (4 * NT) + threadIdx.x * 4;
     const int nv = b0 >= g.nb ? 0 : (int)min(4u, g.nb - b0);
 #pragma unroll
@@ -408,12 +418,9 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
         if (k < nv) {
             c[k] = counts[counter_at(g, b0 + k)];
             counts[counter_at(g, b0 + k)] = 0u;
-            v[0] += c[k];
-            v[2] += c[k] > g.rmax ? 1u : 0u;
-            v[3] += c[k] > 0 ? 1u : 0u;
         }
     }
-    group_tasks(c, nv, g.rmax, zero, g.zrun, v[1], v[4]);
+    group_sums(c, nv, g.rmax, zero, g.zrun, v);
     // Inclusive scan in the wave, then over the wave totals.
     uint32_t x[kScanQ];
 #pragma unroll
@@ -458,9 +465,14 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
         ex[a] = before[a] + x[a] - v[a];
         for (int i = 0; i < wave; ++i) ex[a] += wtot[a][i];
     }
-    uint32_t ro = ex[0], to = ex[1], so = ex[2];
-    // Zero tasks follow all accumulation tasks.
-    uint32_t zo = total[1] + ex[4];
+    uint32_t ro = ex[kQRecords], so = ex[kQSplit], to[kLengths];
+    uint32_t at = 0;   // each length's tasks follow those of the lengths before it
+#pragma unroll
+    for (int q = 0; q < kLengths; ++q) {
+        to[q] = at + ex[kQTasks + q];
+        at += total[kQTasks + q];
+    }
+    uint32_t zo = at + ex[kQZero];
     int run = 0;
     for (int k = 0; k < nv; ++k) {
         const uint32_t b = b0 + k;
@@ -477,18 +489,26 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
             ++run;
         } else {
             run = 0;
-            const uint32_t nt = ntasks_of(c[k], g.rmax);
+            const int len = length_class(c[k], g.rmax);
+            uint32_t t = 0;
+            const uint32_t nt = c[k] > g.rmax ? ntasks_of(c[k], g.rmax) : 1u;
+#pragma unroll
+            for (int q = 0; q < kLengths; ++q) {
+                if (q == len) {
+                    t = to[q];
+                    to[q] += nt;
+                }
+            }
             if (nt == 1) {
-                if (to < task_cap) tasks[to] = make_uint4(b, ro, ro + c[k], 0u);
+                if (t < task_cap) tasks[t] = make_uint4(b, ro, ro + c[k], 0u);
             } else {
                 // Tasks of a split bucket carry its slot in split_list (always
                 // below split_cap: a split bucket holds more than rmax records).
                 const uint32_t i = atomicAdd(&nbig, 1u);
-                big[i] = make_uint4(b, ro, c[k], to);
+                big[i] = make_uint4(b, ro, c[k], t);
                 bigtag[i] = so < split_cap ? kSplitTask + so : 1u;
                 if (so < split_cap) split_list[so++] = b;
             }
-            to += nt;
         }
         ro += c[k];
     }
@@ -496,19 +516,19 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
     // One wave per split bucket.
     for (uint32_t i = wave; i < nbig; i += NW) {
         const uint4 e = big[i];
-        const uint32_t nt = ntasks_of(e.z, g.rmax);
+        const uint32_t nt = ntasks_of(e.z, g.rmax), part = (e.z + nt - 1) / nt;
         for (uint32_t q = lane; q < nt; q += 64) {
-            const uint32_t r0 = e.y + q * g.rmax, r1 = min(r0 + g.rmax, e.y + e.z);
+            const uint32_t r0 = e.y + q * part, r1 = min(r0 + part, e.y + e.z);
             if (e.w + q < task_cap) tasks[e.w + q] = make_uint4(e.x, r0, r1, bigtag[i]);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        offsets[g.nb] = total[0];
-        meta[0] = total[0];             // records
-        meta[1] = total[1] + total[4];  // tasks (accumulation + zero)
-        meta[2] = total[2];             // split buckets
-        meta[3] = total[3];             // non-empty buckets
-        meta[4] = total[1];             // accumulation tasks (stored first)
+        offsets[g.nb] = total[kQRecords];
+        meta[0] = total[kQRecords];
+        meta[1] = at + total[kQZero];   // tasks (accumulation + zero)
+        meta[2] = total[kQSplit];
+        meta[3] = total[kQNonEmpty];
+        meta[4] = at;                   // accumulation tasks (stored first)
         meta[5] = 0;                    // next task for the tile kernel's workgroups
         meta[6] = meta[7] = 0;          // largest |S| of the call (FP32 split buckets)
     }
