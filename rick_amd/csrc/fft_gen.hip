@@ -5,8 +5,8 @@
 // Each axis of the 2-D transform is planned on its own:
 //   * direct     -- one pass over lines of length L <= 4096 whose prime
 //                   factors are <= 13: a mixed-radix Stockham transform held
-//                   in LDS (radices 16, 8, 4, 2, 3, 5, 7, 11, 13), one
-//                   workgroup per G = 4096 / L lines;
+//                   in LDS (every radix from 2 to 16), one workgroup per G
+//                   lines;
 //   * four-step  -- N = N1 * N2 (both direct lengths, N1 closest to sqrt(N)):
 //                   pass A does the N1-point DFTs with the twiddle W_N^(k1 n2)
 //                   into a one-plane scratch, pass B the N2-point DFTs back,
@@ -33,10 +33,34 @@ namespace {
 
 using namespace fftk;
 
-constexpr int kGenThreads = 256;
-constexpr int kGenElems = 4096;       // complex values per workgroup (G * L)
+constexpr int kGenThreads = 512;      // most threads of a workgroup
+constexpr int kGenValues = 16;        // most complex values a thread holds
+constexpr int kGenElems = 4096;       // longest line of one pass
 constexpr int kGenDirectCols = 256;   // longest column transform done in one pass
 constexpr size_t kBlueChunk = size_t(1) << 25;   // Bluestein scratch: elements per chunk
+
+constexpr int kGenLdsBytes = 80 * 1024;          // dynamic LDS of a workgroup, at most
+
+// Butterflies of radix R a thread takes in one pass.
+__host__ __device__ constexpr int gen_bpt(int R) { return kGenValues / R > 1 ? kGenValues / R : 1; }
+
+// floor(x / d) for x * d < 2^32, from m = ceil(2^32 / d) (d > 1; 0 stands for 1).
+__host__ __device__ inline uint32_t gen_magic(uint32_t d)
+{
+    return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u;
+}
+__device__ __forceinline__ int gen_div(int x, uint32_t m)
+{
+    return m ? (int)__umulhi((uint32_t)x, m) : x;
+}
+
+// Occupancy of the first axis transformed (rows of a sparse grid, see
+// Occupancy in fft.hip), or the row flags of the axis after it (columns).
+struct GenOcc {
+    const uint32_t *offsets;        // rows: the gridder's bucket offsets (null: dense)
+    const unsigned char *rows;      // [planes * ny] row flags (null: dense)
+    int tu_shift, tv, tiles_u, tiles_v, ny;
+};
 
 // Line addressing of one launch.  Workgroup (group, set, plane) transforms
 // lines g0 .. g0+G-1 of that set; element n of line g is read at
@@ -47,34 +71,210 @@ constexpr size_t kBlueChunk = size_t(1) << 25;   // Bluestein scratch: elements 
 // (tw_by 2), N the table length, and the scale.
 struct GenAddr {
     int nl, G, ngroups, sets;
+    uint32_t mG;      // gen_magic(G)
     long long pz, ps_in, pg_in, pe_in, ps_out, pg_out, pe_out;
     int tw_by;
     int line_major;   // butterflies along a line are consecutive threads (contiguous lines)
+    int row_mul;      // columns: input row of element n of set s is s * set_mul + n * row_mul
+    int set_mul;
 };
 
-// Butterfly b of a pass with Lr butterflies per line.
-__device__ __forceinline__ void gen_map(int b, int Lr, int G, int line_major, int &g, int &j)
-{
-    if (line_major) { g = b / Lr; j = b % Lr; }
-    else { g = b % G; j = b / G; }
-}
-
+// LDS slot of element n of line g: line-major lines are padded by one slot
+// per 16 elements (the first pass writes with the stride of its radix).
+__host__ __device__ constexpr int gen_pad(int n) { return n + (n >> 4); }
 __device__ __forceinline__ int gen_lds(int g, int n, int L, int G, int line_major)
 {
-    return line_major ? g * L + n : n * G + g;
+    return line_major ? g * (gen_pad(L) + 1) + gen_pad(n) : n * G + g;
+}
+
+// exp(+2 pi i k/R) constants of the odd prime radices: cosines and sines of
+// 2 pi m / R for m = 1 .. (R-1)/2.
+template <int R>
+struct OddRoots;
+template <>
+struct OddRoots<7> {
+    static constexpr double c[3] = {0.62348980185873353053, -0.22252093395631440429,
+                                    -0.90096886790241912624};
+    static constexpr double s[3] = {0.78183148246802980871, 0.97492791218182360702,
+                                    0.43388373911755812048};
+};
+template <>
+struct OddRoots<11> {
+    static constexpr double c[5] = {0.84125353283118116886, 0.41541501300188642553,
+                                    -0.14231483827328514044, -0.65486073394528506406,
+                                    -0.95949297361449738989};
+    static constexpr double s[5] = {0.54064081745559758211, 0.90963199535451837141,
+                                    0.98982144188093273238, 0.75574957435425828377,
+                                    0.28173255684142969771};
+};
+template <>
+struct OddRoots<13> {
+    static constexpr double c[6] = {0.88545602565320989590, 0.56806474673115580251,
+                                    0.12053668025532305335, -0.35460488704253562597,
+                                    -0.74851074817110109863, -0.97094181742605202716};
+    static constexpr double s[6] = {0.46472317204376854566, 0.82298386589365639458,
+                                    0.99270887409805399280, 0.93501624268541482344,
+                                    0.66312265824079520238, 0.23931566428755776715};
+};
+
+// Odd prime radix: with a_m = x_m + x_(R-m) and b_m = x_m - x_(R-m),
+// X_k, X_(R-k) = x_0 + sum_m cos(2 pi k m/R) a_m +- i sum_m sin(2 pi k m/R) b_m.
+template <typename T, int R>
+__device__ __forceinline__ void dft_odd(C2<T> *v)
+{
+    constexpr int H = (R - 1) / 2;
+    C2<T> a[H], b[H];
+#pragma unroll
+    for (int m = 0; m < H; ++m) {
+        a[m] = cadd(v[m + 1], v[R - 1 - m]);
+        b[m] = csub(v[m + 1], v[R - 1 - m]);
+    }
+    const C2<T> x0 = v[0];
+    C2<T> sum = x0;
+#pragma unroll
+    for (int m = 0; m < H; ++m) sum = cadd(sum, a[m]);
+    v[0] = sum;
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+        C2<T> re = x0, im = {T(0), T(0)};
+#pragma unroll
+        for (int m = 1; m <= H; ++m) {
+            const int e = (k * m) % R, f = e > H ? R - e : e;
+            const T c = (T)OddRoots<R>::c[f - 1];
+            const T s = e > H ? -(T)OddRoots<R>::s[f - 1] : (T)OddRoots<R>::s[f - 1];
+            re.x += c * a[m - 1].x;
+            re.y += c * a[m - 1].y;
+            im.x += s * b[m - 1].x;
+            im.y += s * b[m - 1].y;
+        }
+        v[k] = {re.x - im.y, re.y + im.x};
+        v[R - k] = {re.x + im.y, re.y - im.x};
+    }
+}
+
+template <typename T, int R>
+__device__ __forceinline__ void dft_mix(C2<T> *v);
+
+constexpr int inv_mod(int a, int m)
+{
+    for (int x = 1; x < m; ++x)
+        if (a * x % m == 1) return x;
+    return 0;
+}
+
+// R = A * B with coprime factors (the prime-factor algorithm): inputs
+// n = (B n1 + A n2) mod R, outputs k with k mod A = k1, k mod B = k2, no
+// twiddles between the two.
+template <typename T, int A, int B>
+__device__ __forceinline__ void dft_coprime(C2<T> *v)
+{
+    constexpr int R = A * B, U = B * inv_mod(B % A, A), V = A * inv_mod(A % B, B);
+    C2<T> y[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) y[n2][n1] = v[(B * n1 + A * n2) % R];
+        dft_mix<T, A>(y[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        C2<T> t[B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) t[n2] = y[n2][k1];
+        dft_mix<T, B>(t);
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) v[(U * k1 + V * k2) % R] = t[k2];
+    }
+}
+
+// Radix 9 as 3 x 3 with the twiddles exp(2 pi i m/9), m = 1, 2, 4.
+template <typename T>
+__device__ __forceinline__ void dft9(C2<T> *v)
+{
+    constexpr double c1 = 0.76604444311897803520, s1 = 0.64278760968653932632,
+                     c2 = 0.17364817766693034885, s2 = 0.98480775301220805937,
+                     c4 = -0.93969262078590838405, s4 = 0.34202014332566873304;
+    C2<T> y[3][3];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < 3; ++n1) y[n2][n1] = v[3 * n1 + n2];
+        dft3(y[n2]);
+    }
+    y[1][1] = cmul(y[1][1], C2<T>{(T)c1, (T)s1});
+    y[1][2] = cmul(y[1][2], C2<T>{(T)c2, (T)s2});
+    y[2][1] = cmul(y[2][1], C2<T>{(T)c2, (T)s2});
+    y[2][2] = cmul(y[2][2], C2<T>{(T)c4, (T)s4});
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+        C2<T> t[3] = {y[0][k1], y[1][k1], y[2][k1]};
+        dft3(t);
+#pragma unroll
+        for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = t[k2];
+    }
+}
+
+template <typename T, int R>
+__device__ __forceinline__ void dft_mix(C2<T> *v)
+{
+    if constexpr (R == 2 || R == 4 || R == 8 || R == 16) dftR<T, R>(v);
+    else if constexpr (R == 3) dft3(v);
+    else if constexpr (R == 5) dft5(v);
+    else if constexpr (R == 9) dft9(v);
+    else if constexpr (R == 6) dft_coprime<T, 3, 2>(v);
+    else if constexpr (R == 10) dft_coprime<T, 5, 2>(v);
+    else if constexpr (R == 12) dft_coprime<T, 4, 3>(v);
+    else if constexpr (R == 14) dft_coprime<T, 7, 2>(v);
+    else if constexpr (R == 15) dft_coprime<T, 5, 3>(v);
+    else dft_odd<T, R>(v);
+}
+
+// v[q] *= w^q for q = 1 .. R-1, w^1, w^2, w^4, w^8 loaded (index k * step).
+template <typename T, int R>
+__device__ __forceinline__ void gen_twiddle(C2<T> *v, int at, const C2<T> *__restrict__ tw)
+{
+    const C2<T> w1 = tw[at];
+    v[1] = cmul(v[1], w1);
+    if constexpr (R > 2) {
+        const C2<T> w2 = tw[2 * at];
+        v[2] = cmul(v[2], w2);
+        const C2<T> w3 = cmul(w1, w2);
+        if constexpr (R > 3) v[3] = cmul(v[3], w3);
+        if constexpr (R > 4) {
+            const C2<T> w4 = tw[4 * at];
+            v[4] = cmul(v[4], w4);
+            if constexpr (R > 5) v[5] = cmul(v[5], cmul(w1, w4));
+            if constexpr (R > 6) v[6] = cmul(v[6], cmul(w2, w4));
+            const C2<T> w7 = cmul(w3, w4);
+            if constexpr (R > 7) v[7] = cmul(v[7], w7);
+            if constexpr (R > 8) {
+                const C2<T> w8 = tw[8 * at];
+                v[8] = cmul(v[8], w8);
+                if constexpr (R > 9) v[9] = cmul(v[9], cmul(w1, w8));
+                if constexpr (R > 10) v[10] = cmul(v[10], cmul(w2, w8));
+                if constexpr (R > 11) v[11] = cmul(v[11], cmul(w3, w8));
+                if constexpr (R > 12) {
+                    const C2<T> w12 = cmul(w4, w8);
+                    v[12] = cmul(v[12], w12);
+                    if constexpr (R > 13) v[13] = cmul(v[13], cmul(w1, w12));
+                    if constexpr (R > 14) v[14] = cmul(v[14], cmul(w2, w12));
+                    if constexpr (R > 15) v[15] = cmul(v[15], cmul(w7, w8));
+                }
+            }
+        }
+    }
 }
 
 template <typename T>
 struct GenCtx {
-    const GenPassDesc *gp;
     const GenAddr *a;
     const C2<T> *tw;
-    long long ntab;
     const C2<T> *in;
     C2<T> *out;
     C2<T> *lds;
-    size_t ibase, obase;
-    int s, g0, nvalid;
+    const unsigned char *occ;       // LDS: [g * tiles + tile] or [element], null: dense
+    int occ_stride, occ_shift;
+    int L, s, g0, nvalid;
     T scale;
 };
 
@@ -83,118 +283,164 @@ struct GenCtx {
 // memory.  Reads of a pass all complete (barrier) before its writes, so the
 // LDS buffer is used in place.
 template <typename T, int R>
-__device__ __forceinline__ void gen_pass(const GenCtx<T> &c, int Ns, bool first, bool last)
+__device__ __forceinline__ void gen_pass(const GenCtx<T> &c, const GenPass &ps, bool first,
+                                         bool last)
 {
-    constexpr int BPT = (kGenElems / R + kGenThreads - 1) / kGenThreads;
+    constexpr int BPT = gen_bpt(R);
     const GenAddr &a = *c.a;
-    const int L = c.gp->L, G = a.G, Lr = L / R, nb = G * Lr;
-    const int tid = threadIdx.x;
+    const int L = c.L, G = a.G, Lr = ps.Lr, Ns = ps.Ns, nb = G * Lr;
     C2<T> v[BPT][R];
-    int gj[BPT][2];
+    int gi[BPT], ji[BPT];
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
-        const int b = tid + i * kGenThreads;
-        gj[i][0] = -1;
+        const int b = threadIdx.x + i * blockDim.x;
+        gi[i] = -1;
+        ji[i] = 0;
         if (b < nb) {
             int g, j;
-            gen_map(b, Lr, G, a.line_major, g, j);
-            gj[i][0] = g;
-            gj[i][1] = j;
+            if (a.line_major) {
+                g = gen_div(b, ps.mLr);
+                j = b - g * Lr;
+            } else {
+                j = gen_div(b, a.mG);
+                g = b - j * G;
+            }
+            gi[i] = g;
+            ji[i] = j;
+            if (first) {
+                const C2<T> *p = c.in + (size_t)g * a.pg_in + (size_t)j * a.pe_in;
+                const size_t step = (size_t)Lr * a.pe_in;
+                const unsigned char *oc = c.occ ? c.occ + g * c.occ_stride : nullptr;
+                const bool there = g < c.nvalid;
 #pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const int n = j + q * Lr;
-                if (first)
-                    v[i][q] = g < c.nvalid ? c.in[c.ibase + (size_t)g * a.pg_in + (size_t)n * a.pe_in]
-                                           : C2<T>{T(0), T(0)};
-                else
-                    v[i][q] = c.lds[gen_lds(g, n, L, G, a.line_major)];
+                for (int q = 0; q < R; ++q) {
+                    const bool live =
+                        there && (oc == nullptr || oc[(j + q * Lr) >> c.occ_shift]);
+                    v[i][q] = live ? load_stream2(p + q * step) : C2<T>{T(0), T(0)};
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < R; ++q)
+                    v[i][q] = c.lds[gen_lds(g, j + q * Lr, L, G, a.line_major)];
             }
         }
     }
     if (!first) __syncthreads();
-    C2<T> w[R];
-    if constexpr (R == 7 || R == 11 || R == 13) {
-        w[0] = C2<T>{T(1), T(0)};
-#pragma unroll
-        for (int m = 1; m < R; ++m) w[m] = c.tw[(size_t)m * (size_t)(c.ntab / R)];
-    }
-    const long long tstep = c.ntab / ((long long)Ns * R);
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
-        const int g = gj[i][0];
+        const int g = gi[i];
         if (g < 0) continue;
-        const int j = gj[i][1], k = j % Ns;
-        if (Ns > 1) {
-#pragma unroll
-            for (int q = 1; q < R; ++q)
-                v[i][q] = cmul(v[i][q], c.tw[(size_t)((long long)k * q * tstep)]);
+        const int j = ji[i];
+        int dbase = j * R;
+        if (!first) {
+            const int jq = gen_div(j, ps.mNs), k = j - jq * Ns;
+            gen_twiddle<T, R>(v[i], k * ps.tstep, c.tw);
+            dbase = jq * (Ns * R) + k;
         }
-        if constexpr (R == 2 || R == 4 || R == 8 || R == 16) dftR<T, R>(v[i]);
-        else if constexpr (R == 3) dft3(v[i]);
-        else if constexpr (R == 5) dft5(v[i]);
-        else dft_direct<T, R>(v[i], w);
-        const int dbase = (j / Ns) * Ns * R + k;
+        dft_mix<T, R>(v[i]);
+        if (!last) {
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+                c.lds[gen_lds(g, dbase + q * Ns, L, G, a.line_major)] = v[i][q];
+            continue;
+        }
+        if (g >= c.nvalid) continue;   // (its twiddle index would pass the table)
+        C2<T> *p = c.out + (size_t)g * a.pg_out + (size_t)dbase * a.pe_out;
+        const size_t step = (size_t)Ns * a.pe_out;
+        const int e = a.tw_by == 1 ? c.s : c.g0 + g;
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-            const int n = dbase + q * Ns;
-            if (last) {
-                if (g >= c.nvalid) continue;   // (its twiddle index would pass the table)
-                C2<T> o = v[i][q];
-                if (a.tw_by) {
-                    const long long e = a.tw_by == 1 ? c.s : c.g0 + g;
-                    o = cmul(o, c.tw[(size_t)((long long)n * e)]);
-                }
-                o.x *= c.scale;
-                o.y *= c.scale;
-                c.out[c.obase + (size_t)g * a.pg_out + (size_t)n * a.pe_out] = o;
-            } else {
-                c.lds[gen_lds(g, n, L, G, a.line_major)] = v[i][q];
-            }
+            C2<T> o = v[i][q];
+            if (a.tw_by) o = cmul(o, c.tw[(dbase + q * Ns) * e]);
+            o.x *= c.scale;
+            o.y *= c.scale;
+            store_stream2(o, p + q * step);
         }
     }
     if (!last) __syncthreads();
 }
 
-template <typename T>
+// Passes of one workgroup.  A thread holds one butterfly of a radix above 8 (16
+// values at most) or as many smaller ones as make 16 values, so a pass needs no
+// more registers than its largest radix (132 VGPRs in FP64, 3 waves per SIMD;
+// 243 and 2 when each thread held up to 4096 / R / 256 butterflies), and all
+// index divisions are by constants formed on the host.  Bound by memory now:
+// column pass A of 8 planes of 3000^2 FP64 moves 2.3 GB in 0.51 ms where half
+// its rows are live, rows 0.35 ms over the live ones (before, dense: 2.0 ms the
+// columns, 1.33 ms the rows).  HARD: the instance with radices 11 and 13, whose
+// registers the lengths without them do not pay for.
+template <typename T, bool HARD>
 __global__ void __launch_bounds__(kGenThreads)
-k_fft_gen(GenPassDesc gp, GenAddr a, const C2<T> *__restrict__ tw, long long ntab, const C2<T> *in,
-          C2<T> *out, T scale)
+k_fft_gen(GenPassDesc gp, GenAddr a, const C2<T> *__restrict__ tw, const C2<T> *in, C2<T> *out,
+          T scale, GenOcc oc, int occ_off)
 {
-    __shared__ C2<T> lds[kGenElems];
+    extern __shared__ double gen_smem[];
     const unsigned bid = blockIdx.x;
     const int grp = (int)(bid % (unsigned)a.ngroups);
     const unsigned rest = bid / (unsigned)a.ngroups;
     const int s = (int)(rest % (unsigned)a.sets);
     const size_t z = rest / (unsigned)a.sets;
     GenCtx<T> c;
-    c.gp = &gp;
     c.a = &a;
     c.tw = tw;
-    c.ntab = ntab;
-    c.in = in;
-    c.out = out;
-    c.lds = lds;
+    c.lds = reinterpret_cast<C2<T> *>(gen_smem);
+    c.L = gp.L;
     c.s = s;
     c.g0 = grp * a.G;
     c.nvalid = min(a.G, a.nl - c.g0);
-    c.ibase = z * (size_t)a.pz + (size_t)s * (size_t)a.ps_in + (size_t)c.g0 * (size_t)a.pg_in;
-    c.obase = z * (size_t)a.pz + (size_t)s * (size_t)a.ps_out + (size_t)c.g0 * (size_t)a.pg_out;
+    c.in = in + z * (size_t)a.pz + (size_t)s * (size_t)a.ps_in + (size_t)c.g0 * (size_t)a.pg_in;
+    c.out = out + z * (size_t)a.pz + (size_t)s * (size_t)a.ps_out + (size_t)c.g0 * (size_t)a.pg_out;
     c.scale = scale;
-    int Ns = 1;
+    c.occ = nullptr;
+    c.occ_stride = c.occ_shift = 0;
+    if (oc.rows) {
+        unsigned char *occ = reinterpret_cast<unsigned char *>(gen_smem) + occ_off;
+        const unsigned char *rows = oc.rows + z * (size_t)oc.ny;
+        if (oc.offsets) {
+            // Rows g0 .. of plane z: none live -> their transforms are zero,
+            // neither computed nor written; else the tiles of the live ones.
+            int live = 0;
+            for (int g = threadIdx.x; g < c.nvalid; g += blockDim.x) live |= rows[c.g0 + g];
+            if (!__syncthreads_or(live)) return;
+            for (int i = threadIdx.x; i < c.nvalid * oc.tiles_u; i += blockDim.x) {
+                const int g = i / oc.tiles_u, t = i - g * oc.tiles_u, v = c.g0 + g;
+                const size_t b = (z * oc.tiles_v + v / oc.tv) * oc.tiles_u + t;
+                occ[i] = rows[v] && oc.offsets[b] != oc.offsets[b + 1];
+            }
+            c.occ_stride = oc.tiles_u;
+            c.occ_shift = oc.tu_shift;
+        } else {
+            // Columns: the flags of this set's input rows.
+            for (int n = threadIdx.x; n < gp.L; n += blockDim.x)
+                occ[n] = rows[s * a.set_mul + n * a.row_mul];
+        }
+        c.occ = occ;
+        __syncthreads();
+    }
     for (int p = 0; p < gp.np; ++p) {
         const bool first = p == 0, last = p == gp.np - 1;
-        switch (gp.rad[p]) {
-            case 16: gen_pass<T, 16>(c, Ns, first, last); break;
-            case 8: gen_pass<T, 8>(c, Ns, first, last); break;
-            case 4: gen_pass<T, 4>(c, Ns, first, last); break;
-            case 2: gen_pass<T, 2>(c, Ns, first, last); break;
-            case 3: gen_pass<T, 3>(c, Ns, first, last); break;
-            case 5: gen_pass<T, 5>(c, Ns, first, last); break;
-            case 7: gen_pass<T, 7>(c, Ns, first, last); break;
-            case 11: gen_pass<T, 11>(c, Ns, first, last); break;
-            default: gen_pass<T, 13>(c, Ns, first, last); break;
+        const GenPass &ps = gp.pass[p];
+        switch (ps.R) {
+            case 16: gen_pass<T, 16>(c, ps, first, last); break;
+            case 15: gen_pass<T, 15>(c, ps, first, last); break;
+            case 14: gen_pass<T, 14>(c, ps, first, last); break;
+            case 12: gen_pass<T, 12>(c, ps, first, last); break;
+            case 10: gen_pass<T, 10>(c, ps, first, last); break;
+            case 9: gen_pass<T, 9>(c, ps, first, last); break;
+            case 8: gen_pass<T, 8>(c, ps, first, last); break;
+            case 7: gen_pass<T, 7>(c, ps, first, last); break;
+            case 6: gen_pass<T, 6>(c, ps, first, last); break;
+            case 5: gen_pass<T, 5>(c, ps, first, last); break;
+            case 4: gen_pass<T, 4>(c, ps, first, last); break;
+            case 3: gen_pass<T, 3>(c, ps, first, last); break;
+            case 2: gen_pass<T, 2>(c, ps, first, last); break;
+            default:
+                if constexpr (HARD) {
+                    if (ps.R == 11) gen_pass<T, 11>(c, ps, first, last);
+                    else gen_pass<T, 13>(c, ps, first, last);
+                }
+                break;
         }
-        Ns *= gp.rad[p];
     }
 }
 
@@ -244,33 +490,66 @@ k_blue_post(const C2<T> *__restrict__ w, int cl, int N, int M, const C2<T> *__re
 // ---------------------------------------------------------------------------
 // Host side.
 
-// Radices of a direct length (largest first); false if L has a prime factor
-// above 13 or needs more passes than the descriptor holds.
+// Radices of a direct length: the fewest passes, then the largest smallest
+// radix (a small radix leaves lanes idle between the larger ones).  False if L
+// has a prime factor above 13.
+void gen_search(int rest, int max_r, std::vector<int> &cur, std::vector<int> &best)
+{
+    if (rest == 1) {
+        if (best.empty() || cur.size() < best.size() ||
+            (cur.size() == best.size() && cur.back() > best.back()))
+            best = cur;
+        return;
+    }
+    if (!best.empty() && cur.size() >= best.size()) return;
+    for (int r = std::min(max_r, rest); r >= 2; --r)
+        if (rest % r == 0) {
+            cur.push_back(r);
+            gen_search(rest / r, r, cur, best);
+            cur.pop_back();
+        }
+}
+
 bool gen_radices(int L, GenPassDesc &gp)
 {
+    gp = GenPassDesc{};
     gp.L = L;
-    gp.np = 0;
-    if (L < 1 || L > kGenElems) return false;
-    int r = L;
-    auto push = [&](int x) {
-        if (gp.np >= kGenMaxPasses) return false;
-        gp.rad[gp.np++] = x;
-        return true;
-    };
-    while (r % 16 == 0)
-        if (!push(16)) return false; else r /= 16;
-    for (int p2 : {8, 4, 2})
-        if (r % p2 == 0) {
-            if (!push(p2)) return false;
-            r /= p2;
-            break;
-        }
-    for (int p : {3, 5, 7, 11, 13})
-        while (r % p == 0) {
-            if (!push(p)) return false;
-            r /= p;
-        }
-    return r == 1 && gp.np > 0;
+    if (L < 2 || L > kGenElems) return false;
+    std::vector<int> cur, best;
+    gen_search(L, kGenValues, cur, best);
+    if (best.empty() || (int)best.size() > kGenMaxPasses) return false;
+    int Ns = 1;
+    for (int r : best) {
+        GenPass &ps = gp.pass[gp.np++];
+        ps.R = r;
+        ps.Ns = Ns;
+        ps.Lr = L / r;
+        ps.mNs = gen_magic((uint32_t)Ns);
+        ps.mLr = gen_magic((uint32_t)ps.Lr);
+        Ns *= r;
+    }
+    return true;
+}
+
+// Threads that G lines of this plan take (0: more than a workgroup has).
+int gen_threads(const GenPassDesc &gp, int G)
+{
+    int need = 1;
+    for (int p = 0; p < gp.np; ++p) {
+        const int nb = G * gp.pass[p].Lr, bpt = gen_bpt(gp.pass[p].R);
+        need = std::max(need, (nb + bpt - 1) / bpt);
+    }
+    return need > kGenThreads ? 0 : (need + 63) / 64 * 64;
+}
+
+// Lines per workgroup: as many as the threads and `elems` LDS elements take,
+// whole groups of 8 lines where lines are adjacent in memory (128-byte runs).
+int gen_lines(const GenPassDesc &gp, int nl, int elems, bool adjacent)
+{
+    int G = std::max(1, std::min(nl, elems / gp.L));
+    while (G > 1 && !gen_threads(gp, G)) --G;
+    if (adjacent && G > 8 && G < nl) G = G / 8 * 8;
+    return G;
 }
 
 bool smooth(long long n)
@@ -382,18 +661,101 @@ AxisGeom axis_geom(int axis, int nx, int ny)
 
 size_t csize(int precision) { return precision == RICK_FP64 ? 16 : 8; }
 
+// LDS elements of a workgroup's lines: two workgroups per CU in FP64, and as
+// many bytes in FP32 (longer runs of adjacent columns).
 template <typename T>
-hipError_t launch_gen(const GenPassDesc &gp, GenAddr a, long long planes, const void *tw,
-                      long long ntab, const void *in, void *out, double scale, hipStream_t s)
+constexpr int gen_elems() { return sizeof(T) == 8 ? 4096 : 8192; }
+
+template <typename T>
+hipError_t launch_gen(GenPassDesc gp, GenAddr a, long long planes, const void *tw,
+                      long long ntab, const void *in, void *out, double scale, hipStream_t s,
+                      const GenOcc &oc = GenOcc{})
 {
+    a.G = gen_lines(gp, a.nl, gen_elems<T>(), !a.line_major);
+    a.mG = gen_magic((uint32_t)a.G);
     a.ngroups = (a.nl + a.G - 1) / a.G;
+    const int nt = gen_threads(gp, a.G);
+    if (!nt) return hipErrorInvalidConfiguration;
+    bool hard = false;
+    for (int p = 0; p < gp.np; ++p) {
+        gp.pass[p].tstep = (int)(ntab / ((long long)gp.pass[p].Ns * gp.pass[p].R));
+        hard |= gp.pass[p].R == 11 || gp.pass[p].R == 13;
+    }
     const unsigned long long blocks = (unsigned long long)a.ngroups * a.sets * planes;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffull) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_fft_gen<T>, dim3((unsigned)blocks), dim3(kGenThreads), 0, s, gp, a,
-                       static_cast<const C2<T> *>(tw), ntab, static_cast<const C2<T> *>(in),
-                       static_cast<C2<T> *>(out), (T)scale);
+    size_t lds = a.line_major ? (size_t)a.G * (gen_pad(gp.L) + 1) : (size_t)a.G * gp.L;
+    if (gp.np == 1) lds = 0;   // no exchange
+    lds *= sizeof(C2<T>);
+    const int occ_off = (int)lds;
+    if (oc.rows) lds += (size_t)(oc.offsets ? a.G * oc.tiles_u : gp.L) + 16;
+    if (lds > (size_t)kGenLdsBytes) return hipErrorInvalidConfiguration;
+    auto kernel = hard ? k_fft_gen<T, true> : k_fft_gen<T, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(nt), lds, s, gp, a,
+                       static_cast<const C2<T> *>(tw), static_cast<const C2<T> *>(in),
+                       static_cast<C2<T> *>(out), (T)scale, oc, occ_off);
     return hipGetLastError();
+}
+
+// Addresses of a direct axis, and of the two passes of a four-step axis
+// (n = n1 * n2): A reads elements n2 + N2*n1 and writes them, times
+// W_N^(k1*n2), at n2 + N2*k1; B reads N2*k1 + n2 and writes X[k1 + N1*k2] at
+// that element, or (in_place) at N2*k1 + k2.
+GenAddr direct_addr(const AxisGeom &ag, bool rows, long long plane_elems)
+{
+    GenAddr a{};
+    a.nl = ag.nl;
+    a.sets = 1;
+    a.pz = plane_elems;
+    a.pg_in = a.pg_out = ag.ls;
+    a.pe_in = a.pe_out = ag.es;
+    a.line_major = rows ? 1 : 0;
+    a.row_mul = 1;
+    return a;
+}
+
+GenAddr step_a_addr(const GenAxis &ax, const AxisGeom &ag, bool rows, long long plane_elems)
+{
+    GenAddr A{};
+    const int N2 = ax.n2;
+    A.pz = plane_elems;
+    if (rows) {
+        A.nl = N2; A.sets = ag.nl;
+        A.pg_in = A.pg_out = 1;
+        A.ps_in = A.ps_out = ag.ls;
+        A.pe_in = A.pe_out = (long long)N2;
+        A.tw_by = 2;
+    } else {
+        A.nl = ag.nl; A.sets = N2;
+        A.pg_in = A.pg_out = ag.ls;
+        A.ps_in = A.ps_out = ag.es;
+        A.pe_in = A.pe_out = (long long)N2 * ag.es;
+        A.tw_by = 1;
+        A.row_mul = N2;
+        A.set_mul = 1;
+    }
+    return A;
+}
+
+GenAddr step_b_addr(const GenAxis &ax, const AxisGeom &ag, bool rows, long long plane_elems,
+                    bool in_place)
+{
+    GenAddr B{};
+    const int N1 = ax.n1, N2 = ax.n2;
+    B.pz = plane_elems;
+    if (rows) {
+        B.nl = N1; B.sets = ag.nl;
+        B.pg_in = N2; B.pe_in = 1; B.ps_in = ag.ls;
+        B.pg_out = 1; B.pe_out = N1; B.ps_out = ag.ls;
+        B.line_major = 1;
+    } else {
+        B.nl = ag.nl; B.sets = N1;
+        B.pg_in = B.pg_out = ag.ls;
+        B.ps_in = (long long)N2 * ag.es; B.pe_in = ag.es;
+        B.ps_out = in_place ? B.ps_in : ag.es;
+        B.pe_out = in_place ? B.pe_in : (long long)N1 * ag.es;
+    }
+    return B;
 }
 
 // One smooth axis transform of `planes` planes (direct: all planes in one
@@ -404,60 +766,53 @@ hipError_t smooth_axis(const GenAxis &ax, const AxisGeom &ag, bool rows, int pla
                        C2<T> *tmp, double scale, hipStream_t s)
 {
     const int n = ag.n;
-    if (ax.mode == 0) {
-        GenAddr a{};
-        a.nl = ag.nl;
-        a.G = std::max(1, std::min(ag.nl, kGenElems / n));
-        a.sets = 1;
-        a.pz = plane_elems;
-        a.pg_in = a.pg_out = ag.ls;
-        a.pe_in = a.pe_out = ag.es;
-        a.line_major = rows ? 1 : 0;
-        return launch_gen<T>(ax.a, a, planes, tw, n, in, out, scale, s);
-    }
-    const int N1 = ax.n1, N2 = ax.n2;
+    if (ax.mode == 0)
+        return launch_gen<T>(ax.a, direct_addr(ag, rows, plane_elems), planes, tw, n, in, out,
+                             scale, s);
+    const GenAddr A = step_a_addr(ax, ag, rows, 0), B = step_b_addr(ax, ag, rows, 0, false);
     for (int z = 0; z < planes; ++z) {
-        const C2<T> *src = in + (size_t)z * plane_elems;
-        C2<T> *dst = out + (size_t)z * plane_elems;
-        // Pass A: N1-point DFTs over elements n2 + N2*n1 -> tmp at n2 + N2*k1,
-        // times W_N^(k1*n2).
-        GenAddr A{};
-        if (rows) {
-            A.nl = N2; A.sets = ag.nl;
-            A.pg_in = A.pg_out = 1;
-            A.ps_in = A.ps_out = ag.ls;
-            A.pe_in = A.pe_out = (long long)N2;
-            A.tw_by = 2;
-        } else {
-            A.nl = ag.nl; A.sets = N2;
-            A.pg_in = A.pg_out = ag.ls;
-            A.ps_in = A.ps_out = ag.es;
-            A.pe_in = A.pe_out = (long long)N2 * ag.es;
-            A.tw_by = 1;
-        }
-        A.G = std::max(1, std::min(A.nl, kGenElems / N1));
-        A.line_major = 0;
-        hipError_t e = launch_gen<T>(ax.a, A, 1, tw, n, src, tmp, 1.0, s);
+        const size_t at = (size_t)z * plane_elems;
+        hipError_t e = launch_gen<T>(ax.a, A, 1, tw, n, in + at, tmp, 1.0, s);
         if (e != hipSuccess) return e;
-        // Pass B: N2-point DFTs over tmp elements N2*k1 + n2 -> X[k1 + N1*k2].
-        GenAddr B{};
-        if (rows) {
-            B.nl = N1; B.sets = ag.nl;
-            B.pg_in = N2; B.pe_in = 1; B.ps_in = ag.ls;
-            B.pg_out = 1; B.pe_out = N1; B.ps_out = ag.ls;
-            B.line_major = 1;
-        } else {
-            B.nl = ag.nl; B.sets = N1;
-            B.pg_in = B.pg_out = ag.ls;
-            B.ps_in = (long long)N2 * ag.es; B.pe_in = ag.es;
-            B.ps_out = ag.es; B.pe_out = (long long)N1 * ag.es;
-            B.line_major = 0;
-        }
-        B.G = std::max(1, std::min(B.nl, kGenElems / N2));
-        e = launch_gen<T>(ax.b, B, 1, tw, n, tmp, dst, scale, s);
+        e = launch_gen<T>(ax.b, B, 1, tw, n, tmp, out + at, scale, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// The transform of the image chain on a sparse grid, in place: live rows over
+// their occupied tiles, then the columns reading the other rows as zero.  A
+// four-step column axis leaves X[k1 + N1*k2] in row N2*k1 + k2.
+template <typename T>
+hipError_t gen_chain(const GenFft &g, int planes, int nx, int ny, void *grid_v, double scale,
+                     hipStream_t s, Timing *tm, const GridGeom &geom, const uint32_t *offsets,
+                     const unsigned char *rowlive)
+{
+    C2<T> *grid = static_cast<C2<T> *>(grid_v);
+    const long long plane = (long long)nx * ny;
+    const AxisGeom ag0 = axis_geom(0, nx, ny), ag1 = axis_geom(1, nx, ny);
+    const GenAxis &ay = g.ax[1];
+    GenOcc oc{offsets, rowlive, geom.tu_shift, geom.tv, geom.tiles_u, geom.tiles_v, ny};
+    tm->begin(RICK_STAGE_FFT_ROWS, s);
+    hipError_t e = launch_gen<T>(g.ax[0].a, direct_addr(ag0, true, plane), planes, g.ax[0].tw, nx,
+                                 grid, grid, scale, s, oc);
+    tm->end(RICK_STAGE_FFT_ROWS, s);
+    if (e != hipSuccess) return e;
+    oc.offsets = nullptr;
+    tm->begin(RICK_STAGE_FFT_COLS, s);
+    if (ay.mode == 0)
+        e = launch_gen<T>(ay.a, direct_addr(ag1, false, plane), planes, ay.tw, ny, grid, grid,
+                          1.0, s, oc);
+    else
+        e = launch_gen<T>(ay.a, step_a_addr(ay, ag1, false, plane), planes, ay.tw, ny, grid, grid,
+                          1.0, s, oc);
+    tm->end(RICK_STAGE_FFT_COLS, s);
+    if (e != hipSuccess || ay.mode == 0) return e;
+    tm->begin(RICK_STAGE_FFT_COLS_B, s);
+    e = launch_gen<T>(ay.b, step_b_addr(ay, ag1, false, plane, true), planes, ay.tw, ny, grid,
+                      grid, 1.0, s);
+    tm->end(RICK_STAGE_FFT_COLS_B, s);
+    return e;
 }
 
 template <typename T>
@@ -567,6 +922,15 @@ bool gen_fft_prepare(int nx, int ny, int precision, GenFft *g)
 
 hipError_t gen_fft_upload(GenFft *g, int precision, void *tables, void *work)
 {
+    // Padded lines of 4096 FP64 elements take 69 KB of LDS.
+    for (const void *k : {reinterpret_cast<const void *>(&k_fft_gen<double, false>),
+                          reinterpret_cast<const void *>(&k_fft_gen<double, true>),
+                          reinterpret_cast<const void *>(&k_fft_gen<float, false>),
+                          reinterpret_cast<const void *>(&k_fft_gen<float, true>)}) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 kGenLdsBytes);
+        if (e != hipSuccess) return e;
+    }
     char *p = static_cast<char *>(tables);
     const size_t cs = csize(precision);
     auto put = [&](const std::vector<long double> &v, size_t n) -> const void * {
@@ -618,6 +982,25 @@ hipError_t gen_fft_upload(GenFft *g, int precision, void *tables, void *work)
     }
     g->work = work;
     return hipSuccess;
+}
+
+bool gen_chain_ok(const GenFft &g)
+{
+    return g.ax[0].mode == 0 && g.ax[1].mode != 2;
+}
+
+hipError_t launch_gen_chain(const GenFft &g, int precision, int planes, int nx, int ny, void *grid,
+                            double scale, hipStream_t s, Timing *tm, const GridGeom &geom,
+                            const uint32_t *offsets, const unsigned char *rowlive, int *row_n1,
+                            int *row_n2)
+{
+    Timing off;
+    if (tm == nullptr) tm = &off;
+    *row_n1 = g.ax[1].mode == 1 ? g.ax[1].n1 : 1;
+    *row_n2 = g.ax[1].mode == 1 ? g.ax[1].n2 : 0;
+    if (precision == RICK_FP64)
+        return gen_chain<double>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive);
+    return gen_chain<float>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive);
 }
 
 hipError_t launch_fft_gen(const GenFft &g, int precision, int planes, int nx, int ny,

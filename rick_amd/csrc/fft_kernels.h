@@ -138,22 +138,5 @@ __device__ __forceinline__ void dft5(C2<T> *v)
     v[3] = csub(r2, i2);
 }
 
-// Any radix R by direct summation, with the R-th roots of unity w[m] =
-// exp(+2 pi i m/R) supplied by the caller (R = 7, 11, 13 here).
-template <typename T, int R>
-__device__ __forceinline__ void dft_direct(C2<T> *v, const C2<T> *w)
-{
-    C2<T> out[R];
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        C2<T> acc = v[0];
-#pragma unroll
-        for (int n = 1; n < R; ++n) acc = cadd(acc, cmul(v[n], w[(n * k) % R]));
-        out[k] = acc;
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) v[k] = out[k];
-}
-
 }  // namespace fftk
 }  // namespace rick

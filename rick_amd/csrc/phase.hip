@@ -28,18 +28,20 @@ constexpr int kBlk = 256;
 template <int PREC>
 __global__ void __launch_bounds__(kBlk)
 k_phase(PhaseGeom g, const void *__restrict__ gridss_v, double *__restrict__ ore,
-        double *__restrict__ oim, int accumulate)
+        double *__restrict__ oim, int accumulate, int row_n1, int row_n2)
 {
     const int iu = blockIdx.x * kBlk + threadIdx.x;
     const int iv = blockIdx.y;
     if (iu >= g.nx) return;
     const size_t pix = (size_t)iv * g.nx + iu;
+    const int row = row_n2 ? (iv % row_n1) * row_n2 + iv / row_n1 : iv;
+    const size_t cell = (size_t)row * g.nx + iu;
     const size_t plane = (size_t)g.nx * g.ny;
     double acc_re = 0.0, acc_im = 0.0;
     const bool phase = g.phase_on && g.planes > 1;
     const double n = phase ? pixel_n(g.ltab[iu], g.mtab[iv]) : 1.0;
     for (int iw = 0; iw < g.planes; ++iw) {
-        const size_t idx = pix + (size_t)iw * plane;
+        const size_t idx = cell + (size_t)iw * plane;
         if constexpr (PREC == RICK_FP64) {
             const double2 v = reinterpret_cast<const double2 *>(gridss_v)[idx];
             if (phase) phase_add_f64(v.x, v.y, g.wmin + iw * g.dw, n, g.dwnorm, acc_re, acc_im);
@@ -72,14 +74,17 @@ k_phase(PhaseGeom g, const void *__restrict__ gridss_v, double *__restrict__ ore
 }  // namespace
 
 hipError_t launch_phase(const PhaseGeom &g, int precision, const void *gridss, double *re,
-                        double *im, int accumulate, hipStream_t s, Timing *tm)
+                        double *im, int accumulate, hipStream_t s, Timing *tm, int row_n1,
+                        int row_n2)
 {
     const dim3 grd((g.nx + kBlk - 1) / kBlk, g.ny), blk(kBlk);
     if (tm) tm->begin(RICK_STAGE_PHASE, s);
     if (precision == RICK_FP64)
-        hipLaunchKernelGGL(k_phase<RICK_FP64>, grd, blk, 0, s, g, gridss, re, im, accumulate);
+        hipLaunchKernelGGL(k_phase<RICK_FP64>, grd, blk, 0, s, g, gridss, re, im, accumulate,
+                           row_n1, row_n2);
     else
-        hipLaunchKernelGGL(k_phase<RICK_FP32>, grd, blk, 0, s, g, gridss, re, im, accumulate);
+        hipLaunchKernelGGL(k_phase<RICK_FP32>, grd, blk, 0, s, g, gridss, re, im, accumulate,
+                           row_n1, row_n2);
     if (tm) tm->end(RICK_STAGE_PHASE, s);
     return hipGetLastError();
 }

@@ -203,10 +203,15 @@ hipError_t launch_fft(const FftPlan &p, int precision, const void *in, void *out
 
 // FFT of any axis lengths >= 2 (mixed radix 2..16, 3, 5, 7, 11, 13 in
 // LDS; four-step for long or strided axes; Bluestein for other primes).
-constexpr int kGenMaxPasses = 16;
+constexpr int kGenMaxPasses = 8;
+struct GenPass {
+    int R, Ns, Lr;                  // radix, product of the earlier radices, L / R
+    uint32_t mNs, mLr;              // their division constants (gen_magic)
+    int tstep;                      // table length / (Ns * R), set at launch
+};
 struct GenPassDesc {
     int L, np;                      // line length and its passes
-    int rad[kGenMaxPasses];         // radix of each pass
+    GenPass pass[kGenMaxPasses];
 };
 struct GenAxis {
     int n;                          // axis length
@@ -228,6 +233,15 @@ bool gen_fft_prepare(int nx, int ny, int precision, GenFft *g);
 // Writes the tables (synchronously) at `tables` (table_bytes) and records the
 // scratch `work` (work_bytes).
 hipError_t gen_fft_upload(GenFft *g, int precision, void *tables, void *work);
+// Image-chain transform of a sparse grid in place (axes for which
+// gen_chain_ok): rows without a flag in rowlive are read as zero, tiles by the
+// bucket offsets.  Image row v is then in grid row (v % n1) * n2 + v / n1
+// (*row_n2 == 0: in row v).
+bool gen_chain_ok(const GenFft &g);
+hipError_t launch_gen_chain(const GenFft &g, int precision, int planes, int nx, int ny, void *grid,
+                            double scale, hipStream_t s, Timing *tm, const GridGeom &geom,
+                            const uint32_t *offsets, const unsigned char *rowlive, int *row_n1,
+                            int *row_n2);
 // Per-plane backward 2-D transform, in == out allowed, scaled.
 hipError_t launch_fft_gen(const GenFft &g, int precision, int planes, int nx, int ny,
                           const void *in, void *out, double scale, hipStream_t s, Timing *tm);
@@ -239,8 +253,10 @@ struct PhaseGeom {
     int phase_on;
     const double *ltab, *mtab;  // device: sin(xcoord*resolution) per u / per v index
 };
+// With row_n2 > 0 image row v is read from grid row (v % row_n1) * row_n2 + v / row_n1.
 hipError_t launch_phase(const PhaseGeom &p, int precision, const void *gridss, double *re,
-                        double *im, int accumulate, hipStream_t s, Timing *tm);
+                        double *im, int accumulate, hipStream_t s, Timing *tm, int row_n1 = 1,
+                        int row_n2 = 0);
 
 // Image chain after gridding, in place on grid (clobbered) and without
 // scratch: row FFT reading only the tiles whose gridder bucket holds records

@@ -1,0 +1,69 @@
+"""Transforms of axes beside the power-of-two engine: every radix, the longest
+and shortest one-pass lines, and the image chain on a sparse grid of such a
+size against the separate stages on a dense one.
+
+Bars: the suite's 1e-14 / 2e-6 relative L2 for a transform against numpy, and
+1e-12 (FP64) / 1e-5 (FP32) for images."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import rel_l2
+import rick_amd
+from rick_amd import FP32, FP64, Plan
+
+pytestmark = pytest.mark.gpu
+
+
+def cube(plan, flat):
+    c = flat.cpu().numpy().astype(np.float64).reshape(plan.planes, plan.ny, plan.nx, 2)
+    return c[..., 0] + 1j * c[..., 1]
+
+
+@pytest.mark.parametrize("nx,ny,planes", [
+    (196, 81, 2), (240, 143, 1), (176, 156, 3), (4095, 12, 1), (3993, 14, 1), (4096, 100, 1),
+    (3584, 18, 2), (130, 520, 2), (20, 3600, 1), (33, 257 * 2, 1), (17, 300, 1)])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_lengths_of_every_radix_match_numpy(nx, ny, planes, precision):
+    print(f"case fft {nx}x{ny}x{planes} precision={precision}", flush=True)
+    plan = Plan(nx, ny, planes, precision=precision)
+    rng = np.random.default_rng(nx + 7 * ny)
+    src = torch.from_numpy(rng.normal(size=2 * planes * ny * nx)).to("cuda", plan.grid_dtype)
+    want = np.fft.ifft2(cube(plan, src), axes=(1, 2))
+    out = plan.fft(src, torch.empty_like(src))
+    assert rel_l2(cube(plan, out), want) <= (1e-14 if precision == FP64 else 2e-6)
+    plan.fft(src)   # in place
+    assert rel_l2(cube(plan, src), want) <= (1e-14 if precision == FP64 else 2e-6)
+
+
+# Rows in thin v-stripes that start and end inside tile rows, the whole grid
+# width or a part of it; the grid starts as NaN, so a cell that the sparse
+# chain reads without having written it shows.
+@pytest.mark.parametrize("nx,ny,planes,tile", [
+    (18, 300, 3, (32, 32)), (300, 200, 4, (64, 32)), (130, 600, 3, (64, 64)),
+    (143, 169, 2, (0, 0)), (1000, 1500, 2, (128, 32)), (4095, 66, 2, (32, 64)),
+    (12, 14, 1, (0, 0)), (100, 512, 2, (64, 64))])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_sparse_chain_matches_separate_stages(nx, ny, planes, tile, precision):
+    print(f"case chain {nx}x{ny}x{planes} tile={tile} precision={precision}", flush=True)
+    n = 20000
+    plan = Plan(nx, ny, planes, kernel=rick_amd.KAISERBESSEL, support=7, precision=precision,
+                max_points=n, tile=tile, resolution=1.0 / (4.0 * max(nx, ny)), wmin=-300.0,
+                wmax=500.0)
+    for call in range(2):
+        rng = np.random.default_rng(11 + call)
+        uu = rng.uniform(0.1 * call, 0.9, n)
+        vv = (rng.choice([0.13, 0.47, 0.71], n) + rng.uniform(0.0, 0.04, n)) * ny / nx
+        ww = rng.uniform(0.0, 0.6, n)             # the last planes stay empty
+        ins = [torch.from_numpy(a).to("cuda") for a in (
+            uu, vv, ww, rng.normal(size=n).astype(np.float32),
+            rng.normal(size=n).astype(np.float32), np.ones(n, np.float32))]
+        grid = plan.new_grid()
+        grid.fill_(float("nan"))
+        re, im, _ = plan.image(*ins, grid=grid)
+        dense = plan.grid(*ins)
+        plan.fft(dense)
+        wre, wim = plan.phase(dense)
+        got, want = ((a.cpu().numpy() + 1j * b.cpu().numpy()) for a, b in ((re, im), (wre, wim)))
+        assert np.isfinite(want).all() and np.abs(want).max() > 0
+        assert rel_l2(got, want) <= (1e-12 if precision == FP64 else 1e-5)
