@@ -344,8 +344,14 @@ constexpr int lines_per_wg(int L) { return L >= 4096 ? 1 : 4096 / L; }
 // Columns per workgroup of a plain column pass: FP32 lines of 64 or 128
 // elements take 8192 elements (512 threads), so each row segment a
 // workgroup reads or writes is 1 KB, as in FP64.
+// One-pass lines of 1024 points and more take 8 or 16 columns (col_strip pairs
+// the workgroups of half a 128-byte line).
 template <typename T>
-constexpr int col_lines(int L) { return sizeof(T) == 4 && L >= 64 && L <= 128 ? 8192 / L : lines_per_wg(L); }
+constexpr int col_lines(int L)
+{
+    if (L >= 1024) return sizeof(T) == 8 ? 8 : 16384 / L;
+    return sizeof(T) == 4 && L >= 64 && L <= 128 ? 8192 / L : lines_per_wg(L);
+}
 constexpr int lds_elems(int L, bool rows)
 {
     return rows ? lines_per_wg(L) * (lpad(L) + 1) : lines_per_wg(L) * L;
@@ -472,17 +478,29 @@ struct ColArgs {
     int ts;                        // table stride for the L-point DFT
 };
 
+// Strip of workgroup x.  Strips narrower than a 128-byte line share lines with
+// their neighbour: workgroups x and x + 8, which the round-robin over the eight
+// XCDs puts behind one L2, take neighbouring strips.
+template <typename T, int G>
+__device__ __forceinline__ int col_strip(int x, int n)
+{
+    if constexpr (G * sizeof(C2<T>) >= 128) return x;
+    const int base = x & ~15, r = x & 15;
+    return base + 16 <= n ? base + (r & 7) * 2 + (r >> 3) : x;
+}
+
 template <typename T, int L, int G, int E>
 __global__ void __launch_bounds__(G * L / E)
 k_fft_cols(ColArgs a, const C2<T> *__restrict__ tw, const C2<T> *gin, C2<T> *gout, T scale,
            ColOcc co)
 {
-    // FP64 only: an FP32 workgroup here (up to 1024 threads) is already at
-    // two per CU with whole exchanges, so halving its LDS adds none.
-    constexpr bool kSplit = sizeof(T) == 8;
+    // FP64 and long lines: an FP32 workgroup of a short line (up to 1024
+    // threads) is already at two per CU with whole exchanges, so halving its
+    // LDS adds none.
+    constexpr bool kSplit = sizeof(T) == 8 || L >= 1024;
     __shared__ C2<T> lds[kSplit ? G * L / 2 : G * L];
     __shared__ unsigned char rl[L];
-    const int c0 = blockIdx.x * G;
+    const int c0 = col_strip<T, G>(blockIdx.x, gridDim.x) * G;
     const int s = blockIdx.y;
     const size_t plane = (size_t)blockIdx.z * (size_t)a.nx * (size_t)a.ny;
     Lines ln;
@@ -736,20 +754,25 @@ template <typename T>
 hipError_t launch_cols(int L, const ColArgs &a, int sets, int planes, const C2<T> *tw,
                        const C2<T> *in, C2<T> *out, hipStream_t s, const ColOcc &co = ColOcc{})
 {
-#define RICK_COLS(LL)                                                                        \
-    case LL: {                                                                               \
+#define RICK_COLS_BODY(LL)                                                                   \
+    {                                                                                        \
         constexpr int G = col_lines<T>(LL);                                                  \
-        constexpr int E = col_values<T>();                                                   \
+        constexpr int E = LL >= 1024 ? kE : col_values<T>();                                 \
         hipLaunchKernelGGL((k_fft_cols<T, LL, G, E>), dim3((a.nx + G - 1) / G, sets, planes), \
                            dim3(G * LL / E), 0, s, a, tw, in, out, T(1), co);                \
         return hipGetLastError();                                                            \
     }
+#define RICK_COLS(LL) case LL: RICK_COLS_BODY(LL)
     switch (L) {
         RICK_COLS(16) RICK_COLS(32) RICK_COLS(64) RICK_COLS(128) RICK_COLS(256)
-        RICK_COLS(512)
+        RICK_COLS(512) RICK_COLS(1024)
+        case 2048:   // FP32 only: FP64 transforms of 2048 rows take two passes
+            if constexpr (sizeof(T) == 4) { RICK_COLS_BODY(2048) }
+            return hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 #undef RICK_COLS
+#undef RICK_COLS_BODY
 }
 
 template <typename T>
@@ -856,7 +879,8 @@ hipError_t image_chain_impl(const FftPlan &p, void *grid_v, double scale_d, hipS
     hipError_t e = launch_rows<T>(nx, planes * ny, twx, grid, grid, (T)scale_d, s, oc);
     tm->end(RICK_STAGE_FFT_ROWS, s);
     if (e != hipSuccess) return e;
-    if (!fft_needs_tmp(sizeof(T) == 8 ? RICK_FP64 : RICK_FP32, ny)) {
+    // (512-point lines keep >= 8 columns, >= 64 B, per row access.)
+    if (ny <= 512) {
         const ColArgs a{nx, ny, 0, 1, 0, 1, 0, 1};
         tm->begin(RICK_STAGE_PHASE, s);
         e = launch_cols_phase<T>(ny, a, 1, planes, twy, grid, pg, 0, 1, re, im, s, co, pj,
@@ -889,11 +913,11 @@ hipError_t image_chain_impl(const FftPlan &p, void *grid_v, double scale_d, hipS
 
 }  // namespace
 
-bool fft_needs_tmp(int precision, int ny)
-{
-    (void)precision;
-    return ny > 512;  // keeps >= 8 columns (>= 64 B) per row access in every pass
-}
+// One pass while a workgroup's columns make 64-byte runs and its values fit the
+// registers; else four-step.  In-place transform, one pass against two: 1024^2 x
+// 16 planes 391 -> 210 us (FP64), 294 -> 130 us (FP32); 2048^2 x 16 FP32 596 ->
+// 508 us, FP64 (64-byte runs) 1144 -> 1147 us, so FP64 stops at 1024 rows.
+bool fft_needs_tmp(int precision, int ny) { return ny > (precision == RICK_FP64 ? 1024 : 2048); }
 
 hipError_t launch_fft(const FftPlan &p, int precision, const void *in, void *out, void *tmp,
                       double scale, hipStream_t s, Timing *tm)

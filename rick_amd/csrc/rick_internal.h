@@ -195,8 +195,9 @@ struct FftPlan {
     int planes, nx, ny;
     const void *tw_x, *tw_y;   // device twiddle tables exp(+2 pi i m/N), N entries
 };
-// Long columns (ny above 512) use two passes; an in-place transform stages
-// each plane through tmp (one plane).  Output in natural row order.
+// Long columns (above 1024 rows in FP64, 2048 in FP32) take two passes; an
+// in-place transform then stages each plane through tmp (one plane).  Output in
+// natural row order.
 bool fft_needs_tmp(int precision, int ny);
 hipError_t launch_fft(const FftPlan &p, int precision, const void *in, void *out, void *tmp,
                       double scale, hipStream_t s, Timing *tm);

@@ -67,3 +67,20 @@ def test_sparse_chain_matches_separate_stages(nx, ny, planes, tile, precision):
         got, want = ((a.cpu().numpy() + 1j * b.cpu().numpy()) for a, b in ((re, im), (wre, wim)))
         assert np.isfinite(want).all() and np.abs(want).max() > 0
         assert rel_l2(got, want) <= (1e-12 if precision == FP64 else 1e-5)
+
+
+# Column transforms of one pass (up to 1024 rows in FP64, 2048 in FP32) and the
+# first of two passes above: fewer strips than a round over the XCDs, and paired
+# strips.
+@pytest.mark.parametrize("nx,ny", [(16, 1024), (64, 2048), (512, 1024), (512, 2048), (256, 512)])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_long_columns_match_numpy(nx, ny, precision):
+    print(f"case columns {nx}x{ny} precision={precision}", flush=True)
+    plan = Plan(nx, ny, 3, precision=precision)
+    rng = np.random.default_rng(nx + ny)
+    src = torch.from_numpy(rng.normal(size=6 * ny * nx)).to("cuda", plan.grid_dtype)
+    want = np.fft.ifft2(cube(plan, src), axes=(1, 2))
+    out = plan.fft(src, torch.empty_like(src))
+    assert rel_l2(cube(plan, out), want) <= (1e-14 if precision == FP64 else 2e-6)
+    plan.fft(src)
+    assert rel_l2(cube(plan, src), want) <= (1e-14 if precision == FP64 else 2e-6)
