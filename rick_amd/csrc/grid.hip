@@ -610,6 +610,67 @@ __device__ __forceinline__ void wave_row_sums(uint32_t r0, uint32_t n, uint32_t 
     }
 }
 
+// Sums of the 64 rows of one wave when a row holds F*P = 4 n4 floats, any n4
+// above 2: four lanes share a row, lane q taking its 16-byte pieces q, q + 4, ...
+// (64 bytes of a row per load instruction), and add up their parts at the end.
+// One lane per row made every load instruction touch 64 lines, whose other
+// parts were evicted before their turn: 2.9 M rows of 64 values took 1.88 ms
+// where this takes 0.47 (1.6 GB, 3.4 TB/s), 1.2 M rows of 12 values 134 and 112
+// us.  The sums come before the coordinate loads, whose registers they use.  Lane l returns the sums of row r0 + l.
+__device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, uint32_t n, uint32_t n4,
+                                                      uint32_t P, const float *__restrict__ vr,
+                                                      const float *__restrict__ vi,
+                                                      const float *__restrict__ wt,
+                                                      double &out_re, double &out_im)
+{
+    const uint32_t lane = threadIdx.x & 63u, q = lane & 3u;
+    const float4 *r4 = reinterpret_cast<const float4 *>(vr);
+    const float4 *i4 = reinterpret_cast<const float4 *>(vi);
+    const bool fixed_w = P == 1u || P == 2u || P == 4u;   // element c always weighs w[c % P]
+    out_re = out_im = 0.0;
+#pragma unroll 1
+    for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t row = r0 + j * 16u + lane / 4u;
+        double a_re = 0.0, a_im = 0.0;
+        if (row < n) {
+            const float *wrow = wt + (size_t)row * P;
+            const size_t e0 = (size_t)row * n4;
+            float w[4];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) w[c] = wrow[fixed_w ? c & (P - 1u) : (4u * q + c) % P];
+#pragma unroll 2
+            for (uint32_t i = q; i < n4; i += 4u) {
+                const float4 ra = load_stream4(&r4[e0 + i]), ia = load_stream4(&i4[e0 + i]);
+                const float rr[4] = {ra.x, ra.y, ra.z, ra.w}, ii[4] = {ia.x, ia.y, ia.z, ia.w};
+                if (!fixed_w && i != q) {
+#pragma unroll
+                    for (uint32_t c = 0; c < 4; ++c) w[c] = wrow[(4u * i + c) % P];
+                }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (!isnan(rr[c])) {
+                        const float wr = w[c] * rr[c];
+                        const float wi = w[c] * ii[c];
+                        a_re += (double)wr;
+                        a_im += (double)wi;
+                    }
+                }
+            }
+        }
+        a_re += __shfl_xor(a_re, 1);
+        a_im += __shfl_xor(a_im, 1);
+        a_re += __shfl_xor(a_re, 2);
+        a_im += __shfl_xor(a_im, 2);
+        // Row j*16 + m is in lanes 4m .. 4m+3.
+        const int src = (int)(lane & 15u) * 4;
+        const double t_re = __shfl(a_re, src), t_im = __shfl(a_im, src);
+        if (lane / 16u == j) {
+            out_re = t_re;
+            out_im = t_im;
+        }
+    }
+}
+
 // Clears the tiles of buckets that several tasks accumulate into atomically:
 // the split buckets first, first + stride, ... (one workgroup each).
 template <typename T2>
@@ -635,9 +696,10 @@ __device__ __forceinline__ void zero_split_tiles(const GridGeom &g, uint32_t fir
     }
 }
 
-// VMODE: 0 = per-row scalar reads, 1 = per-row 16-byte reads (F*P a multiple
-// of 4), 2 or 4 = wave-cooperative reads with VMODE lanes per row (F*P = 8 or
-// 16); 16-byte modes need 16-byte aligned visibility arrays.
+// VMODE: 0 = per-row scalar reads, 1 = one 16-byte read per row (F*P = 4),
+// 2 or 4 = wave-cooperative reads with VMODE lanes per row (F*P = 8 or 16),
+// 3 = wave-cooperative reads of any larger multiple of 4; the 16-byte modes need
+// 16-byte aligned visibility arrays.
 template <int PREC, int VMODE, bool BATCH>
 __global__ void __launch_bounds__(kScatterThreads, 8)
 k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__restrict__ uu_all,
@@ -671,6 +733,14 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
     // The read path is chosen on the host, so each instantiation carries one.
     constexpr bool vec4 = VMODE == 1;
     const uint32_t FP = F * P;
+    double w_re[kRowsPerThread] = {}, w_im[kRowsPerThread] = {};
+    if constexpr (VMODE == 3) {
+        // Before the coordinates are loaded: the sums take their registers.
+#pragma unroll
+        for (int k = 0; k < kRowsPerThread; ++k)
+            wave_row_sums_strided(base + k * kScatterThreads + threadIdx.x - (threadIdx.x & 63u),
+                                  n, FP / 4u, P, vr, vi, wt, w_re[k], w_im[k]);
+    }
     // Every coordinate of the thread's rows (and, with one value per row,
     // its visibility and weight) is requested before any is used, so the
     // loads of both rows overlap instead of each waiting on the arithmetic
@@ -693,13 +763,11 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
             }
         }
     }
-    double w_re[kRowsPerThread], w_im[kRowsPerThread];
     uint32_t widx[4] = {0u, 0u, 0u, 0u};
-    if constexpr (VMODE >= 2) row_weight_index<VMODE>(P, widx);
+    if constexpr (VMODE == 2 || VMODE == 4) row_weight_index<VMODE>(P, widx);
 #pragma unroll
     for (int k = 0; k < kRowsPerThread; ++k) {
-        w_re[k] = w_im[k] = 0.0;
-        if constexpr (VMODE >= 2)  // whole wave, before any lane leaves
+        if constexpr (VMODE == 2 || VMODE == 4)  // whole wave, before any lane leaves
             wave_row_sums<VMODE>(base + k * kScatterThreads + threadIdx.x - (threadIdx.x & 63u),
                                  n, P, widx, vr, vi, wt, w_re[k], w_im[k]);
     }
@@ -732,21 +800,18 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
             a_re = w_re[k];
             a_im = w_im[k];
         } else if (vec4) {
-            // Same sum in the same element order, read 16 bytes at a time.
-            const float4 *r4 = reinterpret_cast<const float4 *>(vr + vb);
-            const float4 *i4 = reinterpret_cast<const float4 *>(vi + vb);
-            for (uint32_t e4 = 0; e4 < FP / 4; ++e4) {
-                const float4 ra = load_stream4(&r4[e4]), ia = load_stream4(&i4[e4]);
-                const float rr[4] = {ra.x, ra.y, ra.z, ra.w}, ii[4] = {ia.x, ia.y, ia.z, ia.w};
+            // The row's four values in one 16-byte read per array.
+            const float4 ra = load_stream4(reinterpret_cast<const float4 *>(vr + vb));
+            const float4 ia = load_stream4(reinterpret_cast<const float4 *>(vi + vb));
+            const float rr[4] = {ra.x, ra.y, ra.z, ra.w}, ii[4] = {ia.x, ia.y, ia.z, ia.w};
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    if (!isnan(rr[c])) {
-                        const float wv = wrow[P == 1 ? 0u : (4 * e4 + c) % P];
-                        const float wr = wv * rr[c];
-                        const float wi = wv * ii[c];
-                        a_re += (double)wr;
-                        a_im += (double)wi;
-                    }
+            for (int c = 0; c < 4; ++c) {
+                if (!isnan(rr[c])) {
+                    const float wv = wrow[P == 1u ? 0u : (uint32_t)c % P];
+                    const float wr = wv * rr[c];
+                    const float wi = wv * ii[c];
+                    a_re += (double)wr;
+                    a_im += (double)wi;
                 }
             }
         } else if (FP == 1u) {
@@ -1469,7 +1534,7 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
         const bool vec4 = (FP % 4u) == 0u &&
                           ((reinterpret_cast<uintptr_t>(vr) | reinterpret_cast<uintptr_t>(vi)) &
                            15u) == 0u;   // batch: vr = vi = null, the caller checked the jobs
-        const int mode = !vec4 ? 0 : FP == 8u ? 2 : FP == 16u ? 4 : 1;
+        const int mode = !vec4 ? 0 : FP == 4u ? 1 : FP == 8u ? 2 : FP == 16u ? 4 : 3;
         // Overwritten grids: the split buckets' tiles start at zero (FP32: for
         // the non-finite fallback; its finite sums go through integer tiles).
         const uint32_t zblk = accumulate ? 0u : std::min(w.split_cap, kZeroBlocks);
@@ -1486,6 +1551,7 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
 #define RICK_SCATTER_MODES(PR)                                                                \
     switch (mode) {                                                                           \
     case 4: RICK_SCATTER(PR, 4); break;                                                       \
+    case 3: RICK_SCATTER(PR, 3); break;                                                       \
     case 2: RICK_SCATTER(PR, 2); break;                                                       \
     case 1: RICK_SCATTER(PR, 1); break;                                                       \
     default: RICK_SCATTER(PR, 0); break;                                                      \

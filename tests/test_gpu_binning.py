@@ -44,3 +44,30 @@ def test_binning_launch_edges_match_oracle(n, planes, rows_per_task):
         got = out.cpu().numpy()
         assert np.isfinite(got).all()
         assert rel_l2(got, ref) <= 1e-12
+
+
+# Rows of more than 16 values, or of 12, in 16-byte pieces shared by four lanes:
+# the last piece missing on some lanes, weights that do and do not repeat with
+# the piece, rows that end inside a wave, a misaligned array (scalar reads).
+@pytest.mark.parametrize("F,P", [(3, 4), (5, 4), (8, 3), (12, 3), (64, 1), (17, 4), (10, 2)])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n", [1, 4133])
+def test_wide_rows_match_oracle(F, P, shift, n):
+    nx, planes = 256, 4
+    print(f"case wide rows F={F} P={P} shift={shift} n={n}", flush=True)
+    rng = np.random.default_rng(F * 100 + P)
+    uu, vv, ww = (rng.uniform(0.0, 1.0, n) for _ in range(3))
+    vr, vi = (rng.normal(size=n * F * P).astype(np.float32) for _ in range(2))
+    vr[1::29] = np.nan
+    wt = rng.uniform(0.5, 1.5, n * P).astype(np.float32)
+    ref = O.wstack(O.KAISERBESSEL, planes, uu, vv, ww, vr, vi, wt, F, P, 1.0 / nx, 1.0 / planes,
+                   7, nx, nx, threads=8)
+    plan = Plan(nx, nx, planes, kernel=rick_amd.KAISERBESSEL, support=7, max_points=n)
+
+    def on_gpu(a):
+        t = torch.zeros(a.size + shift, dtype=torch.float32, device="cuda")[shift:]
+        return t.copy_(torch.from_numpy(a))
+    got = plan.grid(*[torch.from_numpy(a).to("cuda") for a in (uu, vv, ww)], on_gpu(vr),
+                    on_gpu(vi), torch.from_numpy(wt).to("cuda"), F, P).cpu().numpy()
+    assert np.isfinite(got).all()
+    assert rel_l2(got, ref) <= 1e-12
