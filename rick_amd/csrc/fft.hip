@@ -35,6 +35,7 @@ namespace {
 using namespace fftk;
 
 constexpr int kE = 16;  // complex values per thread
+constexpr int kFusedStrips = 256;   // column strips from which the fused phase pass fills the chip
 
 // The fused column/phase pass: complex values per thread for FP64 and FP32
 // plane data, and whether FP64 prefetches the next plane into registers.
@@ -882,6 +883,20 @@ hipError_t image_chain_impl(const FftPlan &p, void *grid_v, double scale_d, hipS
     // (512-point lines keep >= 8 columns, >= 64 B, per row access.)
     if (ny <= 512) {
         const ColArgs a{nx, ny, 0, 1, 0, 1, 0, 1};
+        // The fused pass walks the planes one after another with one workgroup
+        // per strip, so an image of fewer strips than CUs leaves most of the
+        // chip waiting: its columns are transformed in place, all planes at
+        // once, and the phase kernel sums them from the last-level cache.
+        // Columns and phase, fused against apart: 256^2 x 4 FP32 (16 strips) 23
+        // -> 15 us, 512^2 x 8 FP64 (64) 45 -> 28 us, 512^2 x 40 FP64 174 -> 94
+        // us, 1024 x 512 x 16 FP64 (128) 79 -> 80 us.
+        if (pj == nullptr && nx / lines_per_wg(ny) < kFusedStrips) {
+            tm->begin(RICK_STAGE_FFT_COLS, s);
+            e = launch_cols<T>(ny, a, 1, planes, twy, grid, grid, s, co);
+            tm->end(RICK_STAGE_FFT_COLS, s);
+            if (e != hipSuccess) return e;
+            return launch_phase(pg, sizeof(T) == 8 ? RICK_FP64 : RICK_FP32, grid, re, im, 0, s, tm);
+        }
         tm->begin(RICK_STAGE_PHASE, s);
         e = launch_cols_phase<T>(ny, a, 1, planes, twy, grid, pg, 0, 1, re, im, s, co, pj,
                                  njobs);

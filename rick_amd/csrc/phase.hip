@@ -40,6 +40,7 @@ k_phase(PhaseGeom g, const void *__restrict__ gridss_v, double *__restrict__ ore
     double acc_re = 0.0, acc_im = 0.0;
     const bool phase = g.phase_on && g.planes > 1;
     const double n = phase ? pixel_n(g.ltab[iu], g.mtab[iv]) : 1.0;
+#pragma unroll 4
     for (int iw = 0; iw < g.planes; ++iw) {
         const size_t idx = cell + (size_t)iw * plane;
         if constexpr (PREC == RICK_FP64) {

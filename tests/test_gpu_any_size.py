@@ -42,7 +42,9 @@ def test_lengths_of_every_radix_match_numpy(nx, ny, planes, precision):
 @pytest.mark.parametrize("nx,ny,planes,tile", [
     (18, 300, 3, (32, 32)), (300, 200, 4, (64, 32)), (130, 600, 3, (64, 64)),
     (143, 169, 2, (0, 0)), (1000, 1500, 2, (128, 32)), (4095, 66, 2, (32, 64)),
-    (12, 14, 1, (0, 0)), (100, 512, 2, (64, 64))])
+    (12, 14, 1, (0, 0)), (100, 512, 2, (64, 64)),
+    # power-of-two axes on both sides of the fused phase pass
+    (1024, 512, 3, (64, 32)), (2048, 512, 3, (0, 0)), (32, 16, 5, (32, 32))])
 @pytest.mark.parametrize("precision", [FP64, FP32])
 def test_sparse_chain_matches_separate_stages(nx, ny, planes, tile, precision):
     print(f"case chain {nx}x{ny}x{planes} tile={tile} precision={precision}", flush=True)
