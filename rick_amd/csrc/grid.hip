@@ -616,9 +616,11 @@ __device__ __forceinline__ void wave_row_sums(uint32_t r0, uint32_t n, uint32_t 
 // One lane per row made every load instruction touch 64 lines, whose other
 // parts were evicted before their turn: 2.9 M rows of 64 values took 1.88 ms
 // where this takes 0.47 (1.6 GB, 3.4 TB/s), 1.2 M rows of 12 values 134 and 112
-// us.  The sums come before the coordinate loads, whose registers they use.  Lane l returns the sums of row r0 + l.
-__device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, uint32_t n, uint32_t n4,
-                                                      uint32_t P, const float *__restrict__ vr,
+// us.  `in` has a bit for each row that is to be read; lane l returns the sums of
+// row r0 + l (zero without its bit).
+__device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, unsigned long long in,
+                                                      uint32_t n4, uint32_t P,
+                                                      const float *__restrict__ vr,
                                                       const float *__restrict__ vi,
                                                       const float *__restrict__ wt,
                                                       double &out_re, double &out_im)
@@ -630,9 +632,10 @@ __device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, uint32_t n, u
     out_re = out_im = 0.0;
 #pragma unroll 1
     for (uint32_t j = 0; j < 4; ++j) {
+        if (((in >> (j * 16u)) & 0xffffull) == 0ull) continue;   // uniform
         const uint32_t row = r0 + j * 16u + lane / 4u;
         double a_re = 0.0, a_im = 0.0;
-        if (row < n) {
+        if ((in >> (j * 16u + lane / 4u)) & 1ull) {
             const float *wrow = wt + (size_t)row * P;
             const size_t e0 = (size_t)row * n4;
             float w[4];
@@ -735,11 +738,24 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
     const uint32_t FP = F * P;
     double w_re[kRowsPerThread] = {}, w_im[kRowsPerThread] = {};
     if constexpr (VMODE == 3) {
-        // Before the coordinates are loaded: the sums take their registers.
+        // The sums first, over the rows that fall into the grid; coordinates are
+        // loaded once more below, from the cache: held over the sums they cost
+        // more in spilled registers (112 -> 140 us on 1.2 M rows of 12 values).
+        unsigned long long in[kRowsPerThread];
+#pragma unroll
+        for (int k = 0; k < kRowsPerThread; ++k) {
+            const uint32_t i = base + k * kScatterThreads + threadIdx.x;
+            Foot f;
+            in[k] = __ballot(i < n &&
+                             footprint(g, div_by(as_global(uu)[i < n ? i : 0], g.dx, g.inv_dx),
+                                       div_by(as_global(vv)[i < n ? i : 0], g.dx, g.inv_dx),
+                                       div_by(as_global(ww)[i < n ? i : 0], br.dw, br.inv_dw), f,
+                                       br.planes, br.plane0));
+        }
 #pragma unroll
         for (int k = 0; k < kRowsPerThread; ++k)
             wave_row_sums_strided(base + k * kScatterThreads + threadIdx.x - (threadIdx.x & 63u),
-                                  n, FP / 4u, P, vr, vi, wt, w_re[k], w_im[k]);
+                                  in[k], FP / 4u, P, vr, vi, wt, w_re[k], w_im[k]);
     }
     // Every coordinate of the thread's rows (and, with one value per row,
     // its visibility and weight) is requested before any is used, so the
