@@ -316,6 +316,7 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
 // g.rmax / 8), then the short ones, so that no long task starts when the others
 // are done, and the zero tasks last; the tile kernel interleaves accumulation
 // and zero tasks evenly over its workgroups.
+constexpr uint32_t kOwnTasks = 8;   // parts of a split bucket that one scan thread writes
 constexpr int kLengths = 3;
 enum { kQRecords, kQSplit, kQNonEmpty, kQZero, kQTasks, kScanQ = kQTasks + kLengths };
 
@@ -388,6 +389,20 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
     }
 }
 
+// Tasks first, first + stride, ... of the nt equal parts of split bucket b with
+// c records from ro; they start at slot t.
+__device__ __forceinline__ void split_tasks(uint4 *__restrict__ tasks, uint32_t task_cap,
+                                            uint32_t b, uint32_t ro, uint32_t c, uint32_t t,
+                                            uint32_t nt, uint32_t tag, uint32_t first,
+                                            uint32_t stride)
+{
+    const uint32_t part = (c + nt - 1) / nt;
+    for (uint32_t q = first; q < nt; q += stride) {
+        const uint32_t r0 = ro + q * part, r1 = min(r0 + part, ro + c);
+        if (t + q < task_cap) tasks[t + q] = make_uint4(b, r0, r1, tag);
+    }
+}
+
 // Offsets, cursors, tasks and split list of 1024 buckets per workgroup.  The
 // counters it has read and the row flags are cleared on the way: the counters
 // for the next call's count, the flags for this call's tile kernel.  With nscan == 1
@@ -404,7 +419,7 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
     constexpr int NT = kThreads, NW = NT / 64;
     __shared__ uint32_t wtot[kScanQ][NW];       // wave totals
     __shared__ uint32_t before[kScanQ], total[kScanQ];
-    // Split buckets of this block, whose tasks the whole workgroup writes.
+    // Buckets of more than kOwnTasks parts, whose tasks a wave writes.
     __shared__ uint4 big[4 * NT];               // bucket, first record, records, first task
     __shared__ uint32_t bigtag[4 * NT], nbig;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -504,23 +519,25 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
             } else {
                 // Tasks of a split bucket carry its slot in split_list (always
                 // below split_cap: a split bucket holds more than rmax records).
-                const uint32_t i = atomicAdd(&nbig, 1u);
-                big[i] = make_uint4(b, ro, c[k], t);
-                bigtag[i] = so < split_cap ? kSplitTask + so : 1u;
+                const uint32_t tag = so < split_cap ? kSplitTask + so : 1u;
                 if (so < split_cap) split_list[so++] = b;
+                if (nt <= kOwnTasks) {
+                    split_tasks(tasks, task_cap, b, ro, c[k], t, nt, tag, 0u, 1u);
+                } else {
+                    const uint32_t i = atomicAdd(&nbig, 1u);
+                    big[i] = make_uint4(b, ro, c[k], t);
+                    bigtag[i] = tag;
+                }
             }
         }
         ro += c[k];
     }
     __syncthreads();
-    // One wave per split bucket.
+    // One wave per bucket of many parts.
     for (uint32_t i = wave; i < nbig; i += NW) {
         const uint4 e = big[i];
-        const uint32_t nt = ntasks_of(e.z, g.rmax), part = (e.z + nt - 1) / nt;
-        for (uint32_t q = lane; q < nt; q += 64) {
-            const uint32_t r0 = e.y + q * part, r1 = min(r0 + part, e.y + e.z);
-            if (e.w + q < task_cap) tasks[e.w + q] = make_uint4(e.x, r0, r1, bigtag[i]);
-        }
+        split_tasks(tasks, task_cap, e.x, e.y, e.z, e.w, ntasks_of(e.z, g.rmax), bigtag[i], lane,
+                    64u);
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         offsets[g.nb] = total[kQRecords];
