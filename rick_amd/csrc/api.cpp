@@ -89,16 +89,21 @@ TileShape default_tile(const rick_plan_desc &d)
     return nb <= 1024 ? TileShape{64, 32} : TileShape{64, 64};
 }
 
-// Built-in records per task: the power of two that makes a full task the share
-// of one of 512 resident workgroups (two per CU).  Shorter tasks split more
-// buckets, whose parts meet in atomics; longer ones leave the last workgroups
-// running alone (image, best against 4096: 50 k rows 512 records 75 / 98 us,
-// 1 M rows 2048 records 670 / 691 us, 3 M 4096, 7.7 M rows 8192-16384 records,
-// dense FP32 gridding 1.30 / 1.33 ms).
-uint32_t default_rows_per_task(uint32_t max_points)
+// Built-in records per task: the power of two from the share of one of 192
+// workgroups up where the tile kernel takes full tasks by footprint class, whose
+// fixed cost wants long tasks, and of 512 (two per CU) where it does not.
+// Shorter tasks split more buckets, whose parts meet in atomics; longer ones
+// leave the last workgroups running alone.  Image by records per task: 516 k rows
+// on 512^2 x 8 FP64 137 us at 1024, 119 at 4096, 143 at 8192; 1 M rows on 1024^2
+// x 16 464 us at 2048, 444 at 8192, 482 at 16384; 3 M rows on 2048^2 x 12 FP32 861
+// us at 2048, 802 at 8192; dense FP32 gridding of 7.7 M rows 1.36 ms at 4096, 1.27
+// at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us at 512,
+// 98 at 4096.
+uint32_t default_rows_per_task(const rick_plan_desc &d, int tu, int tv, int smax)
 {
+    const uint32_t share = d.max_points / (tile_by_class(d, tu, tv, smax) ? 192u : 512u);
     uint32_t r = 512;
-    while (r < 16384 && r < max_points / 512) r *= 2;
+    while (r < 16384 && r < share) r *= 2;
     return r;
 }
 
@@ -225,8 +230,6 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
     if (nb >= (1ull << 31)) return set_error(RICK_ERR_INVALID, "too many grid tiles");
     g.nb = (uint32_t)nb;
     g.cshift = counter_shift(g.nb);
-    g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
-                                 : default_rows_per_task(d.max_points);
     g.ntable = kTableOversample * d.w_support;
     // ~64-128 KB of grid per zero task measured best (LOFAR-like grid).
     g.zrun = d.precision == RICK_FP64 ? 2 : 4;
@@ -242,6 +245,8 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
                              "footprint_unroll %d: must be 0 or one of 7, 9, 11, 15 and >= "
                              "w_support %d", d.footprint_unroll, d.w_support);
     }
+    g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
+                                 : default_rows_per_task(d, tu, tv, g.smax);
     if ((uint64_t)d.max_points * 4ull >= (1ull << 32))
         return set_error(RICK_ERR_INVALID, "max_points %u too large (limit 2^30)", d.max_points);
 
@@ -304,6 +309,9 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
     double kmax = 0.0;
     for (int i = 0; i < g.ntable; ++i) kmax = std::max(kmax, std::fabs(h[i]));
     g.cmax = d.kernel == RICK_GAUSS_HI_PRECISION ? (1.0 / (2.0 * 1.0 * 1.0)) / kRefPi : kmax * kmax;
+    g.fscale = 1.0;
+    if (d.kernel != RICK_GAUSS_HI_PRECISION && kmax > 0.0)
+        while (g.fscale > kmax) g.fscale *= 0.5;   // cmax / kmax = kmax
     e = hipMemcpy(p->table_d, h.data(), sizeof(double) * kMaxTable, hipMemcpyHostToDevice);
     std::vector<double> tw;
     auto put_tw = [&](int n, size_t o) {

@@ -1000,8 +1000,88 @@ __host__ __device__ constexpr bool tile_persistent(int tu, int tv)
     return 3 * (2 * tv * (tu + kPadU) * (int)sizeof(double)) > kLdsBytes;
 }
 
+// Accumulation by footprint class.  A row's v-weights K[kKer(k)] depend only on
+// its cell gv and on which fifth of a cell it lies in: v_dist + KL grows by one
+// from footprint row to footprint row, so kKer = i1 + 5 (dk - 1) for dk >= 1, with
+// i1 = 2 .. 7 (the half-cell offset makes six classes), and fabs mirrors the first
+// row, kKer = |i1 - 5| folded to 2, 1, 0, 0, 1, 2.  So the task takes one class at
+// a time: each record adds S * K[jKer] to the S cells of row gv of an array F (2S
+// LDS atomics instead of 2S^2), and then every thread adds, for its column of the
+// tile, sum over dk of K[kKer(dk)] * F[k + KL - dk] to the rows it keeps in
+// registers.  The weights, and which cells a record reaches, are those of the
+// per-record accumulation; the sums only associate differently.  Records whose
+// kKer do not follow the pattern (positions within rounding of a class border,
+// rows at negative positions) are added to the finished tile one by one.
+// Bound before by the LDS atomics (54 % of their conflict-free rate with random
+// cells), now by the rounds' barriers and LDS reads in short tasks.  Tile kernel
+// with and without: 7.7 M rows on 4096^2 x 32 FP64 706 -> 491 us, 3 M rows of
+// support 9 on 2048^2 x 12 FP32 339 -> 281 us, 1 M rows on 1024^2 x 16 FP64 181 ->
+// 130 us, 516 k rows on 512^2 x 8 FP64 64 -> 47 us.
+constexpr int kClasses = 6;
+constexpr uint32_t kClassParts = 12; // most parts of an FP32 split bucket taken by classes: every
+                                     // part walks the whole bucket's positions
+constexpr int kQueue = 128;          // record indices a wave gathers for one class
+__host__ __device__ constexpr bool class_tile(int tu, int tv, int smax)
+{
+    return smax <= 11 && 2 * (tv + smax - 1) * tu * (int)sizeof(double) <= 76000;
+}
+// Records from which a task is taken by classes: six rounds of clearing F and of
+// the sums over dk cost a 64 x 64 tile about as much as adding 700 records cell by
+// cell.  Flat around the best (FP32 3 M rows, KB 9: 293 / 288 / 281 / 286 us at
+// 512 / 768 / 1024 / 1536; FP64 1 M rows: 129 / 131 / 132 / 139 us).
+__host__ __device__ constexpr uint32_t class_min(int prec) { return prec == RICK_FP64 ? 768u : 1024u; }
+
+// kKer of footprint row k (w-stacking.cu:484, 493).
+__device__ __forceinline__ int table_index(int k, double pos, int kl)
+{
+    const double dist = (double)k + 0.5 - pos;
+    return (int)(kOversample * (fabs(dist + (double)kl)));
+}
+// Class of a position from its second footprint row; outside 0 .. 5: none.
+__device__ __forceinline__ int foot_class(double pos, int cell, int kl)
+{
+    return cell < 0 ? -1 : table_index(cell - kl + 1, pos, kl) - 2;
+}
+__device__ __forceinline__ int class_first(int c) { return c < 2 ? 2 - c : c < 4 ? 0 : c - 3; }
+// Whether every footprint row of the position has the index its class gives it.
+template <int S>
+__device__ __forceinline__ bool class_regular(double pos, int cell, int c)
+{
+    constexpr int KL = (S - 1) / 2;
+    bool ok = (unsigned)c < (unsigned)kClasses &&
+              table_index(cell - KL, pos, KL) == class_first(c);
+#pragma unroll
+    for (int d = 2; d < S; ++d) ok = ok && table_index(cell - KL + d, pos, KL) == c + 2 + 5 * (d - 1);
+    return ok;
+}
+// One of `parts` sets, chosen by a record's position alone.
+__device__ __forceinline__ uint32_t hash_part(double pu, double pv, uint32_t parts)
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(pu),
+                             b = (unsigned long long)__double_as_longlong(pv);
+    const unsigned long long h = (a ^ (b << 21 | b >> 43)) * 0x9E3779B97F4A7C15ull;
+    return (uint32_t)(((h >> 32) * parts) >> 32);
+}
+// FP32 sums of a split bucket must not depend on which records meet in a task
+// (the scatter's order varies), so its tasks take their records from the whole
+// bucket: the bucket has kClasses * `sets` portions, portion x holding the
+// records of class x % kClasses in hash set x / kClasses, and task t of nt takes
+// portions t, t + nt, ...
+__device__ __forceinline__ uint32_t portion_sets(uint32_t nt)
+{
+    return (nt + kClasses - 1) / kClasses;
+}
+// Task that adds a record which no class has.
+__device__ __forceinline__ uint32_t odd_owner(double pu, double pv, int c, uint32_t nt)
+{
+    if ((unsigned)c >= (unsigned)kClasses) return hash_part(pu, pv, nt);
+    return (hash_part(pu, pv, portion_sets(nt)) * kClasses + (uint32_t)c) % nt;
+}
+
+// Tiles that LDS holds to two workgroups per CU keep within the registers of
+// four waves per SIMD.
 template <int PREC, int TU, int TV, int SMAX, bool HIPREC>
-__global__ void __launch_bounds__(kTileThreads)
+__global__ void __launch_bounds__(kTileThreads, tile_persistent(TU, TV) ? 4 : 1)
 k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
        const typename RecOf<PREC>::type *__restrict__ rec, const double *__restrict__ table,
        void *grid_v, int accumulate, const uint32_t *__restrict__ offsets,
@@ -1011,8 +1091,11 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
     using T = typename std::conditional<PREC == RICK_FP64, double, float>::type;
     using T2 = typename std::conditional<PREC == RICK_FP64, double2, float2>::type;
     constexpr int LDU = TU + kPadU;
-    __shared__ double lds[2 * TV * LDU];
-    __shared__ T stab[kMaxTable];
+    constexpr bool CLS = !HIPREC && class_tile(TU, TV, SMAX);
+    constexpr int RF = TV + SMAX - 1;   // rows of F
+    __shared__ double lds[CLS && RF * TU > TV * LDU ? 2 * RF * TU : 2 * TV * LDU];
+    __shared__ double stab[kMaxTable];
+    __shared__ uint32_t queue[CLS ? kTileThreads / 64 : 1][CLS ? kQueue : 1];
     double *sre = lds, *sim = lds + TV * LDU;
 
     // Workgroup k runs slot k; persistent workgroups (tile_persistent) then
@@ -1093,14 +1176,16 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
             continue;
         }
 
-        for (int idx = threadIdx.x; idx < 2 * TV * LDU; idx += kTileThreads) lds[idx] = 0.0;
-        for (int idx = threadIdx.x; idx < g.ntable; idx += kTileThreads) stab[idx] = (T)table[idx];
+        for (int idx = threadIdx.x; idx < g.ntable; idx += kTileThreads) stab[idx] = table[idx];
         // FP32: fixed-point scale from the bound of the task's cell sums.
         bool fixed = false;
-        double scale = 1.0;
+        double scale = 1.0, fscale = 1.0;   // of tile cells, of F
         if (PREC == RICK_FP32 && det) {
             fixed = true;
             scale = bucket_scale;
+            // F holds sums of S * K[jKer], the tile sums of S * K[jKer] * K[kKer]:
+            // their bounds differ by one factor of the largest table entry.
+            fscale = scale * g.fscale;
         } else if constexpr (PREC == RICK_FP32) {
             __shared__ double red[2][kTileThreads / 64];
             double ar = 0.0, ai = 0.0;
@@ -1129,8 +1214,27 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
                 int e;
                 frexp(bound, &e);                    // bound < 2^e
                 scale = ldexp(1.0, 50 - e);          // bound * scale < 2^50
+                fscale = scale * g.fscale;
             }
         }
+        // The records of the task, or (FP32 split bucket by classes) of its bucket,
+        // of which it takes its portions.
+        uint32_t nt = 1, my = 0, q0 = r0, q1 = r1, len = r1 - r0;
+        if (PREC == RICK_FP32 && det) {
+            q0 = offsets[b];
+            q1 = offsets[b + 1];
+            nt = ntasks_of(q1 - q0, g.rmax);
+            len = (q1 - q0 + nt - 1) / nt;   // the same for all tasks of the bucket
+            my = (r0 - q0) / len;
+        }
+        const bool by_class = CLS && g.support == SMAX && len >= class_min(PREC) &&
+                              (PREC == RICK_FP64 || fixed) && nt <= kClassParts;
+        if (!by_class) {
+            q0 = r0;
+            q1 = r1;
+        }
+        if (!by_class)
+            for (int idx = threadIdx.x; idx < 2 * TV * LDU; idx += kTileThreads) lds[idx] = 0.0;
         __syncthreads();
 
         const int S = g.support, KL = g.kl;
@@ -1149,13 +1253,21 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
         const uint32_t roff = (threadIdx.x & 63u) * (kTileThreads / 64) + (threadIdx.x >> 6);
         // The FP32 fixed-point and the FP64-atomic accumulation are separate
         // loops, so the hot one carries no code of the other.
-        auto accumulate_all = [&](auto fixed_tag) {
+        // With odd_only it takes the records that no class has.
+        auto accumulate_all = [&](auto fixed_tag, bool odd_only) {
             constexpr bool FIXED = decltype(fixed_tag)::value;
-            for (uint32_t c0 = r0; c0 < r1; c0 += kTileThreads) {
+            const uint32_t a0 = odd_only ? q0 : r0, a1 = odd_only ? q1 : r1;
+            for (uint32_t c0 = a0; c0 < a1; c0 += kTileThreads) {
                 const uint32_t r = c0 + roff;
-                if (r >= r1) continue;
+                if (r >= a1) continue;
                 const auto rc = rec[r];
                 const double pu = rc.pu, pv = rc.pv;
+                if (odd_only) {
+                    const int cell = (int)pv, cls = foot_class(pv, cell, KL);
+                    if (class_regular<SMAX>(pv, cell, cls) ||
+                        (nt > 1 && odd_owner(pu, pv, cls, nt) != my))
+                        continue;
+                }
                 const T s_re = rc.sre, s_im = rc.sim;
                 Foot f;
                 uv_range(g, pu, pv, f);
@@ -1178,7 +1290,7 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
                         if (hiprec) {
                             umask |= 1u << dj;
                         } else if (jKer >= 0 && jKer < g.ntable) {
-                            wu[dj] = stab[jKer];
+                            wu[dj] = (T)stab[jKer];
                             umask |= 1u << dj;
                         }
                     }
@@ -1194,7 +1306,7 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
                     if (!hiprec) {
                         const int kKer = (int)(kOversample * (fabs(v_dist + (double)KL)));
                         if (kKer < 0 || kKer >= g.ntable) continue;
-                        wv = stab[kKer];
+                        wv = (T)stab[kKer];
                     }
                     // LDS index of footprint column 0 on this row; only columns with
                     // their umask bit set (inside the tile) are ever accessed.
@@ -1228,11 +1340,146 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
                 }
             }
         };
-        if constexpr (PREC == RICK_FP32) {
-            if (fixed) accumulate_all(std::true_type{});
-            else accumulate_all(std::false_type{});
-        } else {
-            accumulate_all(std::false_type{});
+        bool direct = !by_class;
+        if constexpr (CLS) {
+            if (by_class) {
+                constexpr int NG = kTileThreads / TU, RP = TV / NG;   // row groups, rows of a thread
+                constexpr double M = 6755399441055744.0;              // to_fixed()'s offset
+                double *fre = lds, *fim = lds + RF * TU;
+                const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                const int cu = threadIdx.x % TU, rg = threadIdx.x / TU;
+                volatile uint32_t *q = queue[wave];
+                int odd = 0;
+                double ar[RP], ai[RP];
+#pragma unroll
+                for (int o = 0; o < RP; ++o) ar[o] = ai[o] = 0.0;
+                // Adds record r to row gv of F.
+                auto add_row = [&](uint32_t r, int c) {
+                    const auto rc = rec[r];
+                    if (!class_regular<SMAX>(rc.pv, (int)rc.pv, c)) {
+                        odd = 1;
+                        return;
+                    }
+                    Foot f;
+                    uv_range(g, rc.pu, rc.pv, f);
+                    const int row = f.gv - k0 + KL;
+                    if ((unsigned)row >= (unsigned)RF) return;
+                    const int ja = max(f.jmin, jlo), jb = min(f.jmax, jhi), ju0 = f.gu - KL;
+                    const int at = row * TU + (ju0 - j0);
+#pragma unroll
+                    for (int dj = 0; dj < SMAX; ++dj) {
+                        const int j = ju0 + dj;
+                        const int jKer = table_index(j, rc.pu, KL);
+                        if (j < ja || j > jb || jKer >= g.ntable) continue;
+                        const double k = stab[jKer];
+                        if constexpr (PREC == RICK_FP32) {
+                            __hip_atomic_fetch_add(
+                                reinterpret_cast<unsigned long long *>(&fre[at + dj]),
+                                to_fixed((double)rc.sre * k, fscale), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WORKGROUP);
+                            __hip_atomic_fetch_add(
+                                reinterpret_cast<unsigned long long *>(&fim[at + dj]),
+                                to_fixed((double)rc.sim * k, fscale), __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_WORKGROUP);
+                        } else {
+                            __hip_atomic_fetch_add(&fre[at + dj], rc.sre * k, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                            __hip_atomic_fetch_add(&fim[at + dj], rc.sim * k, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                    }
+                };
+#pragma unroll 1
+                for (uint32_t x = my; x < kClasses * portion_sets(nt); x += nt) {
+                    const int c = (int)(x % kClasses);
+                    // FP32 cells start at the bits of M: the integer sums then read
+                    // as the doubles M + sum.
+                    for (int i = threadIdx.x; i < 2 * RF * TU; i += kTileThreads)
+                        lds[i] = PREC == RICK_FP32 ? M : 0.0;
+                    __syncthreads();
+                    // Each wave gathers the indices of this class's records until 64
+                    // lanes have one.
+                    int held = 0;
+                    constexpr int AHEAD = 4;   // batches whose positions are loaded together
+                    for (uint32_t base = q0 + wave * 64; base < q1; base += AHEAD * kTileThreads) {
+                        double pv[AHEAD], pu[AHEAD];
+#pragma unroll
+                        for (int j = 0; j < AHEAD; ++j) {
+                            const uint32_t r = base + j * kTileThreads + lane;
+                            pv[j] = pu[j] = 0.0;
+                            if (r < q1) {
+                                pv[j] = rec[r].pv;
+                                if (PREC == RICK_FP32 && nt > kClasses) pu[j] = rec[r].pu;
+                            }
+                        }
+#pragma unroll
+                        for (int j = 0; j < AHEAD; ++j) {
+                            const uint32_t r = base + j * kTileThreads + lane;
+                            const int cls = foot_class(pv[j], (int)pv[j], KL);
+                            bool mine = r < q1 && cls == c;
+                            if (r < q1) odd |= (unsigned)cls >= (unsigned)kClasses;
+                            if (PREC == RICK_FP32 && nt > kClasses)
+                                mine = mine && hash_part(pu[j], pv[j], portion_sets(nt)) ==
+                                                   x / kClasses;
+                            const unsigned long long m = __ballot(mine);
+                            if (mine) q[held + __popcll(m & ((1ull << lane) - 1ull))] = r;
+                            held += __popcll(m);
+                            if (held >= 64) {
+                                add_row(q[lane], c);
+                                held -= 64;
+                                if (lane < held) q[lane] = q[64 + lane];
+                            }
+                        }
+                    }
+                    if (lane < held) add_row(q[lane], c);
+                    __syncthreads();
+                    double kw[SMAX];
+                    kw[0] = stab[class_first(c)];
+#pragma unroll
+                    for (int d = 1; d < SMAX; ++d) kw[d] = stab[c + 2 + 5 * (d - 1)];
+                    const int f0 = rg * RP * TU + cu;
+#pragma unroll
+                    for (int r = 0; r < RP + SMAX - 1; ++r) {
+                        double xr = fre[f0 + r * TU], xi = fim[f0 + r * TU];
+                        if (PREC == RICK_FP32) {
+                            xr -= M;
+                            xi -= M;
+                        }
+#pragma unroll
+                        for (int o = 0; o < RP; ++o) {
+                            const int d = o + SMAX - 1 - r;   // row of F r: cell k + KL - d
+                            if (d >= 0 && d < SMAX) {
+                                ar[o] = __fma_rn(kw[d], xr, ar[o]);
+                                ai[o] = __fma_rn(kw[d], xi, ai[o]);
+                            }
+                        }
+                    }
+                    __syncthreads();
+                }
+                direct = __syncthreads_or(odd) != 0;
+                // The sums into the tile, in the form the direct accumulation leaves.
+#pragma unroll
+                for (int o = 0; o < RP; ++o) {
+                    const int li = (rg * RP + o) * LDU + cu;
+                    if constexpr (PREC == RICK_FP32) {
+                        const double back = scale / fscale;   // a power of two
+                        reinterpret_cast<unsigned long long *>(sre)[li] = to_fixed(ar[o], back);
+                        reinterpret_cast<unsigned long long *>(sim)[li] = to_fixed(ai[o], back);
+                    } else {
+                        sre[li] = ar[o];
+                        sim[li] = ai[o];
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        if (direct) {
+            if constexpr (PREC == RICK_FP32) {
+                if (fixed) accumulate_all(std::true_type{}, by_class);
+                else accumulate_all(std::false_type{}, by_class);
+            } else {
+                accumulate_all(std::false_type{}, by_class);
+            }
         }
         __syncthreads();
 
@@ -1428,6 +1675,11 @@ int count_rows_per_thread(uint32_t n)
 {
     if (n >= 160u * 16 * kBinThreads) return 16;
     return n >= 128u * 4 * kBinThreads ? 4 : 1;
+}
+
+bool tile_by_class(const rick_plan_desc &d, int tu, int tv, int smax)
+{
+    return d.kernel != RICK_GAUSS_HI_PRECISION && d.w_support == smax && class_tile(tu, tv, smax);
 }
 
 int counter_shift(uint32_t nb)

@@ -112,6 +112,9 @@ struct GridGeom {
     uint32_t rmax;          // rows per task
     int ntable;
     double cmax;            // largest per-cell convolution weight (a bound)
+    // Power of two <= cmax / (largest table entry): sums of S * K[jKer] scaled by
+    // it stay within the bound of sums of S * K[jKer] * K[kKer].
+    double fscale;
     int zrun;               // empty buckets cleared per zero task (1..4)
     int smax;               // unrolled footprint length of the tile kernel (>= support)
     // 1/dx and 1/dw when dx / dw are powers of two (then x * inv is exactly
@@ -166,6 +169,9 @@ struct BatchJob {
     int plane0, planes;     // the job's planes in the group's plane stack
     double dw, inv_dw;      // inv_dw: exact_inverse(dw)
 };
+// Whether the tile kernel of a plan with this tile and footprint unroll takes
+// long tasks by footprint class.
+bool tile_by_class(const rick_plan_desc &d, int tu, int tv, int smax);
 // log2 of the words between the counters of consecutive buckets.
 int counter_shift(uint32_t nb);
 // Rows per block of the count kernel: batch jobs start at multiples of it.
