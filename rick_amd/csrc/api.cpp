@@ -86,7 +86,11 @@ TileShape default_tile(const rick_plan_desc &d)
     if (d.grid_size_x > 4096) return {128, 32};
     const uint64_t nb = (uint64_t)d.num_w_planes * ((d.grid_size_x + 63) / 64) *
                         ((d.grid_size_y + 63) / 64);
-    return nb <= 1024 ? TileShape{64, 32} : TileShape{64, 64};
+    // 64 x 32 tiles take one workgroup per task, of which a launch holds fewer
+    // than 2^32 threads; the larger tiles' workgroups stay and take many.
+    const uint64_t rows = d.rows_per_task > 0 ? d.rows_per_task : 512;
+    const bool fits = (2 * nb + 4ull * d.max_points / rows + 1) * 512 < (1ull << 32);
+    return nb <= 1024 && fits ? TileShape{64, 32} : TileShape{64, 64};
 }
 
 // Built-in records per task: the power of two from the share of one of 192
