@@ -33,7 +33,7 @@ constexpr int kExtBlocks = 1024;        // blocks of the extrema pass (max)
 constexpr int kSecRows = 4096;          // rows per sector-binning block
 constexpr int kSecRowsPerWave = kSecRows / (kPrepThreads / 64);
 constexpr int kMaxSlots = 4096;         // nsectors + 1 <= kMaxSlots
-constexpr int kAggregateSectors = 4;    // up to this many: wave-aggregated counting
+constexpr int kFewSectors = 4;          // up to this many: one ballot per slot
 constexpr int kScanChunk = 4096;        // elements per scan block (16 per thread)
 constexpr int kScanTopThreads = 1024;
 constexpr int kMaxScanChunks = kScanTopThreads * 16;
@@ -241,38 +241,54 @@ __device__ inline void for_each_sector(const int s[3], Fn &&f)
     }
 }
 
-__global__ void __launch_bounds__(kPrepThreads)
-k_sector_count(SectorGeom g, const double *__restrict__ vv, uint32_t *__restrict__ counts,
-               uint32_t *__restrict__ bad_total)
+// Lanes of the wave with an entry for `slot`.
+__device__ __forceinline__ unsigned long long slot_lanes(const int s[3], int slot)
 {
-    __shared__ uint32_t hist[kMaxSlots];
-    __shared__ uint32_t bad_blk;
+    return __ballot(s[0] == slot || s[1] == slot || s[2] == slot);
+}
+
+// Histogram of one block's entries.  FEW (at most kFewSectors slabs): one ballot
+// per slot and round, the counts in scalar registers (3 M rows in 4 slabs 14.3 us;
+// walking the distinct sectors of a wave one by one 17.8 us).  With more slabs a
+// ballot per slot would cost more than the LDS atomics of the rows' own slots.
+template <bool FEW>
+__global__ void __launch_bounds__(kPrepThreads)
+k_sector_count(SectorGeom g, const double *__restrict__ vv, uint32_t *__restrict__ counts)
+{
+    __shared__ uint32_t hist[FEW ? kFewSectors + 1 : kMaxSlots];
     const int slots = g.nsectors + 1;
     for (int s = threadIdx.x; s < slots; s += kPrepThreads) hist[s] = 0;
-    if (threadIdx.x == 0) bad_blk = 0;
-    __syncthreads();
-    uint32_t bad = 0;
+    constexpr int kRounds = kSecRows / kPrepThreads;
     const int lane = threadIdx.x & 63;
-    const size_t r0 = (size_t)blockIdx.x * kSecRows;
-    for (int k = 0; k < kSecRows / kPrepThreads; ++k) {
-        const size_t r = r0 + (size_t)k * kPrepThreads + threadIdx.x;
+    const size_t r0 = (size_t)blockIdx.x * kSecRows + threadIdx.x;
+    double v[kRounds];   // all loads under way before the first is used
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k)
+        v[k] = r0 + k * kPrepThreads < g.n ? vv[r0 + k * kPrepThreads] : 0.0;
+    __syncthreads();
+    uint32_t bad = 0;    // counted by k_sector_fill
+    uint32_t cnt[kFewSectors + 1] = {};
+#pragma unroll
+    for (int k = 0; k < kRounds; ++k) {
         int s[3] = {-1, -1, -1};
-        if (r < g.n) row_sectors(g, vv[r], s, bad);
-        if (g.nsectors <= kAggregateSectors) {
-            // Few sectors: most lanes share one; one LDS atomic per sector.
-            for_each_sector(s, [&](int sec, unsigned long long m, bool) {
-                if (lane == 0) atomicAdd(&hist[sec], (uint32_t)__popcll(m));
-            });
+        if (r0 + k * kPrepThreads < g.n) row_sectors(g, v[k], s, bad);
+        if constexpr (FEW) {
+#pragma unroll
+            for (int q = 0; q <= kFewSectors; ++q) cnt[q] += (uint32_t)__popcll(slot_lanes(s, q));
         } else {
             for (int j = 0; j < 3; ++j)
                 if (s[j] >= 0) atomicAdd(&hist[s[j]], 1u);
         }
     }
-    if (bad) atomicAdd(&bad_blk, bad);
+    if constexpr (FEW) {
+        if (lane == 0)
+#pragma unroll
+            for (int q = 0; q <= kFewSectors; ++q)
+                if (q < slots && cnt[q]) atomicAdd(&hist[q], cnt[q]);
+    }
     __syncthreads();
     for (int s = threadIdx.x; s < slots; s += kPrepThreads)
         counts[(size_t)s * g.nb + blockIdx.x] = hist[s];
-    if (threadIdx.x == 0 && bad_blk) atomicAdd(bad_total, bad_blk);
 }
 
 // Exclusive scan of len u32 values: per-chunk sums, one-block scan of the
@@ -319,7 +335,8 @@ k_scan_sums(const uint32_t *__restrict__ in, size_t len, uint32_t *__restrict__ 
 }
 
 __global__ void __launch_bounds__(kScanTopThreads)
-k_scan_top(uint32_t *__restrict__ sums, int nchunks, uint32_t *__restrict__ out_total)
+k_scan_top(uint32_t *__restrict__ sums, int nchunks, uint32_t *__restrict__ out_total,
+           uint32_t *__restrict__ totals)
 {
     uint32_t v[16], s = 0;
     for (int k = 0; k < 16; ++k) {
@@ -334,7 +351,46 @@ k_scan_top(uint32_t *__restrict__ sums, int nchunks, uint32_t *__restrict__ out_
         if (i < nchunks) sums[i] = run;
         run += v[k];
     }
-    if (threadIdx.x == 0) *out_total = tot;
+    if (threadIdx.x == 0) {
+        *out_total = tot;
+        totals[0] = 0;      // dropped entries, added up by k_sector_fill
+        totals[1] = tot;
+    }
+}
+
+// The whole scan where one workgroup holds it (up to kScanOne values), with the
+// slots' sizes and starts: one launch for four.
+constexpr int kScanOne = kScanTopThreads * 16;
+__global__ void __launch_bounds__(kScanTopThreads)
+k_scan_one(const uint32_t *__restrict__ in, int len, uint32_t *__restrict__ out,
+           uint32_t *__restrict__ totals, int slots, uint32_t nb, uint32_t *__restrict__ histo,
+           uint32_t *__restrict__ start)
+{
+    uint32_t v[16], s = 0;
+    const int base = threadIdx.x * 16;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        v[k] = base + k < len ? in[base + k] : 0u;
+        s += v[k];
+    }
+    uint32_t tot;
+    uint32_t run = block_excl_scan<kScanTopThreads>(s, &tot);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (base + k < len) out[base + k] = run;
+        run += v[k];
+    }
+    if (threadIdx.x == 0) {
+        out[len] = tot;
+        totals[0] = 0;
+        totals[1] = tot;
+    }
+    __syncthreads();   // the block's own stores are visible to it
+    for (int i = threadIdx.x; i < slots; i += kScanTopThreads) {
+        const uint32_t a = out[(size_t)i * nb], b = out[(size_t)(i + 1) * nb];
+        start[i] = a;
+        histo[i] = b - a;
+    }
 }
 
 __global__ void __launch_bounds__(kPrepThreads)
@@ -360,9 +416,12 @@ k_scan_down(const uint32_t *__restrict__ in, size_t len, const uint32_t *__restr
 // cursors start at the block's offset plus the entries of the waves before
 // it, and within a 64-row chunk the lanes that share a sector take
 // consecutive slots in lane order.
+// FEW: the cursors of a wave are scalars, one ballot per slot and chunk (28.8 ->
+// 25.2 us on the same rows).
+template <bool FEW>
 __global__ void __launch_bounds__(kPrepThreads)
 k_sector_fill(SectorGeom g, const double *__restrict__ vv, const uint32_t *__restrict__ offsets,
-              uint32_t *__restrict__ rows, uint32_t cap)
+              uint32_t *__restrict__ rows, uint32_t cap, uint32_t *__restrict__ dropped)
 {
     extern __shared__ uint32_t cur[];  // [waves][slots]
     const int slots = g.nsectors + 1;
@@ -380,19 +439,29 @@ k_sector_fill(SectorGeom g, const double *__restrict__ vv, const uint32_t *__res
         v[c] = r < g.n ? vv[r] : 0.0;
     }
     uint32_t *my = cur + wave * slots;
+    uint32_t again = 0, at[kFewSectors + 1] = {};
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
         const size_t r = r0 + c * 64 + lane;
         int s[3] = {-1, -1, -1};
         if (r < g.n) row_sectors(g, v[c], s, bad);
-        if (g.nsectors <= kAggregateSectors) {
-            for_each_sector(s, [&](int sec, unsigned long long m, bool) {
-                if (lane == 0) my[sec] += (uint32_t)__popcll(m);
-            });
+        if constexpr (FEW) {
+#pragma unroll
+            for (int q = 0; q <= kFewSectors; ++q) at[q] += (uint32_t)__popcll(slot_lanes(s, q));
         } else {
             for (int j = 0; j < 3; ++j)
                 if (s[j] >= 0) atomicAdd(&my[s[j]], 1u);
         }
+    }
+    if constexpr (FEW) {
+        if (lane == 0)
+#pragma unroll
+            for (int q = 0; q <= kFewSectors; ++q)
+                if (q < slots) my[q] = at[q];
+    }
+    if (__any(bad != 0)) {   // one atomic a wave; cur may fill the LDS of a block
+        for (int o = 32; o; o >>= 1) bad += __shfl_down(bad, o);
+        if (lane == 0) atomicAdd(dropped, bad);
     }
     __syncthreads();
     for (int s = threadIdx.x; s < slots; s += kPrepThreads) {
@@ -404,12 +473,30 @@ k_sector_fill(SectorGeom g, const double *__restrict__ vv, const uint32_t *__res
         }
     }
     __syncthreads();
+    if constexpr (FEW) {
+#pragma unroll
+        for (int q = 0; q <= kFewSectors; ++q)
+            at[q] = q < slots ? __builtin_amdgcn_readfirstlane(my[q]) : 0u;
+    }
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
         const size_t r = r0 + c * 64 + lane;
         int s[3] = {-1, -1, -1};
-        if (r < g.n) row_sectors(g, v[c], s, bad);
+        if (r < g.n) row_sectors(g, v[c], s, again);
         // Lanes sharing a sector take consecutive slots in lane order.
+        if constexpr (FEW) {
+#pragma unroll
+            for (int q = 0; q <= kFewSectors; ++q) {
+                const unsigned long long m = slot_lanes(s, q);
+                if (s[0] == q || s[1] == q || s[2] == q) {
+                    const uint32_t pos = at[q] + __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    if (pos < cap) rows[pos] = (uint32_t)r;
+                }
+                at[q] += (uint32_t)__popcll(m);
+            }
+            continue;
+        }
         for_each_sector(s, [&](int sec, unsigned long long m, bool mine) {
             const uint32_t base = my[sec];
             if (mine) {
@@ -437,53 +524,40 @@ __global__ void k_sector_histo(int slots, uint32_t nb, const uint32_t *__restric
 // Sector gather (gridding_cpu.c:118-138): output row icount takes list entry
 // nsec-1-icount.
 
+// One thread per visibility of each output row (V float, or float4 when F*P is a
+// multiple of 4 and the arrays are 16-byte aligned); a row's first thread moves
+// its coordinates and weights too, so all of a row's loads are under way at once
+// (two launches before; a slab of 750 k rows of 4 channels 27.3 -> 24.6 us, bound
+// by the 64-byte segments that the scattered rows are read in).
+// shift: log2 of FPV, or -1 if it is not a power of two.
+template <typename V>
 __global__ void __launch_bounds__(kPrepThreads)
-k_gather_rows(const uint32_t *__restrict__ list, uint32_t nsec, uint32_t n, double vshift,
-              uint32_t P, const double *__restrict__ uu, const double *__restrict__ vv,
-              const double *__restrict__ ww, const float *__restrict__ wt,
-              double *__restrict__ uus, double *__restrict__ vvs, double *__restrict__ wws,
-              float *__restrict__ wts)
-{
-    const uint32_t ic = blockIdx.x * kPrepThreads + threadIdx.x;
-    if (ic >= nsec) return;
-    const uint32_t src = list[nsec - 1 - ic];
-    if (src >= n) return;
-    uus[ic] = uu[src];
-    vvs[ic] = vv[src] - vshift;
-    wws[ic] = ww[src];
-    for (uint32_t p = 0; p < P; ++p) wts[(size_t)ic * P + p] = wt[(size_t)src * P + p];
-}
-
-__global__ void __launch_bounds__(kPrepThreads)
-k_gather_vis(const uint32_t *__restrict__ list, uint32_t nsec, uint32_t n, uint32_t FP,
-             const float *__restrict__ vr, const float *__restrict__ vi, float *__restrict__ vrs,
-             float *__restrict__ vis)
+k_gather(const uint32_t *__restrict__ list, uint32_t nsec, uint32_t n, double vshift, uint32_t P,
+         uint32_t FPV, int shift, const double *__restrict__ uu, const double *__restrict__ vv,
+         const double *__restrict__ ww, const float *__restrict__ wt, const V *__restrict__ vr,
+         const V *__restrict__ vi, double *__restrict__ uus, double *__restrict__ vvs,
+         double *__restrict__ wws, float *__restrict__ wts, V *__restrict__ vrs,
+         V *__restrict__ vis)
 {
     const size_t e = (size_t)blockIdx.x * kPrepThreads + threadIdx.x;
-    if (e >= (size_t)nsec * FP) return;
-    const uint32_t ic = (uint32_t)(e / FP), k = (uint32_t)(e - (size_t)ic * FP);
+    const size_t row = shift >= 0 ? e >> shift : e / FPV;
+    if (row >= nsec) return;
+    const uint32_t ic = (uint32_t)row, k = (uint32_t)(e - row * FPV);
     const uint32_t src = list[nsec - 1 - ic];
     if (src >= n) return;
-    const size_t from = (size_t)src * FP + k;
-    vrs[e] = vr[from];
-    vis[e] = vi[from];
-}
-
-// Same, four floats per thread when F*P is a multiple of 4 (16-byte aligned
-// row segments).
-__global__ void __launch_bounds__(kPrepThreads)
-k_gather_vis4(const uint32_t *__restrict__ list, uint32_t nsec, uint32_t n, uint32_t FP4,
-              const float4 *__restrict__ vr, const float4 *__restrict__ vi,
-              float4 *__restrict__ vrs, float4 *__restrict__ vis)
-{
-    const size_t e = (size_t)blockIdx.x * kPrepThreads + threadIdx.x;
-    if (e >= (size_t)nsec * FP4) return;
-    const uint32_t ic = (uint32_t)(e / FP4), k = (uint32_t)(e - (size_t)ic * FP4);
-    const uint32_t src = list[nsec - 1 - ic];
-    if (src >= n) return;
-    const size_t from = (size_t)src * FP4 + k;
-    vrs[e] = vr[from];
-    vis[e] = vi[from];
+    const size_t from = (size_t)src * FPV + k;
+    const V a = vr[from], b = vi[from];
+    if (k == 0) {
+        const double u = uu[src], v = vv[src], w = ww[src];
+        const float w0 = wt[(size_t)src * P];
+        uus[ic] = u;
+        vvs[ic] = v - vshift;
+        wws[ic] = w;
+        wts[(size_t)ic * P] = w0;
+        for (uint32_t p = 1; p < P; ++p) wts[(size_t)ic * P + p] = wt[(size_t)src * P + p];
+    }
+    vrs[e] = a;
+    vis[e] = b;
 }
 
 // ---------------------------------------------------------------------------
@@ -513,7 +587,7 @@ size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 struct SectorLayout {
     uint32_t nb;
     size_t len, nchunks;
-    size_t counts, offsets, sums, bad, bytes;  // byte offsets into the workspace
+    size_t counts, offsets, sums, totals, bytes;  // byte offsets into the workspace
 };
 
 bool sector_layout(uint32_t n, int nsectors, SectorLayout &L)
@@ -524,8 +598,8 @@ bool sector_layout(uint32_t n, int nsectors, SectorLayout &L)
     L.counts = 0;
     L.offsets = align256(L.counts + L.len * 4);
     L.sums = align256(L.offsets + (L.len + 1) * 4);
-    L.bad = align256(L.sums + L.nchunks * 4);
-    L.bytes = align256(L.bad + 4);
+    L.totals = align256(L.sums + L.nchunks * 4);   // dropped entries, all entries
+    L.bytes = align256(L.totals + 8);
     return L.nchunks <= (size_t)kMaxScanChunks;
 }
 
@@ -597,7 +671,7 @@ int sector_bin_run(unsigned int num_points, const double *vv, int nsectors, int 
     uint32_t *counts = reinterpret_cast<uint32_t *>(w + L.counts);
     uint32_t *offsets = reinterpret_cast<uint32_t *>(w + L.offsets);
     uint32_t *sums = reinterpret_cast<uint32_t *>(w + L.sums);
-    uint32_t *bad = reinterpret_cast<uint32_t *>(w + L.bad);
+    uint32_t *totals = reinterpret_cast<uint32_t *>(w + L.totals);
     SectorGeom g;
     g.nsectors = nsectors;
     g.yaxis = yaxis;
@@ -605,35 +679,52 @@ int sector_bin_run(unsigned int num_points, const double *vv, int nsectors, int 
     g.supporth = (double)((w_support - 1) / 2) * dx;  // init.c:13
     g.n = num_points;
     g.nb = L.nb;
-    PREP_HIP(hipMemsetAsync(bad, 0, 4, s));
-    hipLaunchKernelGGL(k_sector_count, dim3(L.nb), dim3(kPrepThreads), 0, s, g, vv, counts, bad);
-    PREP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)L.nchunks), dim3(kPrepThreads), 0, s, counts,
-                       L.len, sums);
-    PREP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, s, sums, (int)L.nchunks,
-                       offsets + L.len);
-    PREP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_scan_down, dim3((unsigned)L.nchunks), dim3(kPrepThreads), 0, s, counts,
-                       L.len, sums, offsets);
-    PREP_HIP(hipGetLastError());
     const int slots = nsectors + 1;
+    const bool one = L.len <= (size_t)kScanOne;
+    const bool few = nsectors <= kFewSectors;
+    if (few)
+        hipLaunchKernelGGL(k_sector_count<true>, dim3(L.nb), dim3(kPrepThreads), 0, s, g, vv,
+                           counts);
+    else
+        hipLaunchKernelGGL(k_sector_count<false>, dim3(L.nb), dim3(kPrepThreads), 0, s, g, vv,
+                           counts);
+    PREP_HIP(hipGetLastError());
+    if (one) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(kScanTopThreads), 0, s, counts, (int)L.len,
+                           offsets, totals, slots, L.nb, histo, start);
+        PREP_HIP(hipGetLastError());
+    } else {
+        hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)L.nchunks), dim3(kPrepThreads), 0, s,
+                           counts, L.len, sums);
+        PREP_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, s, sums, (int)L.nchunks,
+                           offsets + L.len, totals);
+        PREP_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_scan_down, dim3((unsigned)L.nchunks), dim3(kPrepThreads), 0, s,
+                           counts, L.len, sums, offsets);
+        PREP_HIP(hipGetLastError());
+    }
     const size_t lds = (size_t)(kPrepThreads / 64) * slots * sizeof(uint32_t);
-    hipLaunchKernelGGL(k_sector_fill, dim3(L.nb), dim3(kPrepThreads), lds, s, g, vv, offsets,
-                       rows, rows_capacity);
+    if (few)
+        hipLaunchKernelGGL(k_sector_fill<true>, dim3(L.nb), dim3(kPrepThreads), lds, s, g, vv,
+                           offsets, rows, rows_capacity, totals);
+    else
+        hipLaunchKernelGGL(k_sector_fill<false>, dim3(L.nb), dim3(kPrepThreads), lds, s, g, vv,
+                           offsets, rows, rows_capacity, totals);
     PREP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_sector_histo, dim3((slots + 255) / 256), dim3(256), 0, s, slots, L.nb,
-                       offsets, histo, start);
-    PREP_HIP(hipGetLastError());
-    uint32_t host[2];
-    PREP_HIP(hipMemcpyAsync(&host[0], offsets + L.len, 4, hipMemcpyDeviceToHost, s));
-    PREP_HIP(hipMemcpyAsync(&host[1], bad, 4, hipMemcpyDeviceToHost, s));
+    if (!one) {
+        hipLaunchKernelGGL(k_sector_histo, dim3((slots + 255) / 256), dim3(256), 0, s, slots, L.nb,
+                           offsets, histo, start);
+        PREP_HIP(hipGetLastError());
+    }
+    uint32_t host[2];   // dropped, total
+    PREP_HIP(hipMemcpyAsync(host, totals, 8, hipMemcpyDeviceToHost, s));
     PREP_HIP(hipStreamSynchronize(s));
-    if (total_entries) *total_entries = host[0];
-    if (dropped) *dropped = host[1];
-    if (host[0] > rows_capacity)
+    if (total_entries) *total_entries = host[1];
+    if (dropped) *dropped = host[0];
+    if (host[1] > rows_capacity)
         return set_status(RICK_ERR_INVALID, "rows capacity %u < %u sector entries", rows_capacity,
-                          host[0]);
+                          host[1]);
     return RICK_OK;
 }
 
@@ -756,25 +847,25 @@ int rick_sector_gather(const unsigned int *list, unsigned int nsec, int isector,
     // gridding_cpu.c:24 shift = dx*yaxis; vvs = vv - isector*shift (line 121).
     const double shift = (double)(dx * yaxis);
     const double vshift = (double)(unsigned)isector * shift;
-    hipLaunchKernelGGL(k_gather_rows, dim3((nsec + kPrepThreads - 1) / kPrepThreads),
-                       dim3(kPrepThreads), 0, s, list, nsec, num_points, vshift, polarizations,
-                       uu, vv, ww, weight, uus, vvs, wws, weightss);
-    PREP_HIP(hipGetLastError());
     const uint32_t FP = freq_per_chan * polarizations;
     const bool vec = FP % 4 == 0 &&
                      ((uintptr_t)vis_real | (uintptr_t)vis_img | (uintptr_t)visreals |
                       (uintptr_t)visimgs) % 16 == 0;
     const size_t ne = (size_t)nsec * (vec ? FP / 4 : FP);
     const dim3 grd((unsigned)((ne + kPrepThreads - 1) / kPrepThreads));
+    const uint32_t fpv = vec ? FP / 4 : FP;
+    const int sh = (fpv & (fpv - 1)) == 0 ? __builtin_ctz(fpv) : -1;
     if (vec)
-        hipLaunchKernelGGL(k_gather_vis4, grd, dim3(kPrepThreads), 0, s, list, nsec, num_points,
-                           FP / 4, reinterpret_cast<const float4 *>(vis_real),
-                           reinterpret_cast<const float4 *>(vis_img),
+        hipLaunchKernelGGL(k_gather<float4>, grd, dim3(kPrepThreads), 0, s, list, nsec, num_points,
+                           vshift, polarizations, fpv, sh, uu, vv, ww, weight,
+                           reinterpret_cast<const float4 *>(vis_real),
+                           reinterpret_cast<const float4 *>(vis_img), uus, vvs, wws, weightss,
                            reinterpret_cast<float4 *>(visreals),
                            reinterpret_cast<float4 *>(visimgs));
     else
-        hipLaunchKernelGGL(k_gather_vis, grd, dim3(kPrepThreads), 0, s, list, nsec, num_points,
-                           FP, vis_real, vis_img, visreals, visimgs);
+        hipLaunchKernelGGL(k_gather<float>, grd, dim3(kPrepThreads), 0, s, list, nsec, num_points,
+                           vshift, polarizations, fpv, sh, uu, vv, ww, weight, vis_real, vis_img,
+                           uus, vvs, wws, weightss, visreals, visimgs);
     PREP_HIP(hipGetLastError());
     return RICK_OK;
 }

@@ -75,8 +75,8 @@ def sector_bin(vv, nsectors: int, yaxis: int, dx: float, w_support: int) -> Sect
         raise ValueError(f"sector binning does not handle {n} rows x {nsectors} sectors")
     work = torch.empty(ws, dtype=torch.uint8, device=dev)
     cap = max(1, 3 * n)
-    histo = torch.empty(nsectors + 1, dtype=torch.int32, device=dev)
-    start = torch.empty(nsectors + 1, dtype=torch.int32, device=dev)
+    both = torch.empty(2, nsectors + 1, dtype=torch.int32, device=dev)
+    histo, start = both[0], both[1]
     rows = torch.empty(cap, dtype=torch.int32, device=dev)
     total = ctypes.c_ulong()
     dropped = ctypes.c_uint()
@@ -85,7 +85,8 @@ def sector_bin(vv, nsectors: int, yaxis: int, dx: float, w_support: int) -> Sect
         ctypes.c_void_p(histo.data_ptr()), ctypes.c_void_p(start.data_ptr()),
         ctypes.c_void_p(rows.data_ptr()), cap, ctypes.c_void_p(work.data_ptr()), _stream(dev),
         ctypes.byref(total), ctypes.byref(dropped)))
-    return SectorBins(histo.cpu(), start.cpu(), rows[:total.value], int(total.value),
+    both = both.cpu()
+    return SectorBins(both[0], both[1], rows[:total.value], int(total.value),
                       int(dropped.value), nsectors)
 
 

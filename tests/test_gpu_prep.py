@@ -112,6 +112,17 @@ def test_sector_bin_empty_and_tiny():
     check_bins(np.array([0.5]), 1, 512, 1 / 512, 7)
 
 
+# Ballots per slot up to 4 slabs and LDS atomics above; the one-workgroup scan up to
+# 16384 values (4096 slots x 4 blocks) and the three-launch one above.
+@pytest.mark.parametrize("S,n", [(3, 12_289), (4, 12_289), (5, 12_289), (4095, 16_384),
+                                 (4095, 16_385)])
+def test_sector_bin_either_side_of_its_rules(S, n):
+    print(f"case sector_bin S={S} n={n}", flush=True)
+    vv = np.random.default_rng(S + n).uniform(-0.4, 1.4, n)     # some rows in no slab
+    vv[::97] = np.nan
+    assert check_bins(vv, S, max(1, 8192 // S), 1 / 8192, 7).dropped > 0
+
+
 @pytest.mark.parametrize("isector,F,P", [(0, 4, 2), (2, 4, 2), (1, 3, 1)])
 def test_sector_gather_matches_oracle(isector, F, P):
     n, S = 70_001, 4
