@@ -38,15 +38,12 @@ constexpr int kE = 16;  // complex values per thread
 constexpr int kFusedStrips = 256;   // column strips from which the fused phase pass fills the chip
 
 // The fused column/phase pass: complex values per thread for FP64 and FP32
-// plane data, and whether FP64 prefetches the next plane into registers.
+// plane data.
 #ifndef RICK_PHASE_E_F64
 #define RICK_PHASE_E_F64 8
 #endif
 #ifndef RICK_PHASE_E_F32
 #define RICK_PHASE_E_F32 8
-#endif
-#ifndef RICK_PHASE_PREFETCH_F64
-#define RICK_PHASE_PREFETCH_F64 0
 #endif
 // FP64: the w-phase rotation of a pixel advances plane to plane by a fixed
 // step (exp(i 2 pi dw (n-1))), one complex multiply per plane instead of a
@@ -74,7 +71,6 @@ template <typename T>
 constexpr int row_values() { return sizeof(T) == 8 ? RICK_ROWS_E_F64 : RICK_ROWS_E_F32; }
 template <typename T>
 constexpr int col_values() { return sizeof(T) == 8 ? RICK_COLS_E_F64 : RICK_COLS_E_F32; }
-constexpr bool kPhasePrefetchF64 = RICK_PHASE_PREFETCH_F64 != 0;
 constexpr bool kPhaseRecurF64 = RICK_PHASE_RECUR_F64 != 0;
 template <typename T>
 constexpr int phase_values(int L)
@@ -192,18 +188,41 @@ __device__ __forceinline__ void bmap(int b, int &g, int &j)
     else { g = b % G; j = b / G; }
 }
 
-// Where the last pass delivers element n of line g (register slot idx):
-// by default to global memory, after the optional four-step twiddle and the
-// output scale.
+// Reads of a column strip through a buffer descriptor: 32-bit offsets (a plane is at
+// most 8192^2 x 16 bytes), the uniform part of an address in a scalar register, and
+// a read at kNowhere, past the descriptor's end, gives zero -- so lines that do not
+// exist and rows without a cell need no branch, and a thread's reads are all under
+// way at once.
+constexpr uint32_t kNowhere = 0x80000000u;
+template <typename T>
+struct ColBuf {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ ColBuf(const C2<T> *p, size_t elements)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<C2<T> *>(p), 0,
+                                              (int)(uint32_t)(elements * sizeof(C2<T>)), 0x00027000))
+    {
+    }
+    // At byte offset `v` (of the lane) + `s` (uniform); streamed, not kept in caches.
+    __device__ __forceinline__ C2<T> load(uint32_t v, uint32_t s) const
+    {
+        if constexpr (sizeof(T) == 4)
+            return __builtin_bit_cast(C2<T>, __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 2));
+        else
+            return __builtin_bit_cast(C2<T>, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 2));
+    }
+};
+
+// Where the last pass delivers element n of line g: to global memory, after the
+// optional four-step twiddle and the output scale.
 template <typename T>
 struct GlobalSink {
+    static constexpr bool kLoops = false;
     C2<T> *gout;
     const Lines *ln;
     const C2<T> *tw;
     T scale;
-    __device__ __forceinline__ void operator()(int g, int n, int idx, C2<T> o) const
+    __device__ __forceinline__ void operator()(int g, int n, C2<T> o) const
     {
-        (void)idx;
         if (ln->tw_set) o = cmul(o, tw[(size_t)n * ln->tw_set]);
         o.x *= scale;
         o.y *= scale;
@@ -212,24 +231,47 @@ struct GlobalSink {
     }
 };
 
-// First-pass input of this thread: element n of line g for butterfly slot
-// i*R + r, or zero where the line does not exist or the input is known zero.
-template <typename T, int L, int G, bool ROWS, int E = kE>
+// Whether the fused column/phase pass loads the next plane while it transforms one.
+// FP64 has registers for two waves per SIMD, and the loads hide what two waves leave
+// open; lines of 128 points and more have none left for it (8 planes of 4096^2,
+// 64-point lines: 506 -> 433 us; 16 planes of 4096 x 512, 512-point lines: 139 -> 170).
+// FP32 has four waves per SIMD and is slower with it (64 planes of 8192^2: 7.5 -> 8.7 ms).
+template <typename T, int L>
+constexpr bool phase_prefetch() { return sizeof(T) == 8 && L <= 64; }
+
+// First-pass input of this thread of a column strip: element n of line g for
+// butterfly slot i*R + r, or zero where the line does not exist or the input is known
+// zero.  Loads that the butterflies wait for go out together through the buffer
+// (FP32, 64 planes of 8192^2: 11.0 ms one by one, 7.5 together); prefetched ones are
+// better spread over the transform (FP64, 8 planes of 8192^2: 1.98 ms together, 1.69).
+template <typename T, int L, int G, int E>
 __device__ __forceinline__ void load_first(C2<T> *vals, int tid, const Lines &ln,
                                            const C2<T> *gin)
 {
     constexpr int R = radix_of(L, 0, E), LR = L / R, BPT = E / R;
     constexpr int NT = G * L / E;
+    const uint32_t el = (uint32_t)ln.in_el * (uint32_t)sizeof(C2<T>);
+    const ColBuf<T> buf(gin + ln.in_base, (size_t)(L - 1) * ln.in_el + ln.nvalid);
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
         int g, j;
-        bmap<ROWS, LR, G>(tid + i * NT, g, j);
+        bmap<false, LR, G>(tid + i * NT, g, j);
+        if constexpr (phase_prefetch<T, L>()) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int n = j + r * LR;
-            const bool live = elem_live(ln, g, n);
-            const size_t at = ln.in_base + (size_t)g * ln.in_line + (size_t)n * ln.in_el;
-            vals[i * R + r] = live ? load_stream2(&gin[at]) : C2<T>{T(0), T(0)};
+            for (int r = 0; r < R; ++r) {
+                const int n = j + r * LR;
+                vals[i * R + r] = elem_live(ln, g, n)
+                                      ? load_stream2(&gin[ln.in_base + g + (size_t)n * ln.in_el])
+                                      : C2<T>{T(0), T(0)};
+            }
+        } else {
+            const uint32_t at = g < ln.nvalid ? j * el + g * (uint32_t)sizeof(C2<T>) : kNowhere;
+            bool live[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) live[r] = !ln.rowlive || ln.rowlive[j + r * LR];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                vals[i * R + r] = buf.load(live[r] ? at : kNowhere, r * LR * el);
         }
     }
 }
@@ -259,7 +301,9 @@ __device__ __forceinline__ void pass(C2<T> *vals, int tid, const Lines &ln, int 
         constexpr int R = radix_of(L, P, E), Ns = ns_of(L, P, E), LR = L / R, BPT = E / R;
         constexpr int NT = G * L / E;
         constexpr bool from_lds = P > 0, to_lds = P + 1 < NP;
-        if constexpr (!PRE) {
+        if constexpr (!PRE && !from_lds && Sink::kLoops) {
+            load_first<T, L, G, E>(vals, tid, ln, gin);
+        } else if constexpr (!PRE) {
 #pragma unroll
             for (int i = 0; i < BPT; ++i) {
                 int g, j;
@@ -278,7 +322,7 @@ __device__ __forceinline__ void pass(C2<T> *vals, int tid, const Lines &ln, int 
                     }
                 }
             }
-            if constexpr (from_lds) __syncthreads();
+            if constexpr (from_lds && (to_lds || !Sink::kLoops)) __syncthreads();
         }
 #pragma unroll
         for (int i = 0; i < BPT; ++i) {
@@ -287,16 +331,21 @@ __device__ __forceinline__ void pass(C2<T> *vals, int tid, const Lines &ln, int 
             C2<T> *v = vals + i * R;
             if constexpr (Ns > 1) twiddle<T, R>(v, j % Ns, (L / (Ns * R)) * ts, tw);
             dftR<T, R>(v);
-            if constexpr (!(to_lds && SPLIT)) {
+            if constexpr (to_lds ? !SPLIT : !Sink::kLoops) {
+                // A repeated transform: the one before has been read first.
+                if constexpr (Sink::kLoops && P == 0) {
+                    if (i == 0) __syncthreads();
+                }
                 const int dbase = (j / Ns) * Ns * R + j % Ns;
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const int n = dbase + r * Ns;
                     if constexpr (to_lds) lds[lds_at<ROWS, L, G>(g, n)] = v[r];
-                    else sink(g, n, i * R + r, v[r]);
+                    else sink(g, n, v[r]);
                 }
             }
         }
+        if constexpr (!to_lds && Sink::kLoops) sink.finish(vals, tid);
         if constexpr (to_lds && SPLIT) {
             // Outputs of this pass are in vals; move them to the next pass's
             // layout one component at a time.
@@ -525,39 +574,64 @@ k_fft_cols(ColArgs a, const C2<T> *__restrict__ tw, const C2<T> *gin, C2<T> *gou
 // every w-plane in turn and accumulates the phase-rotated results of each
 // output pixel in registers; only the image is written.  Output element n of
 // set s is image row  s*vs_mul + n*v_stride.
-template <typename T, int E>
+// All of a thread's pixels take their phase together after the transform's last
+// butterfly; one by one, each behind the test of the option, every pixel waited for
+// its own LDS read and sine (FP32 64 planes of 8192^2 8.2 -> 7.5 ms, 16 planes of
+// 4096 x 512 134 -> 84 us; FP64 32 planes of 4096^2 1.85 -> 1.64 ms, with the
+// prefetch 1.39).  The pass reads its planes at 4.6 TB/s (FP32) and 6.2 TB/s (FP64)
+// then, the FP32 one with its vector units two thirds busy.
+template <typename T, int L, int E>
 struct PhaseSink {
     static constexpr bool kRecur = sizeof(T) == 8 && kPhaseRecurF64;
+    static constexpr bool kLoops = true;
+    static constexpr int G = lines_per_wg(L), NT = G * L / E;
+    // The last pass's element layout: register i * R + r holds element n0 + r * Ns.
+    static constexpr int P = npasses(L, E) - 1, R = radix_of(L, P, E), Ns = ns_of(L, P, E),
+                         LR = L / R, BPT = E / R;
     double are[E], aim[E];
     // FP64: n of each of this thread's pixels (set once), or, with the
     // recurrence, each pixel's current rotation and its per-plane step.
-    double nfv[kRecur ? 1 : E];
+    double nfv[kRecur || sizeof(T) == 4 ? 1 : E];
     double rc[kRecur ? E : 1], rs[kRecur ? E : 1], sc[kRecur ? E : 1], ss[kRecur ? E : 1];
     const double *nfl;    // FP32: n - 1 of the workgroup's pixels in LDS, [n * G + g]
-    int G;
-    const double *ltab, *mtab;
     double wterm, dwnorm;
-    int u0, s, vs_mul, v_stride, nvalid;
     bool phase;
-    __device__ __forceinline__ void operator()(int g, int n, int idx, C2<T> o)
+    // (Lines that do not exist were read as zero and add zero.)
+    __device__ __forceinline__ void finish(const C2<T> *o, int tid)
     {
-        if (g >= nvalid) return;
         if (!phase) {
-            are[idx] += (double)o.x;
-            aim[idx] += (double)o.y;
-            return;
-        }
-        if constexpr (kRecur) {
-            // (p + iq) * exp(i arg_w); dwnorm * n is applied once at the end.
-            const double r = rc[idx], q = rs[idx];
-            are[idx] += (double)o.x * r - (double)o.y * q;
-            aim[idx] += (double)o.x * q + (double)o.y * r;
-            rc[idx] = r * sc[idx] - q * ss[idx];
-            rs[idx] = r * ss[idx] + q * sc[idx];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                are[e] += (double)o[e].x;
+                aim[e] += (double)o[e].y;
+            }
+        } else if constexpr (kRecur) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                // (p + iq) * exp(i arg_w); dwnorm * n is applied once at the end.
+                const double r = rc[e], q = rs[e];
+                are[e] += (double)o[e].x * r - (double)o[e].y * q;
+                aim[e] += (double)o[e].x * q + (double)o[e].y * r;
+                rc[e] = r * sc[e] - q * ss[e];
+                rs[e] = r * ss[e] + q * sc[e];
+            }
         } else if constexpr (sizeof(T) == 8) {
-            phase_add_f64(o.x, o.y, wterm, nfv[idx], dwnorm, are[idx], aim[idx]);
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                phase_add_f64(o[e].x, o[e].y, wterm, nfv[e], dwnorm, are[e], aim[e]);
         } else {
-            phase_add_f32(o.x, o.y, wterm, nfl[n * G + g], are[idx], aim[idx]);
+            double nm1[E];
+#pragma unroll
+            for (int i = 0; i < BPT; ++i) {
+                int g, j;
+                bmap<false, LR, G>(tid + i * NT, g, j);
+                const double *p = nfl + ((j / Ns) * Ns * R + j % Ns) * G + g;
+#pragma unroll
+                for (int r = 0; r < R; ++r) nm1[i * R + r] = p[r * Ns * G];
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                phase_add_f32(o[e].x, o[e].y, wterm, nm1[e], are[e], aim[e]);
         }
     }
 };
@@ -596,23 +670,17 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
     __shared__ double nfl[sizeof(T) == 4 ? G * L : 1];
     const int c0 = blockIdx.x * G;
     const int s = blockIdx.y;
-    PhaseSink<T, E> sink;
+    PhaseSink<T, L, E> sink;
 #pragma unroll
     for (int i = 0; i < E; ++i) sink.are[i] = sink.aim[i] = 0.0;
-    sink.ltab = pg.ltab;
-    sink.mtab = pg.mtab;
     sink.dwnorm = pg.dwnorm;
-    sink.u0 = c0;
-    sink.s = s;
-    sink.vs_mul = vs_mul;
-    sink.v_stride = v_stride;
-    sink.nvalid = min(G, a.nx - c0);
+    const int nvalid = min(G, a.nx - c0);
     sink.phase = pg.phase_on && planes > 1;
     Lines ln;
     ln.in_line = ln.out_line = 1;
     ln.in_el = (size_t)a.in_stride * a.nx;
     ln.out_el = 0;
-    ln.nvalid = sink.nvalid;
+    ln.nvalid = nvalid;
     ln.tw_set = 0;
     ln.occ = nullptr;
     ln.rowlive = nullptr;
@@ -625,12 +693,11 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
         // two waves per SIMD).
         for (int e = threadIdx.x; e < G * L; e += NT) {
             const int g = e % G, n = e / G;
-            nfl[e] = g < sink.nvalid
+            nfl[e] = g < nvalid
                          ? pixel_n(pg.ltab[c0 + g], pg.mtab[s * vs_mul + n * v_stride]) - 1.0
                          : 0.0;
         }
         sink.nfl = nfl;
-        sink.G = G;
         __syncthreads();
     } else {
         // FP64: n of every pixel once, in registers.
@@ -643,9 +710,9 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
             for (int r = 0; r < R; ++r) {
                 const int n = dbase + r * Ns;
                 const double nf =
-                    g < sink.nvalid ? pixel_n(pg.ltab[c0 + g], pg.mtab[s * vs_mul + n * v_stride])
+                    g < nvalid ? pixel_n(pg.ltab[c0 + g], pg.mtab[s * vs_mul + n * v_stride])
                                     : 1.0;
-                if constexpr (PhaseSink<T, E>::kRecur) {
+                if constexpr (PhaseSink<T, L, E>::kRecur) {
                     // Plane 0's argument is the reference's (wterm = wmin,
                     // phase_correction.cu:200, 222); each plane adds dw.
                     double a0, a1;
@@ -668,14 +735,11 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
         ln.in_base = (size_t)pw * (size_t)a.nx * (size_t)a.ny +
                      (size_t)s * a.in_set_mul * (size_t)a.nx + c0;
     };
-    // FP64 runs one wave per SIMD at this register count: the next plane's
-    // inputs are loaded into registers while this plane is transformed.  (The
-    // FP32 variant keeps two waves per SIMD instead, which measured faster.)
-    constexpr bool kPrefetch = sizeof(T) == 8 && kPhasePrefetchF64;
+    constexpr bool kPrefetch = phase_prefetch<T, L>();
     C2<T> vals[E];
     if constexpr (kPrefetch) {
         plane_lines(0);
-        load_first<T, L, G, false, E>(vals, threadIdx.x, ln, grid);
+        load_first<T, L, G, E>(vals, threadIdx.x, ln, grid);
     }
     for (int iw = 0; iw < planes; ++iw) {
         sink.wterm = pg.wmin + iw * pg.dw;  // phase_correction.cu:200
@@ -683,18 +747,16 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
             C2<T> nxt[E];
             if (iw + 1 < planes) {
                 plane_lines(iw + 1);
-                load_first<T, L, G, false, E>(nxt, threadIdx.x, ln, grid);
+                load_first<T, L, G, E>(nxt, threadIdx.x, ln, grid);
             }
-            pass<T, L, G, false, 0, PhaseSink<T, E>, true, false, E>(vals, threadIdx.x, ln, a.ts,
+            pass<T, L, G, false, 0, PhaseSink<T, L, E>, true, false, E>(vals, threadIdx.x, ln, a.ts,
                                                                     tw, lds, grid, sink);
-            __syncthreads();  // LDS is reused by the next plane
 #pragma unroll
             for (int e = 0; e < E; ++e) vals[e] = nxt[e];
         } else {
             plane_lines(iw);
-            pass<T, L, G, false, 0, PhaseSink<T, E>, false, false, E>(vals, threadIdx.x, ln,
+            pass<T, L, G, false, 0, PhaseSink<T, L, E>, false, false, E>(vals, threadIdx.x, ln,
                                                                      a.ts, tw, lds, grid, sink);
-            __syncthreads();  // LDS is reused by the next plane
         }
     }
     // Write the accumulated pixels.
@@ -706,10 +768,10 @@ k_fft_cols_phase(ColArgs a, int planes_in, const C2<T> *__restrict__ tw,
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int n = dbase + r * Ns;
-            if (g < sink.nvalid) {
+            if (g < nvalid) {
                 const size_t pix = (size_t)(s * vs_mul + n * v_stride) * a.nx + (c0 + g);
                 double vre = sink.are[i * R + r], vim = sink.aim[i * R + r];
-                if constexpr (PhaseSink<T, E>::kRecur || sizeof(T) == 4) {
+                if constexpr (PhaseSink<T, L, E>::kRecur || sizeof(T) == 4) {
                     if (sink.phase) {
                         const double nf = pixel_n(pg.ltab[c0 + g], pg.mtab[s * vs_mul + n * v_stride]);
                         vre = vre * pg.dwnorm * nf;

@@ -71,6 +71,35 @@ def test_sparse_chain_matches_separate_stages(nx, ny, planes, tile, precision):
         assert rel_l2(got, want) <= (1e-12 if precision == FP64 else 1e-5)
 
 
+# The fused column/phase pass: lines with and without the prefetch (16 to 64 and 128
+# to 512 points), strips wider than the grid, rows without a cell, one plane (no
+# phase), two and an odd number of them.
+@pytest.mark.parametrize("nx,ny", [
+    (16, 1024), (64, 2048), (32, 4096), (16, 8192), (8192, 128), (4096, 256), (2048, 512)])
+@pytest.mark.parametrize("planes", [1, 2, 5])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_phase_pass_of_every_line_length_matches_stages(nx, ny, planes, precision):
+    print(f"case phase pass {nx}x{ny}x{planes} precision={precision}", flush=True)
+    n = 5000
+    plan = Plan(nx, ny, planes, kernel=rick_amd.KAISERBESSEL, support=7, precision=precision,
+                max_points=n, resolution=1.0 / (4.0 * max(nx, ny)), wmin=-300.0, wmax=500.0)
+    rng = np.random.default_rng(nx + ny + planes)
+    uu = rng.uniform(0.0, 0.9, n)
+    vv = (rng.choice([0.13, 0.71], n) + rng.uniform(0.0, 0.04, n)) * ny / nx
+    ins = [torch.from_numpy(a).to("cuda") for a in (
+        uu, vv, rng.uniform(0.0, 0.9, n), rng.normal(size=n).astype(np.float32),
+        rng.normal(size=n).astype(np.float32), np.ones(n, np.float32))]
+    grid = plan.new_grid()
+    grid.fill_(float("nan"))
+    re, im, _ = plan.image(*ins, grid=grid)
+    dense = plan.grid(*ins)
+    plan.fft(dense)
+    wre, wim = plan.phase(dense)
+    got, want = ((a.cpu().numpy() + 1j * b.cpu().numpy()) for a, b in ((re, im), (wre, wim)))
+    assert np.isfinite(want).all() and np.abs(want).max() > 0
+    assert rel_l2(got, want) <= (1e-12 if precision == FP64 else 1e-5)
+
+
 # Column transforms of one pass (up to 1024 rows in FP64, 2048 in FP32) and the
 # first of two passes above: fewer strips than a round over the XCDs, and paired
 # strips.
