@@ -547,7 +547,7 @@ k_fft_cols(ColArgs a, const C2<T> *__restrict__ tw, const C2<T> *gin, C2<T> *gou
     // FP64 and long lines: an FP32 workgroup of a short line (up to 1024
     // threads) is already at two per CU with whole exchanges, so halving its
     // LDS adds none.
-    constexpr bool kSplit = sizeof(T) == 8 || L >= 1024;
+    constexpr bool kSplit = sizeof(T) == 8 || L >= 1024 || G * L > 8192;
     __shared__ C2<T> lds[kSplit ? G * L / 2 : G * L];
     __shared__ unsigned char rl[L];
     const int c0 = col_strip<T, G>(blockIdx.x, gridDim.x) * G;
@@ -813,12 +813,34 @@ hipError_t launch_rows(int L, int rows_total, const C2<T> *tw, const C2<T> *in, 
 #undef RICK_ROWS
 }
 
+// FP32 lines of 64 points over 256 columns (2 KB a row, 1024 threads of 16 values,
+// split exchange) instead of 128 (of 8 values): longer runs in each page, half as
+// many workgroups.  Pass A, 128 against 256 columns: 16 planes of 4096^2 650 -> 607
+// us, of 8192 x 2048 528 -> 500, 12 of 2048^2 144 -> 131; in-place transform of 8
+// planes of 4096^2 527 -> 458.  It loses where a strip's rows lie more than 2 MB
+// apart (4096 x 8192, 4 MB: 1180 -> 1315 us; 8192 x 4096: 1288 -> 1541) and with one
+// workgroup a CU (512 x 1024 x 8: 13.7 -> 16.5 us; two: 23.6 -> 23.0).  FP64 strips of
+// 2 KB: 4096 x 2048 x 16 635 -> 577 us, but 2048^2 x 16 288 -> 306; left at 1 KB.
+constexpr int kWideStrip = 256;
+bool wide_strips(const ColArgs &a, int sets, int planes)
+{
+    const size_t apart = (size_t)std::max(a.in_stride, a.out_stride) * a.nx * sizeof(C2<float>);
+    return apart <= ((size_t)2 << 20) && (size_t)(a.nx / kWideStrip) * sets * planes >= 512;
+}
+
 template <typename T>
 hipError_t launch_cols(int L, const ColArgs &a, int sets, int planes, const C2<T> *tw,
                        const C2<T> *in, C2<T> *out, hipStream_t s, const ColOcc &co = ColOcc{})
 {
 #define RICK_COLS_BODY(LL)                                                                   \
     {                                                                                        \
+        if constexpr (sizeof(T) == 4 && LL == 64)                                            \
+            if (wide_strips(a, sets, planes)) {                                              \
+                hipLaunchKernelGGL((k_fft_cols<T, LL, kWideStrip, kE>),                      \
+                                   dim3((a.nx + kWideStrip - 1) / kWideStrip, sets, planes), \
+                                   dim3(kWideStrip * LL / kE), 0, s, a, tw, in, out, T(1), co); \
+                return hipGetLastError();                                                    \
+            }                                                                                \
         constexpr int G = col_lines<T>(LL);                                                  \
         constexpr int E = LL >= 1024 ? kE : col_values<T>();                                 \
         hipLaunchKernelGGL((k_fft_cols<T, LL, G, E>), dim3((a.nx + G - 1) / G, sets, planes), \

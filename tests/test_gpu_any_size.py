@@ -115,3 +115,40 @@ def test_long_columns_match_numpy(nx, ny, precision):
     assert rel_l2(cube(plan, out), want) <= (1e-14 if precision == FP64 else 2e-6)
     plan.fft(src)
     assert rel_l2(cube(plan, src), want) <= (1e-14 if precision == FP64 else 2e-6)
+
+
+# FP32 strips of 256 columns from 512 workgroups on (out of place here; in place, a
+# plane at a time, stays below) and of 128 below or where rows lie over 2 MB apart.
+@pytest.mark.parametrize("nx,ny,planes", [(1024, 4096, 2), (2048, 4096, 1), (512, 8192, 2)])
+def test_wide_column_strips_match_numpy(nx, ny, planes):
+    print(f"case wide columns {nx}x{ny}x{planes}", flush=True)
+    plan = Plan(nx, ny, planes, precision=FP32)
+    rng = np.random.default_rng(nx + ny)
+    src = torch.from_numpy(rng.normal(size=2 * planes * ny * nx)).to("cuda", plan.grid_dtype)
+    want = np.fft.ifft2(cube(plan, src), axes=(1, 2))
+    out = plan.fft(src, torch.empty_like(src))
+    assert rel_l2(cube(plan, out), want) <= 2e-6
+    plan.fft(src)
+    assert rel_l2(cube(plan, src), want) <= 2e-6
+
+
+@pytest.mark.parametrize("planes", [7, 8])      # 448 and 512 workgroups of 256 columns
+def test_wide_column_strips_on_a_sparse_grid(planes):
+    print(f"case wide chain planes={planes}", flush=True)
+    n, nx, ny = 20000, 1024, 1024
+    plan = Plan(nx, ny, planes, kernel=rick_amd.KAISERBESSEL, support=7, precision=FP32,
+                max_points=n, resolution=1.0 / (4.0 * nx), wmin=-300.0, wmax=500.0)
+    rng = np.random.default_rng(planes)
+    ins = [torch.from_numpy(a).to("cuda") for a in (
+        rng.uniform(0.0, 0.9, n), rng.choice([0.13, 0.47], n) + rng.uniform(0.0, 0.04, n),
+        rng.uniform(0.0, 0.9, n), rng.normal(size=n).astype(np.float32),
+        rng.normal(size=n).astype(np.float32), np.ones(n, np.float32))]
+    grid = plan.new_grid()
+    grid.fill_(float("nan"))
+    re, im, _ = plan.image(*ins, grid=grid)
+    dense = plan.grid(*ins)
+    plan.fft(dense)
+    wre, wim = plan.phase(dense)
+    got, want = ((a.cpu().numpy() + 1j * b.cpu().numpy()) for a, b in ((re, im), (wre, wim)))
+    assert np.isfinite(want).all() and np.abs(want).max() > 0
+    assert rel_l2(got, want) <= 1e-5
