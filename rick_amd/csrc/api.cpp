@@ -499,15 +499,15 @@ int rick_plan_image(rick_plan p, unsigned int n, unsigned int F, unsigned int P,
         const bool chain = gen_chain_ok(p->gen);
         RICK_HIP(launch_grid(p->geom, p->work, p->d.precision, p->table_d, n, F, P, uu, vv, ww,
                              vr, vi, wt, grid, 0, s, &p->timing, !chain));
-        int n1 = 1, n2 = 0;
-        if (chain)
+        if (chain) {
             RICK_HIP(launch_gen_chain(p->gen, p->d.precision, p->geom.planes, p->geom.nx,
                                       p->geom.ny, grid, norm, s, &p->timing, p->geom,
-                                      p->work.offsets, p->work.rowlive, &n1, &n2));
-        else
-            RICK_HIP(launch_fft_gen(p->gen, p->d.precision, p->geom.planes, p->geom.nx,
-                                    p->geom.ny, grid, grid, norm, s, &p->timing));
-        RICK_HIP(launch_phase(p->phase, p->d.precision, grid, re, im, 0, s, &p->timing, n1, n2));
+                                      p->work.offsets, p->work.rowlive, p->phase, re, im));
+            return RICK_OK;
+        }
+        RICK_HIP(launch_fft_gen(p->gen, p->d.precision, p->geom.planes, p->geom.nx, p->geom.ny,
+                                grid, grid, norm, s, &p->timing));
+        RICK_HIP(launch_phase(p->phase, p->d.precision, grid, re, im, 0, s, &p->timing));
         return RICK_OK;
     }
     // Sparse grid: tiles of empty buckets are left unwritten; the row FFT

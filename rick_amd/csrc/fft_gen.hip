@@ -26,6 +26,7 @@
 
 #include "fft_kernels.h"
 #include "rick_internal.h"
+#include "rick_math.h"
 #include "rick_tables.h"
 
 namespace rick {
@@ -41,8 +42,10 @@ constexpr size_t kBlueChunk = size_t(1) << 25;   // Bluestein scratch: elements 
 
 constexpr int kGenLdsBytes = 80 * 1024;          // dynamic LDS of a workgroup, at most
 
-// Butterflies of radix R a thread takes in one pass.
-__host__ __device__ constexpr int gen_bpt(int R) { return kGenValues / R > 1 ? kGenValues / R : 1; }
+constexpr int kPhaseValues = 10;      // the same in the fused phase pass (its largest radix)
+
+// Butterflies of radix R a thread of V values takes in one pass.
+__host__ __device__ constexpr int gen_bpt(int R, int V) { return V / R > 1 ? V / R : 1; }
 
 // floor(x / d) for x * d < 2^32, from m = ceil(2^32 / d) (d > 1; 0 stands for 1).
 __host__ __device__ inline uint32_t gen_magic(uint32_t d)
@@ -278,15 +281,55 @@ struct GenCtx {
     T scale;
 };
 
+// The last column pass of the FP64 image chain: instead of the transformed planes,
+// their phase-rotated sum, kept per pixel by the thread that transforms it.  Element n
+// of set s is image row s + n * row_mul (k1 + N1 * k2).
+struct GenPhase {
+    static constexpr bool kOn = true;
+    static constexpr int kValues = kPhaseValues;
+    PhaseGeom g;
+    double *ore, *oim;
+    int iw, row_mul;
+    bool phase;
+    double are[kValues], aim[kValues], nf[kValues];
+    __device__ __forceinline__ void add(C2<double> o, int idx, int iu, int iv)
+    {
+        if (iw == 0) {
+            are[idx] = aim[idx] = 0.0;
+            nf[idx] = phase ? pixel_n(g.ltab[iu], g.mtab[iv]) : 1.0;
+        }
+        if (phase) {
+            double wterm;   // the plane's w as the separate pass forms it
+            {
+#pragma clang fp contract(off)
+                wterm = g.wmin + iw * g.dw;
+            }
+            phase_add_f64(o.x, o.y, wterm, nf[idx], g.dwnorm, are[idx], aim[idx]);
+        } else {
+            are[idx] += o.x;
+            aim[idx] += o.y;
+        }
+        if (iw == g.planes - 1) {
+            const size_t pix = (size_t)iv * g.nx + iu;
+            store_stream(are[idx], &ore[pix]);
+            store_stream(aim[idx], &oim[pix]);
+        }
+    }
+};
+struct GenStore {
+    static constexpr bool kOn = false;
+    static constexpr int kValues = kGenValues;
+};
+
 // One radix-R pass (Stockham: Ns = product of the earlier radices).  The
 // first pass reads global memory, later ones LDS; the last writes global
-// memory.  Reads of a pass all complete (barrier) before its writes, so the
+// memory, or hands its values to the phase sum.  Reads of a pass all complete (barrier) before its writes, so the
 // LDS buffer is used in place.
-template <typename T, int R>
+template <typename T, int R, typename Sink>
 __device__ __forceinline__ void gen_pass(const GenCtx<T> &c, const GenPass &ps, bool first,
-                                         bool last)
+                                         bool last, Sink &sink)
 {
-    constexpr int BPT = gen_bpt(R);
+    constexpr int BPT = gen_bpt(R, Sink::kValues);
     const GenAddr &a = *c.a;
     const int L = c.L, G = a.G, Lr = ps.Lr, Ns = ps.Ns, nb = G * Lr;
     C2<T> v[BPT][R];
@@ -345,6 +388,12 @@ __device__ __forceinline__ void gen_pass(const GenCtx<T> &c, const GenPass &ps, 
             continue;
         }
         if (g >= c.nvalid) continue;   // (its twiddle index would pass the table)
+        if constexpr (Sink::kOn) {
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+                sink.add(v[i][q], i * R + q, c.g0 + g, c.s + (dbase + q * Ns) * sink.row_mul);
+            continue;
+        }
         C2<T> *p = c.out + (size_t)g * a.pg_out + (size_t)dbase * a.pe_out;
         const size_t step = (size_t)Ns * a.pe_out;
         const int e = a.tw_by == 1 ? c.s : c.g0 + g;
@@ -359,6 +408,38 @@ __device__ __forceinline__ void gen_pass(const GenCtx<T> &c, const GenPass &ps, 
     }
     if (!last) __syncthreads();
 }
+
+// All passes of a workgroup's lines.
+template <typename T, bool HARD, typename Sink>
+__device__ __forceinline__ void gen_lines_of(const GenCtx<T> &c, const GenPassDesc &gp, Sink &sink)
+{
+    for (int p = 0; p < gp.np; ++p) {
+        const bool first = p == 0, last = p == gp.np - 1;
+        const GenPass &ps = gp.pass[p];
+        switch (ps.R) {
+            case 10: gen_pass<T, 10>(c, ps, first, last, sink); break;
+            case 9: gen_pass<T, 9>(c, ps, first, last, sink); break;
+            case 8: gen_pass<T, 8>(c, ps, first, last, sink); break;
+            case 7: gen_pass<T, 7>(c, ps, first, last, sink); break;
+            case 6: gen_pass<T, 6>(c, ps, first, last, sink); break;
+            case 5: gen_pass<T, 5>(c, ps, first, last, sink); break;
+            case 4: gen_pass<T, 4>(c, ps, first, last, sink); break;
+            case 3: gen_pass<T, 3>(c, ps, first, last, sink); break;
+            case 2: gen_pass<T, 2>(c, ps, first, last, sink); break;
+            default:
+                if constexpr (!Sink::kOn) {
+                    if (ps.R == 16) gen_pass<T, 16>(c, ps, first, last, sink);
+                    else if (ps.R == 15) gen_pass<T, 15>(c, ps, first, last, sink);
+                    else if (ps.R == 14) gen_pass<T, 14>(c, ps, first, last, sink);
+                    else if (ps.R == 12) gen_pass<T, 12>(c, ps, first, last, sink);
+                }
+                if constexpr (HARD) {
+                    if (ps.R == 11) gen_pass<T, 11>(c, ps, first, last, sink);
+                    else if (ps.R == 13) gen_pass<T, 13>(c, ps, first, last, sink);
+                }
+                break;
+        }
+    }}
 
 // Passes of one workgroup.  A thread holds one butterfly of a radix above 8 (16
 // values at most) or as many smaller ones as make 16 values, so a pass needs no
@@ -417,30 +498,45 @@ k_fft_gen(GenPassDesc gp, GenAddr a, const C2<T> *__restrict__ tw, const C2<T> *
         c.occ = occ;
         __syncthreads();
     }
-    for (int p = 0; p < gp.np; ++p) {
-        const bool first = p == 0, last = p == gp.np - 1;
-        const GenPass &ps = gp.pass[p];
-        switch (ps.R) {
-            case 16: gen_pass<T, 16>(c, ps, first, last); break;
-            case 15: gen_pass<T, 15>(c, ps, first, last); break;
-            case 14: gen_pass<T, 14>(c, ps, first, last); break;
-            case 12: gen_pass<T, 12>(c, ps, first, last); break;
-            case 10: gen_pass<T, 10>(c, ps, first, last); break;
-            case 9: gen_pass<T, 9>(c, ps, first, last); break;
-            case 8: gen_pass<T, 8>(c, ps, first, last); break;
-            case 7: gen_pass<T, 7>(c, ps, first, last); break;
-            case 6: gen_pass<T, 6>(c, ps, first, last); break;
-            case 5: gen_pass<T, 5>(c, ps, first, last); break;
-            case 4: gen_pass<T, 4>(c, ps, first, last); break;
-            case 3: gen_pass<T, 3>(c, ps, first, last); break;
-            case 2: gen_pass<T, 2>(c, ps, first, last); break;
-            default:
-                if constexpr (HARD) {
-                    if (ps.R == 11) gen_pass<T, 11>(c, ps, first, last);
-                    else gen_pass<T, 13>(c, ps, first, last);
-                }
-                break;
-        }
+    GenStore sink;
+    gen_lines_of<T, HARD>(c, gp, sink);
+}
+
+// Last pass of a four-step column axis, the phase correction and the plane sum in
+// one: each plane is read once, and not written and read again.  A thread holds 10
+// values (with 16, and their sums, 776 registers spill), so radices above 10 are not
+// used here.  Bound by the vector units now, half of it the sines, at 2 waves per
+// SIMD: both passes of 8 planes of 3000^2 736 -> 650 us, of 10 of 1920 x 2560 459 ->
+// 370, of 16 of 960 x 3000 473 -> 383, of 30 of 2400 x 1280 793 -> 800.
+__global__ void __launch_bounds__(kGenThreads)
+k_fft_gen_phase(GenPassDesc gp, GenAddr a, const C2<double> *__restrict__ tw,
+                const C2<double> *in, PhaseGeom pg, double *ore, double *oim)
+{
+    extern __shared__ double gen_smem[];
+    const int grp = (int)(blockIdx.x % (unsigned)a.ngroups);
+    const int s = (int)(blockIdx.x / (unsigned)a.ngroups);
+    GenCtx<double> c;
+    c.a = &a;
+    c.tw = tw;
+    c.lds = reinterpret_cast<C2<double> *>(gen_smem);
+    c.L = gp.L;
+    c.s = s;
+    c.g0 = grp * a.G;
+    c.nvalid = min(a.G, a.nl - c.g0);
+    c.in = in + (size_t)s * (size_t)a.ps_in + (size_t)c.g0 * (size_t)a.pg_in;
+    c.out = nullptr;
+    c.scale = 1.0;
+    c.occ = nullptr;
+    c.occ_stride = c.occ_shift = 0;
+    GenPhase sink;
+    sink.g = pg;
+    sink.ore = ore;
+    sink.oim = oim;
+    sink.row_mul = a.sets;
+    sink.phase = pg.phase_on && pg.planes > 1;
+    for (int iw = 0; iw < pg.planes; ++iw, c.in += a.pz) {
+        sink.iw = iw;
+        gen_lines_of<double, false>(c, gp, sink);
     }
 }
 
@@ -510,13 +606,13 @@ void gen_search(int rest, int max_r, std::vector<int> &cur, std::vector<int> &be
         }
 }
 
-bool gen_radices(int L, GenPassDesc &gp)
+bool gen_radices(int L, GenPassDesc &gp, int values = kGenValues)
 {
     gp = GenPassDesc{};
     gp.L = L;
     if (L < 2 || L > kGenElems) return false;
     std::vector<int> cur, best;
-    gen_search(L, kGenValues, cur, best);
+    gen_search(L, values, cur, best);
     if (best.empty() || (int)best.size() > kGenMaxPasses) return false;
     int Ns = 1;
     for (int r : best) {
@@ -532,11 +628,11 @@ bool gen_radices(int L, GenPassDesc &gp)
 }
 
 // Threads that G lines of this plan take (0: more than a workgroup has).
-int gen_threads(const GenPassDesc &gp, int G)
+int gen_threads(const GenPassDesc &gp, int G, int values = kGenValues)
 {
     int need = 1;
     for (int p = 0; p < gp.np; ++p) {
-        const int nb = G * gp.pass[p].Lr, bpt = gen_bpt(gp.pass[p].R);
+        const int nb = G * gp.pass[p].Lr, bpt = gen_bpt(gp.pass[p].R, values);
         need = std::max(need, (nb + bpt - 1) / bpt);
     }
     return need > kGenThreads ? 0 : (need + 63) / 64 * 64;
@@ -544,10 +640,10 @@ int gen_threads(const GenPassDesc &gp, int G)
 
 // Lines per workgroup: as many as the threads and `elems` LDS elements take,
 // whole groups of 8 lines where lines are adjacent in memory (128-byte runs).
-int gen_lines(const GenPassDesc &gp, int nl, int elems, bool adjacent)
+int gen_lines(const GenPassDesc &gp, int nl, int elems, bool adjacent, int values = kGenValues)
 {
     int G = std::max(1, std::min(nl, elems / gp.L));
-    while (G > 1 && !gen_threads(gp, G)) --G;
+    while (G > 1 && !gen_threads(gp, G, values)) --G;
     if (adjacent && G > 8 && G < nl) G = G / 8 * 8;
     return G;
 }
@@ -665,6 +761,38 @@ size_t csize(int precision) { return precision == RICK_FP64 ? 16 : 8; }
 // many bytes in FP32 (longer runs of adjacent columns).
 template <typename T>
 constexpr int gen_elems() { return sizeof(T) == 8 ? 4096 : 8192; }
+
+// Lines of a workgroup of the fused last column pass, or 0 where the pass is not
+// used: it walks the planes one after another, so images that fill the chip less
+// than four times over are faster apart (1000^2 x 8 85 us, fused 111; 1500^2 x 8 197
+// and 189; 2000^2 x 8 331 and 281).  FP32 is too, the plain pass having six waves per
+// SIMD (3000^2 x 8: 375 us, fused 463).
+int gen_phase_lines(const GenPassDesc &gp, int nl, int sets)
+{
+    if (gp.np == 0) return 0;
+    const int G = gen_lines(gp, nl, gen_elems<double>(), true, kPhaseValues);
+    return (long long)((nl + G - 1) / G) * sets >= 1024 ? G : 0;
+}
+
+hipError_t launch_gen_phase(GenPassDesc gp, GenAddr a, int G, const void *tw, long long ntab,
+                            const void *in, const PhaseGeom &pg, double *re, double *im,
+                            hipStream_t s)
+{
+    a.G = G;
+    a.mG = gen_magic((uint32_t)G);
+    a.ngroups = (a.nl + G - 1) / G;
+    const int nt = gen_threads(gp, G, kPhaseValues);
+    const size_t lds = gp.np == 1 ? 0 : (size_t)G * gp.L * sizeof(C2<double>);
+    const unsigned long long blocks = (unsigned long long)a.ngroups * a.sets;
+    if (!nt || blocks > 0x7fffffffull || lds > (size_t)kGenLdsBytes)
+        return hipErrorInvalidConfiguration;
+    for (int p = 0; p < gp.np; ++p)
+        gp.pass[p].tstep = (int)(ntab / ((long long)gp.pass[p].Ns * gp.pass[p].R));
+    hipLaunchKernelGGL(k_fft_gen_phase, dim3((unsigned)blocks), dim3(nt), lds, s, gp, a,
+                       static_cast<const C2<double> *>(tw), static_cast<const C2<double> *>(in),
+                       pg, re, im);
+    return hipGetLastError();
+}
 
 template <typename T>
 hipError_t launch_gen(GenPassDesc gp, GenAddr a, long long planes, const void *tw,
@@ -786,7 +914,7 @@ hipError_t smooth_axis(const GenAxis &ax, const AxisGeom &ag, bool rows, int pla
 template <typename T>
 hipError_t gen_chain(const GenFft &g, int planes, int nx, int ny, void *grid_v, double scale,
                      hipStream_t s, Timing *tm, const GridGeom &geom, const uint32_t *offsets,
-                     const unsigned char *rowlive)
+                     const unsigned char *rowlive, const PhaseGeom &pg, double *re, double *im)
 {
     C2<T> *grid = static_cast<C2<T> *>(grid_v);
     const long long plane = (long long)nx * ny;
@@ -807,12 +935,22 @@ hipError_t gen_chain(const GenFft &g, int planes, int nx, int ny, void *grid_v, 
         e = launch_gen<T>(ay.a, step_a_addr(ay, ag1, false, plane), planes, ay.tw, ny, grid, grid,
                           1.0, s, oc);
     tm->end(RICK_STAGE_FFT_COLS, s);
-    if (e != hipSuccess || ay.mode == 0) return e;
+    if (e != hipSuccess) return e;
+    const int prec = sizeof(T) == 8 ? RICK_FP64 : RICK_FP32;
+    if (ay.mode == 0) return launch_phase(pg, prec, grid, re, im, 0, s, tm);
+    const GenAddr B = step_b_addr(ay, ag1, false, plane, true);
+    const int G = prec == RICK_FP64 ? gen_phase_lines(ay.p, B.nl, B.sets) : 0;
+    if (G) {
+        tm->begin(RICK_STAGE_PHASE, s);
+        e = launch_gen_phase(ay.p, B, G, ay.tw, ny, grid, pg, re, im, s);
+        tm->end(RICK_STAGE_PHASE, s);
+        return e;
+    }
     tm->begin(RICK_STAGE_FFT_COLS_B, s);
-    e = launch_gen<T>(ay.b, step_b_addr(ay, ag1, false, plane, true), planes, ay.tw, ny, grid,
-                      grid, 1.0, s);
+    e = launch_gen<T>(ay.b, B, planes, ay.tw, ny, grid, grid, 1.0, s);
     tm->end(RICK_STAGE_FFT_COLS_B, s);
-    return e;
+    if (e != hipSuccess) return e;
+    return launch_phase(pg, prec, grid, re, im, 0, s, tm, ay.n1, ay.n2);
 }
 
 template <typename T>
@@ -900,6 +1038,7 @@ bool gen_fft_prepare(int nx, int ny, int precision, GenFft *g)
         ax.n = ag.n;
         if (ag.n < 2) return false;
         if (smooth(ag.n) && plan_smooth(ag.n, axis == 0, ax.mode, ax.n1, ax.n2, ax.a, ax.b)) {
+            if (axis == 1 && ax.mode == 1) gen_radices(ax.n2, ax.p, kPhaseValues);
             tables += (cs * (size_t)ag.n + 255) / 256 * 256;
             if (ax.mode == 1) work = std::max(work, cs * (size_t)nx * ny);
             continue;
@@ -991,16 +1130,16 @@ bool gen_chain_ok(const GenFft &g)
 
 hipError_t launch_gen_chain(const GenFft &g, int precision, int planes, int nx, int ny, void *grid,
                             double scale, hipStream_t s, Timing *tm, const GridGeom &geom,
-                            const uint32_t *offsets, const unsigned char *rowlive, int *row_n1,
-                            int *row_n2)
+                            const uint32_t *offsets, const unsigned char *rowlive,
+                            const PhaseGeom &pg, double *re, double *im)
 {
     Timing off;
     if (tm == nullptr) tm = &off;
-    *row_n1 = g.ax[1].mode == 1 ? g.ax[1].n1 : 1;
-    *row_n2 = g.ax[1].mode == 1 ? g.ax[1].n2 : 0;
     if (precision == RICK_FP64)
-        return gen_chain<double>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive);
-    return gen_chain<float>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive);
+        return gen_chain<double>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive, pg,
+                                 re, im);
+    return gen_chain<float>(g, planes, nx, ny, grid, scale, s, tm, geom, offsets, rowlive, pg, re,
+                            im);
 }
 
 hipError_t launch_fft_gen(const GenFft &g, int precision, int planes, int nx, int ny,

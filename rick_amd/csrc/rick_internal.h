@@ -208,6 +208,14 @@ bool fft_needs_tmp(int precision, int ny);
 hipError_t launch_fft(const FftPlan &p, int precision, const void *in, void *out, void *tmp,
                       double scale, hipStream_t s, Timing *tm);
 
+// Phase correction + plane sum.
+struct PhaseGeom {
+    int planes, nx, ny;
+    double wmin, dw, dwnorm;
+    int phase_on;
+    const double *ltab, *mtab;  // device: sin(xcoord*resolution) per u / per v index
+};
+
 // FFT of any axis lengths >= 2 (mixed radix 2..16, 3, 5, 7, 11, 13 in
 // LDS; four-step for long or strided axes; Bluestein for other primes).
 constexpr int kGenMaxPasses = 8;
@@ -225,6 +233,7 @@ struct GenAxis {
     int mode;                       // 0 direct, 1 four-step, 2 Bluestein
     int n1, n2;                     // four-step split n = n1*n2
     GenPassDesc a, b;               // direct: a; four-step: a (n1), b (n2)
+    GenPassDesc p;                  // four-step columns: b of the fused phase pass (np 0: none)
     int m, mmode, m1, m2;           // Bluestein: convolution length and its plan
     GenPassDesc ma, mb;
     const void *tw;                 // device exp(+2 pi i k/n) [n] (Bluestein: [m])
@@ -240,26 +249,19 @@ bool gen_fft_prepare(int nx, int ny, int precision, GenFft *g);
 // Writes the tables (synchronously) at `tables` (table_bytes) and records the
 // scratch `work` (work_bytes).
 hipError_t gen_fft_upload(GenFft *g, int precision, void *tables, void *work);
-// Image-chain transform of a sparse grid in place (axes for which
-// gen_chain_ok): rows without a flag in rowlive are read as zero, tiles by the
-// bucket offsets.  Image row v is then in grid row (v % n1) * n2 + v / n1
-// (*row_n2 == 0: in row v).
+// Image chain after gridding on a sparse grid (axes for which gen_chain_ok), in place:
+// rows without a flag in rowlive are read as zero, tiles by the bucket offsets; then
+// the phase correction and plane sum into re, im, with the last column pass in one
+// where that pays.
 bool gen_chain_ok(const GenFft &g);
 hipError_t launch_gen_chain(const GenFft &g, int precision, int planes, int nx, int ny, void *grid,
                             double scale, hipStream_t s, Timing *tm, const GridGeom &geom,
-                            const uint32_t *offsets, const unsigned char *rowlive, int *row_n1,
-                            int *row_n2);
+                            const uint32_t *offsets, const unsigned char *rowlive,
+                            const PhaseGeom &pg, double *re, double *im);
 // Per-plane backward 2-D transform, in == out allowed, scaled.
 hipError_t launch_fft_gen(const GenFft &g, int precision, int planes, int nx, int ny,
                           const void *in, void *out, double scale, hipStream_t s, Timing *tm);
 
-// Phase correction + plane sum.
-struct PhaseGeom {
-    int planes, nx, ny;
-    double wmin, dw, dwnorm;
-    int phase_on;
-    const double *ltab, *mtab;  // device: sin(xcoord*resolution) per u / per v index
-};
 // With row_n2 > 0 image row v is read from grid row (v % row_n1) * row_n2 + v / row_n1.
 hipError_t launch_phase(const PhaseGeom &p, int precision, const void *gridss, double *re,
                         double *im, int accumulate, hipStream_t s, Timing *tm, int row_n1 = 1,

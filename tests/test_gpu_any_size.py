@@ -152,3 +152,14 @@ def test_wide_column_strips_on_a_sparse_grid(planes):
     got, want = ((a.cpu().numpy() + 1j * b.cpu().numpy()) for a, b in ((re, im), (wre, wim)))
     assert np.isfinite(want).all() and np.abs(want).max() > 0
     assert rel_l2(got, want) <= 1e-5
+
+
+# The last column pass of a four-step axis with and without the phase in it: rows at
+# 1024 workgroups and below, strips that the width does not fill, a single radix, a
+# factor of 11 (never in one).
+@pytest.mark.parametrize("nx,ny,planes", [
+    (1920, 2560, 3), (2000, 2000, 1), (1500, 1500, 2), (4095, 360, 3), (2100, 3300, 2),
+    (3000, 1920, 2)])
+@pytest.mark.parametrize("precision", [FP64, FP32])
+def test_any_size_phase_pass_matches_separate_stages(nx, ny, planes, precision):
+    test_phase_pass_of_every_line_length_matches_stages(nx, ny, planes, precision)
