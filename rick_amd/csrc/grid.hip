@@ -632,9 +632,11 @@ __device__ __forceinline__ void wave_row_sums(uint32_t r0, uint32_t n, uint32_t 
 // (64 bytes of a row per load instruction), and add up their parts at the end.
 // One lane per row made every load instruction touch 64 lines, whose other
 // parts were evicted before their turn: 2.9 M rows of 64 values took 1.88 ms
-// where this takes 0.47 (1.6 GB, 3.4 TB/s), 1.2 M rows of 12 values 134 and 112
+// where this takes 0.42 (1.6 GB, 3.8 TB/s), 1.2 M rows of 12 values 134 and 112
 // us.  `in` has a bit for each row that is to be read; lane l returns the sums of
-// row r0 + l (zero without its bit).
+// row r0 + l (zero without its bit).  With RANK up to 16 such rows are read in one
+// round, whichever they are, else (and with more) 16 neighbours at a time.
+template <bool RANK>
 __device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, unsigned long long in,
                                                       uint32_t n4, uint32_t P,
                                                       const float *__restrict__ vr,
@@ -647,12 +649,23 @@ __device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, unsigned long
     const float4 *i4 = reinterpret_cast<const float4 *>(vi);
     const bool fixed_w = P == 1u || P == 2u || P == 4u;   // element c always weighs w[c % P]
     out_re = out_im = 0.0;
+    const uint32_t count = (uint32_t)__popcll(in);   // uniform
+    const bool few = RANK && count <= 16u;
+    // With few rows: this row's rank among them, and the row that lane / 4 ranks.
+    uint32_t rank = lane, nth = lane / 4u;
+    if (few) {
+        rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((uint32_t)in, 0u));
+        const uint32_t to = (in >> lane) & 1ull ? rank : count + lane - rank;
+        const int order = __builtin_amdgcn_ds_permute((int)(to * 4u), (int)lane);
+        nth = (uint32_t)__shfl(order, (int)(lane / 4u));
+    }
 #pragma unroll 1
-    for (uint32_t j = 0; j < 4; ++j) {
-        if (((in >> (j * 16u)) & 0xffffull) == 0ull) continue;   // uniform
-        const uint32_t row = r0 + j * 16u + lane / 4u;
+    for (uint32_t j = 0; j < (few ? 1u : 4u); ++j) {
+        if (!few && ((in >> (j * 16u)) & 0xffffull) == 0ull) continue;   // uniform
+        const uint32_t row = r0 + j * 16u + nth;
         double a_re = 0.0, a_im = 0.0;
-        if ((in >> (j * 16u + lane / 4u)) & 1ull) {
+        if ((in >> (j * 16u + nth)) & 1ull) {
             const float *wrow = wt + (size_t)row * P;
             const size_t e0 = (size_t)row * n4;
             float w[4];
@@ -681,10 +694,10 @@ __device__ __forceinline__ void wave_row_sums_strided(uint32_t r0, unsigned long
         a_im += __shfl_xor(a_im, 1);
         a_re += __shfl_xor(a_re, 2);
         a_im += __shfl_xor(a_im, 2);
-        // Row j*16 + m is in lanes 4m .. 4m+3.
-        const int src = (int)(lane & 15u) * 4;
+        // Row j*16 + m (the row of rank m) is in lanes 4m .. 4m+3.
+        const int src = (int)(rank & 15u) * 4;
         const double t_re = __shfl(a_re, src), t_im = __shfl(a_im, src);
-        if (lane / 16u == j) {
+        if (few ? (in >> lane) & 1ull : lane / 16u == j) {
             out_re = t_re;
             out_im = t_im;
         }
@@ -718,10 +731,13 @@ __device__ __forceinline__ void zero_split_tiles(const GridGeom &g, uint32_t fir
 
 // VMODE: 0 = per-row scalar reads, 1 = one 16-byte read per row (F*P = 4),
 // 2 or 4 = wave-cooperative reads with VMODE lanes per row (F*P = 8 or 16),
-// 3 = wave-cooperative reads of any larger multiple of 4; the 16-byte modes need
-// 16-byte aligned visibility arrays.
+// 3 or 5 = wave-cooperative reads of any larger multiple of 4, 5 (from 24 values on)
+// ranking a wave's few rows inside the grid and with the registers of one workgroup
+// per CU; the 16-byte modes need 16-byte aligned visibility arrays.  3 and 5: 2.9 M
+// rows of 64 values 474 and 420 us, 2.8 M rows of 24 values, 84 % outside the grid,
+// 51 and 37; 1.2 M rows of 12 values, one round of loads a row, 47 and 55.
 template <int PREC, int VMODE, bool BATCH>
-__global__ void __launch_bounds__(kScatterThreads, 8)
+__global__ void __launch_bounds__(kScatterThreads, VMODE == 5 ? 4 : 8)
 k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__restrict__ uu_all,
           const double *__restrict__ vv_all, const double *__restrict__ ww_all,
           const float *__restrict__ vr_all, const float *__restrict__ vi_all,
@@ -754,7 +770,7 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
     constexpr bool vec4 = VMODE == 1;
     const uint32_t FP = F * P;
     double w_re[kRowsPerThread] = {}, w_im[kRowsPerThread] = {};
-    if constexpr (VMODE == 3) {
+    if constexpr (VMODE == 3 || VMODE == 5) {
         // The sums first, over the rows that fall into the grid; coordinates are
         // loaded once more below, from the cache: held over the sums they cost
         // more in spilled registers (112 -> 140 us on 1.2 M rows of 12 values).
@@ -771,8 +787,9 @@ k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__re
         }
 #pragma unroll
         for (int k = 0; k < kRowsPerThread; ++k)
-            wave_row_sums_strided(base + k * kScatterThreads + threadIdx.x - (threadIdx.x & 63u),
-                                  in[k], FP / 4u, P, vr, vi, wt, w_re[k], w_im[k]);
+            wave_row_sums_strided<VMODE == 5>(
+                base + k * kScatterThreads + threadIdx.x - (threadIdx.x & 63u), in[k], FP / 4u, P,
+                vr, vi, wt, w_re[k], w_im[k]);
     }
     // Every coordinate of the thread's rows (and, with one value per row,
     // its visibility and weight) is requested before any is used, so the
@@ -1819,7 +1836,7 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
         const bool vec4 = (FP % 4u) == 0u &&
                           ((reinterpret_cast<uintptr_t>(vr) | reinterpret_cast<uintptr_t>(vi)) &
                            15u) == 0u;   // batch: vr = vi = null, the caller checked the jobs
-        const int mode = !vec4 ? 0 : FP == 4u ? 1 : FP == 8u ? 2 : FP == 16u ? 4 : 3;
+        const int mode = !vec4 ? 0 : FP == 4u ? 1 : FP == 8u ? 2 : FP == 16u ? 4 : FP < 24u ? 3 : 5;
         // Overwritten grids: the split buckets' tiles start at zero (FP32: for
         // the non-finite fallback; its finite sums go through integer tiles).
         const uint32_t zblk = accumulate ? 0u : std::min(w.split_cap, kZeroBlocks);
@@ -1835,6 +1852,7 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
         RICK_SCATTER_LAUNCH(PR, VM, false)
 #define RICK_SCATTER_MODES(PR)                                                                \
     switch (mode) {                                                                           \
+    case 5: RICK_SCATTER(PR, 5); break;                                                       \
     case 4: RICK_SCATTER(PR, 4); break;                                                       \
     case 3: RICK_SCATTER(PR, 3); break;                                                       \
     case 2: RICK_SCATTER(PR, 2); break;                                                       \

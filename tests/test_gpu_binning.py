@@ -71,3 +71,26 @@ def test_wide_rows_match_oracle(F, P, shift, n):
                     on_gpu(vi), torch.from_numpy(wt).to("cuda"), F, P).cpu().numpy()
     assert np.isfinite(got).all()
     assert rel_l2(got, ref) <= 1e-12
+
+
+# Waves of which no row, few (to 16, ranked and read at once) or more lie in the grid.
+@pytest.mark.parametrize("F,P", [(5, 4), (6, 4), (12, 3), (64, 1)])
+@pytest.mark.parametrize("inside", [0, 1, 15, 16, 17, 40])
+def test_wide_rows_mostly_outside_match_oracle(F, P, inside):
+    nx, planes, n = 256, 4, 2500
+    print(f"case wide rows F={F} P={P} inside={inside}", flush=True)
+    rng = np.random.default_rng(F * 100 + P + inside)
+    uu, vv, ww = (rng.uniform(0.0, 1.0, n) for _ in range(3))
+    for w0 in range(0, n, 64):      # `inside` rows of every wave, and all of the last part's
+        out = rng.permutation(64)[inside:] + w0
+        vv[out[out < n - 30]] += 1.5
+    vr, vi = (rng.normal(size=n * F * P).astype(np.float32) for _ in range(2))
+    vr[1::29] = np.nan
+    wt = rng.uniform(0.5, 1.5, n * P).astype(np.float32)
+    ref = O.wstack(O.KAISERBESSEL, planes, uu, vv, ww, vr, vi, wt, F, P, 1.0 / nx, 1.0 / planes,
+                   7, nx, nx, threads=8)
+    plan = Plan(nx, nx, planes, kernel=rick_amd.KAISERBESSEL, support=7, max_points=n)
+    got = plan.grid(*[torch.from_numpy(a).to("cuda") for a in (uu, vv, ww, vr, vi, wt)], F,
+                    P).cpu().numpy()
+    assert np.isfinite(got).all()
+    assert rel_l2(got, ref) <= 1e-12
