@@ -828,8 +828,12 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
         RICK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         c.staged.push_back(e);
     }
-    // Pieces below `open` may be worked on; `done` counts finished parts of pieces.
-    std::atomic<size_t> open{how == Copy::to_device ? kPieces : 0}, done{0};
+    // Pieces below `open` may be worked on; done[i] counts the finished parts of piece
+    // i (a count over all pieces would let a thread that is ahead stand in for one
+    // that has not started).
+    std::atomic<size_t> open{how == Copy::to_device ? kPieces : 0};
+    std::vector<std::atomic<int>> done(n);
+    for (auto &d : done) d.store(0, std::memory_order_relaxed);
     std::atomic<int> team{1};       // threads at work, final before `start`
     std::atomic<bool> start{false}, stop{false};
     auto part = [&](size_t i, int t, int nt) {
@@ -846,7 +850,7 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             const double *src = reinterpret_cast<const double *>(buf + a);
             for (size_t q = 0; q < (b - a) / sizeof(double); ++q) dst[q] += src[q];
         }
-        done.fetch_add(1, std::memory_order_release);
+        done[i].fetch_add(1, std::memory_order_release);
     };
     auto helper = [&](int t) {
         while (!start.load(std::memory_order_acquire)) std::this_thread::yield();
@@ -880,7 +884,7 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
         return e != hipSuccess ? e : hipEventRecord(c.staged[i % kPieces], c.stream);
     };
     auto all_done = [&](size_t i) {
-        while (done.load(std::memory_order_acquire) < (i + 1) * nt) std::this_thread::yield();
+        while (done[i].load(std::memory_order_acquire) < nt) std::this_thread::yield();
     };
     hipError_t e = hipSuccess;
     if (how != Copy::to_device)
