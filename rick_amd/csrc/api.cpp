@@ -94,22 +94,27 @@ TileShape default_tile(const rick_plan_desc &d)
     return nb <= 1024 && fits ? TileShape{64, 32} : TileShape{64, 64};
 }
 
-// Built-in records per task: the power of two from the share of one of 192
-// workgroups up where the tile kernel takes full tasks by footprint class, whose
-// fixed cost wants long tasks, and of 512 (two per CU) where it does not.
-// Shorter tasks split more buckets, whose parts meet in atomics; longer ones
-// leave the last workgroups running alone.  Image by records per task: 516 k rows
-// on 512^2 x 8 FP64 137 us at 1024, 119 at 4096, 143 at 8192; 1 M rows on 1024^2
-// x 16 464 us at 2048, 444 at 8192, 482 at 16384; 3 M rows on 2048^2 x 12 FP32 861
-// us at 2048, 802 at 8192; dense FP32 gridding of 7.7 M rows 1.36 ms at 4096, 1.27
-// at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us at 512,
-// 98 at 4096.
+// Built-in records per task: the power of two from the share of one of 512
+// workgroups up (two per CU).  Where the tile kernel takes full tasks by footprint
+// class, whose fixed cost wants long tasks, from the share of one of 192, but over
+// 8192 no longer than the first: a hot tile's tasks would outlast all others (2.8 M
+// rows about the centre of 1024^2 x 23 FP32: tile kernel 170 us at 4096, 145 at 8192,
+// 297 at 16384).  Shorter tasks split more buckets, whose parts meet in atomics;
+// longer ones leave the last workgroups running alone.  Image by records per task:
+// 516 k rows on 512^2 x 8 FP64 137 us at 1024, 119 at 4096, 143 at 8192; 1 M rows on
+// 1024^2 x 16 464 us at 2048, 444 at 8192, 482 at 16384; 3 M rows on 2048^2 x 12 FP32
+// 833 us at 2048, 780 at 8192 and 16384; dense FP32 gridding of 7.7 M rows 1.36 ms at
+// 4096, 1.27 at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us
+// at 512, 98 at 4096.
 uint32_t default_rows_per_task(const rick_plan_desc &d, int tu, int tv, int smax)
 {
-    const uint32_t share = d.max_points / (tile_by_class(d, tu, tv, smax) ? 192u : 512u);
-    uint32_t r = 512;
-    while (r < 16384 && r < share) r *= 2;
-    return r;
+    auto from = [](uint32_t share, uint32_t most) {
+        uint32_t r = 512;
+        while (r < most && r < share) r *= 2;
+        return r;
+    };
+    const uint32_t r = from(d.max_points / 512u, 16384);
+    return tile_by_class(d, tu, tv, smax) ? std::max(r, from(d.max_points / 192u, 8192)) : r;
 }
 
 }  // namespace
