@@ -741,7 +741,8 @@ struct Ctx {
 constexpr size_t kPiece = 4ull << 20;   // bytes of a staging piece
 constexpr size_t kPieces = 4;           // pieces in flight
 constexpr size_t kCopyShare = 256 << 10;   // least bytes of a copy per thread
-constexpr int kCopyThreads = 8;         // most threads of one copy
+constexpr int kCopyThreads = 8;         // most threads of a copy below kManyThreads
+constexpr size_t kManyThreads = 256ull << 20;   // bytes from which it may be twice as many
 
 Ctx *context_for(int rank)
 {
@@ -805,7 +806,8 @@ enum class Copy { to_device, to_host, add_to_host };
 // device and 64 MB pieces back: wstack() 2.86 / 2.02 / 1.87 -> 2.37 / 1.39 / 1.43
 // ms with 1 / 4 / 8 threads, phase_correction() 1.50 / 1.39 / 1.56 -> 1.50 / 0.96
 // / 1.01, rick_fft_planes() 3.21 -> 1.74; more than 8 threads cost more to start
-// than they add (16: 1.60 and 1.18 ms).
+// than they add (16: 1.60 and 1.18 ms), except in copies of gigabytes (wstack() into a
+// grid of 8.6 GB: 214 ms with 8, 209 with 16; 64 MB pieces took 197).
 int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthreads)
 {
     std::vector<HostCopy> pieces;
@@ -868,7 +870,8 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             part(i, t, nt);
         }
     };
-    const int want = (int)std::min<size_t>(std::max(1, std::min(nthreads, kCopyThreads)),
+    const int most = total >= kManyThreads ? 2 * kCopyThreads : kCopyThreads;
+    const int want = (int)std::min<size_t>(std::max(1, std::min(nthreads, most)),
                                            std::max<size_t>(1, total / kCopyShare));
     std::vector<std::thread> th;
     try {
