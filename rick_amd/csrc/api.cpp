@@ -735,14 +735,17 @@ struct Ctx {
     DevBuf in, grid, out, img;
     // Staging between host arrays and the device: pinned pieces and their events.
     char *pinned = nullptr;
+    size_t pinned_bytes = 0;
     std::vector<hipEvent_t> staged;
 };
 
 constexpr size_t kPiece = 4ull << 20;   // bytes of a staging piece
 constexpr size_t kPieces = 4;           // pieces in flight
 constexpr size_t kCopyShare = 256 << 10;   // least bytes of a copy per thread
-constexpr int kCopyThreads = 8;         // most threads of a copy below kManyThreads
-constexpr size_t kManyThreads = 256ull << 20;   // bytes from which it may be twice as many
+constexpr int kCopyThreads = 8;         // most threads of a copy below kLarge
+// Copies of kLarge bytes and more take twice as many threads and pieces four times
+// as long.
+constexpr size_t kLarge = 256ull << 20;
 
 Ctx *context_for(int rank)
 {
@@ -806,17 +809,18 @@ enum class Copy { to_device, to_host, add_to_host };
 // device and 64 MB pieces back: wstack() 2.86 / 2.02 / 1.87 -> 2.37 / 1.39 / 1.43
 // ms with 1 / 4 / 8 threads, phase_correction() 1.50 / 1.39 / 1.56 -> 1.50 / 0.96
 // / 1.01, rick_fft_planes() 3.21 -> 1.74; more than 8 threads cost more to start
-// than they add (16: 1.60 and 1.18 ms), except in copies of gigabytes (wstack() into a
-// grid of 8.6 GB: 214 ms with 8, 209 with 16; 64 MB pieces took 197).
+// than they add (16: 1.60 and 1.18 ms).  Large copies hide that, and want longer
+// pieces: wstack() into a grid of 8.6 GB 214 ms with 8 threads, 209 with 16, 193 with
+// those and 16 MB pieces.
 int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthreads)
 {
     std::vector<HostCopy> pieces;
     size_t total = 0;
-    for (const HostCopy &a : arrays) {
-        for (size_t o = 0; o < a.bytes; o += kPiece)
-            pieces.push_back(HostCopy{a.dev + o, a.host + o, std::min(kPiece, a.bytes - o)});
-        total += a.bytes;
-    }
+    for (const HostCopy &a : arrays) total += a.bytes;
+    const size_t piece = total >= kLarge ? 4 * kPiece : kPiece;
+    for (const HostCopy &a : arrays)
+        for (size_t o = 0; o < a.bytes; o += piece)
+            pieces.push_back(HostCopy{a.dev + o, a.host + o, std::min(piece, a.bytes - o)});
     const size_t n = pieces.size();
     if (how == Copy::to_device && nthreads <= 1) {
         // One thread: the runtime's own copies of pageable memory are as fast.
@@ -824,11 +828,18 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             RICK_HIP(hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c.stream));
         return RICK_OK;
     }
-    if (!c.pinned) {
+    if (c.pinned_bytes < piece * kPieces) {
+        if (c.pinned) {
+            RICK_HIP(hipStreamSynchronize(c.stream));   // its pieces may be under way
+            (void)hipHostFree(c.pinned);
+            c.pinned = nullptr;
+            c.pinned_bytes = 0;
+        }
         void *p = nullptr;
-        if (hipHostMalloc(&p, kPiece * kPieces, hipHostMallocDefault) != hipSuccess)
-            return set_error(RICK_ERR_NOMEM, "hipHostMalloc(%zu) failed", kPiece * kPieces);
+        if (hipHostMalloc(&p, piece * kPieces, hipHostMallocDefault) != hipSuccess)
+            return set_error(RICK_ERR_NOMEM, "hipHostMalloc(%zu) failed", piece * kPieces);
         c.pinned = static_cast<char *>(p);
+        c.pinned_bytes = piece * kPieces;
     }
     while (c.staged.size() < kPieces) {
         hipEvent_t e = nullptr;
@@ -847,7 +858,7 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
         const HostCopy &p = pieces[i];
         const size_t per = ((p.bytes + nt - 1) / nt + 63) / 64 * 64;
         const size_t a = std::min(p.bytes, per * t), b = std::min(p.bytes, a + per);
-        char *buf = c.pinned + (i % kPieces) * kPiece;
+        char *buf = c.pinned + (i % kPieces) * piece;
         if (how == Copy::to_device) {
             memcpy(buf + a, p.host + a, b - a);
         } else if (how == Copy::to_host) {
@@ -870,7 +881,7 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             part(i, t, nt);
         }
     };
-    const int most = total >= kManyThreads ? 2 * kCopyThreads : kCopyThreads;
+    const int most = total >= kLarge ? 2 * kCopyThreads : kCopyThreads;
     const int want = (int)std::min<size_t>(std::max(1, std::min(nthreads, most)),
                                            std::max<size_t>(1, total / kCopyShare));
     std::vector<std::thread> th;
@@ -884,7 +895,7 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
     start.store(true, std::memory_order_release);
     auto queue = [&](size_t i) {
         const HostCopy &p = pieces[i];
-        char *buf = c.pinned + (i % kPieces) * kPiece;
+        char *buf = c.pinned + (i % kPieces) * piece;
         const hipError_t e =
             how == Copy::to_device
                 ? hipMemcpyAsync(p.dev, buf, p.bytes, hipMemcpyHostToDevice, c.stream)
