@@ -467,6 +467,15 @@ def copy_bandwidth(torch, gib=1, reps=5):
     return 2 * (gib << 30) / ms / 1e6
 
 
+def launch_shapes(grid_desc, image_desc, rows):
+    """The launch shapes of the two plans as they run, built-in choices included."""
+    from rick_amd.imaging import describe
+    g, i = describe(grid_desc, rows), describe(image_desc, rows)
+    return {"tile": list(g["tile"]), "rows_per_task": g["rows_per_task"],
+            "footprint_unroll": g["unroll"], "image_tile": list(i["tile"]),
+            "image_rows_per_task": i["rows_per_task"]}
+
+
 def _cpu_model():
     try:
         for line in open("/proc/cpuinfo"):
@@ -529,11 +538,7 @@ def main():
                      "stages": stages, "image_stages": istages, "grid_stats": stats,
                      "img": img,
                      "grid_bytes": plan.grid_bytes,
-                     "tile": [plan.desc.tile_u or 64, plan.desc.tile_v or 64],
-                     "rows_per_task": plan.desc.rows_per_task or 4096,
-                     "footprint_unroll": plan.desc.footprint_unroll or None,
-                     "image_tile": [iplan.desc.tile_u or 64, iplan.desc.tile_v or 64],
-                     "image_rows_per_task": iplan.desc.rows_per_task or 4096}
+                     **launch_shapes(plan.desc, iplan.desc, cfg.n_rows)}
         log(f"{name}: grid {gms:.3f} ms ({vis / gms / 1e6:.3f} Gvis/s), image {ims:.3f} ms")
         del plan, iplan
         torch.cuda.empty_cache()

@@ -137,6 +137,18 @@ typedef struct {
 
 int rick_plan_create(rick_plan *plan, const rick_plan_desc *desc);
 int rick_plan_destroy(rick_plan plan);
+/* What a plan of this description holds and how a call of num_points rows
+ * (<= max_points) is launched, the built-in choices filled in; needs no device.
+ * Fails as rick_plan_create() would for the same description. */
+typedef struct {
+    int tile_u, tile_v;
+    int rows_per_task;      /* records per gridding task */
+    int footprint_unroll;
+    size_t device_bytes;    /* rick_plan_device_bytes() of the plan */
+} rick_plan_shape;
+int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points,
+                       rick_plan_shape *shape);
+
 /* Device bytes held by the plan (tables + gridding workspace). */
 size_t rick_plan_device_bytes(rick_plan plan);
 /* Bytes of one grid (2*planes*Nx*Ny elements of the plan's precision). */

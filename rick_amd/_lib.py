@@ -34,6 +34,12 @@ class PlanDesc(ctypes.Structure):
     ]
 
 
+class PlanShape(ctypes.Structure):
+    """rick_plan_shape (include/rick.h)."""
+    _fields_ = [("tile_u", _c_int), ("tile_v", _c_int), ("rows_per_task", _c_int),
+                ("footprint_unroll", _c_int), ("device_bytes", _c_size)]
+
+
 class BinmsMeta(ctypes.Structure):
     """rick_binms_meta (include/rick.h): the twelve parsed values of meta.txt."""
     _fields_ = [
@@ -84,6 +90,7 @@ SIGNATURES = {
     "rick_device_count": (_c_int, []),
     "rick_version": (ctypes.c_char_p, []),
     "rick_plan_create": (_c_int, [ctypes.POINTER(_vp), ctypes.POINTER(PlanDesc)]),
+    "rick_plan_describe": (_c_int, [ctypes.POINTER(PlanDesc), _c_uint, ctypes.POINTER(PlanShape)]),
     "rick_plan_destroy": (_c_int, [_vp]),
     "rick_plan_device_bytes": (_c_size, [_vp]),
     "rick_plan_grid_bytes": (_c_size, [_vp]),

@@ -136,6 +136,125 @@ struct rick_plan_s {
     Timing timing;
 };
 
+namespace {
+
+// Checks a description and derives its gridding geometry and launch shape.
+int plan_geometry(const rick_plan_desc &d, GridGeom &g)
+{
+    if (d.num_w_planes < 1 || d.grid_size_x < 1 || d.grid_size_y < 1)
+        return set_error(RICK_ERR_INVALID, "bad grid %d x %d x %d planes", d.grid_size_x,
+                         d.grid_size_y, d.num_w_planes);
+    if (d.kernel < RICK_GAUSS || d.kernel > RICK_GAUSS_HI_PRECISION)
+        return set_error(RICK_ERR_INVALID, "unknown kernel kind %d", d.kernel);
+    if (d.w_support < 1 || d.w_support > kMaxSupport || (d.w_support % 2) == 0)
+        return set_error(RICK_ERR_INVALID, "w_support must be odd and in [1, %d], got %d",
+                         kMaxSupport, d.w_support);
+    if (d.precision != RICK_FP64 && d.precision != RICK_FP32)
+        return set_error(RICK_ERR_INVALID, "unknown precision %d", d.precision);
+    if (!(d.dx > 0.0) || !(d.dw > 0.0))
+        return set_error(RICK_ERR_INVALID, "dx and dw must be positive");
+    if (d.xaxistot < 0 || d.yaxistot < 0)
+        return set_error(RICK_ERR_INVALID, "negative image totals %d x %d", d.xaxistot,
+                         d.yaxistot);
+
+    int tu = d.tile_u ? d.tile_u : 64, tv = d.tile_v ? d.tile_v : 64;
+    if (!d.tile_u && !d.tile_v) {
+        const TileShape t = default_tile(d);
+        tu = t.tu;
+        tv = t.tv;
+    }
+    bool tile_ok = false;
+    for (const auto &t : kTiles) tile_ok |= (t.tu == tu && t.tv == tv);
+    if (!tile_ok) return set_error(RICK_ERR_INVALID, "unsupported tile %d x %d", tu, tv);
+    if (tu < d.w_support || tv < d.w_support)
+        return set_error(RICK_ERR_INVALID, "tile %d x %d smaller than support %d", tu, tv,
+                         d.w_support);
+    g.planes = d.num_w_planes;
+    g.nx = d.grid_size_x;
+    g.ny = d.grid_size_y;
+    g.support = d.w_support;
+    g.kl = (d.w_support - 1) / 2;
+    g.kind = d.kernel;
+    g.dx = d.dx;
+    g.dw = d.dw;
+    g.inv_dx = exact_inverse(d.dx);
+    g.inv_dw = exact_inverse(d.dw);
+    g.tu = tu;
+    g.tv = tv;
+    g.tu_shift = __builtin_ctz((unsigned)tu);
+    g.tv_shift = __builtin_ctz((unsigned)tv);
+    g.tiles_u = (g.nx + tu - 1) / tu;
+    g.tiles_v = (g.ny + tv - 1) / tv;
+    const uint64_t nb = (uint64_t)g.planes * g.tiles_u * g.tiles_v;
+    if (nb >= (1ull << 31)) return set_error(RICK_ERR_INVALID, "too many grid tiles");
+    g.nb = (uint32_t)nb;
+    g.cshift = counter_shift(g.nb);
+    g.ntable = kTableOversample * d.w_support;
+    // ~64-128 KB of grid per zero task measured best (LOFAR-like grid).
+    g.zrun = d.precision == RICK_FP64 ? 2 : 4;
+    // Unrolled footprint loops of the tile kernel: the instantiated lengths.
+    {
+        const int unrolls[] = {7, 9, 11, 15};
+        g.smax = 0;
+        for (int u : unrolls)
+            if (u >= d.w_support && (d.footprint_unroll == 0 ? g.smax == 0 : u == d.footprint_unroll))
+                g.smax = u;
+        if (g.smax == 0)
+            return set_error(RICK_ERR_INVALID,
+                             "footprint_unroll %d: must be 0 or one of 7, 9, 11, 15 and >= "
+                             "w_support %d", d.footprint_unroll, d.w_support);
+    }
+    g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
+                                 : default_rows_per_task(d, tu, tv, g.smax);
+    if ((uint64_t)d.max_points * 4ull >= (1ull << 32))
+        return set_error(RICK_ERR_INVALID, "max_points %u too large (limit 2^30)", d.max_points);
+
+    if (d.max_points > 0) {
+        if (const char *why = grid_launch_limit(g, d.max_points))
+            return set_error(RICK_ERR_INVALID, "%d x %d x %d grid, %d x %d tiles, %u points: %s",
+                             g.nx, g.ny, g.planes, tu, tv, d.max_points, why);
+    }
+    return RICK_OK;
+}
+
+// Device memory of a plan: [table | twiddles x | twiddles y | l table | m table |
+// tmp plane | any-size tables and scratch | gridding workspace].
+struct PlanLayout {
+    bool fft_ok = false, gen_ok = false, grid_ok = false;
+    GenFft gen{};
+    size_t table = 0, twx = 0, twy = 0, l = 0, m = 0, tmp = 0, gen_tab = 0, gen_work = 0, work = 0,
+           bytes = 0;
+};
+PlanLayout plan_layout(const rick_plan_desc &d, const GridGeom &g)
+{
+    PlanLayout L;
+    L.grid_ok = d.max_points > 0;
+    L.fft_ok = is_pow2(g.nx) && is_pow2(g.ny) && g.nx >= 16 && g.ny >= 16 && g.nx <= 8192 &&
+               g.ny <= 8192;
+    if (!L.fft_ok) L.gen_ok = gen_fft_prepare(g.nx, g.ny, d.precision, &L.gen);
+    const size_t csz = d.precision == RICK_FP64 ? 16 : 8;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    L.table = take(sizeof(double) * kMaxTable);
+    L.twx = take(csz * (size_t)g.nx);
+    L.twy = take(csz * (size_t)g.ny);
+    L.l = take(sizeof(double) * (size_t)g.nx);
+    L.m = take(sizeof(double) * (size_t)g.ny);
+    L.tmp = take(L.fft_ok && fft_needs_tmp(d.precision, g.ny) ? csz * (size_t)g.nx * g.ny : 0);
+    L.gen_tab = take(L.gen_ok ? L.gen.table_bytes : 0);
+    L.gen_work = take(L.gen_ok ? L.gen.work_bytes : 0);
+    L.work = off;
+    if (L.grid_ok) off += grid_work_bytes(g, d.max_points, d.precision);
+    L.bytes = off;
+    return L;
+}
+
+}  // namespace
+
 extern "C" {
 
 int rick_last_status(void) { return g_status; }
@@ -189,122 +308,33 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
     if (!out || !desc) return set_error(RICK_ERR_INVALID, "null plan or descriptor");
     *out = nullptr;
     const rick_plan_desc &d = *desc;
-    if (d.num_w_planes < 1 || d.grid_size_x < 1 || d.grid_size_y < 1)
-        return set_error(RICK_ERR_INVALID, "bad grid %d x %d x %d planes", d.grid_size_x,
-                         d.grid_size_y, d.num_w_planes);
-    if (d.kernel < RICK_GAUSS || d.kernel > RICK_GAUSS_HI_PRECISION)
-        return set_error(RICK_ERR_INVALID, "unknown kernel kind %d", d.kernel);
-    if (d.w_support < 1 || d.w_support > kMaxSupport || (d.w_support % 2) == 0)
-        return set_error(RICK_ERR_INVALID, "w_support must be odd and in [1, %d], got %d",
-                         kMaxSupport, d.w_support);
-    if (d.precision != RICK_FP64 && d.precision != RICK_FP32)
-        return set_error(RICK_ERR_INVALID, "unknown precision %d", d.precision);
-    if (!(d.dx > 0.0) || !(d.dw > 0.0))
-        return set_error(RICK_ERR_INVALID, "dx and dw must be positive");
-    if (d.xaxistot < 0 || d.yaxistot < 0)
-        return set_error(RICK_ERR_INVALID, "negative image totals %d x %d", d.xaxistot,
-                         d.yaxistot);
-
     auto p = std::make_unique<rick_plan_s>();
     p->d = d;
-    int tu = d.tile_u ? d.tile_u : 64, tv = d.tile_v ? d.tile_v : 64;
-    if (!d.tile_u && !d.tile_v) {
-        const TileShape t = default_tile(d);
-        tu = t.tu;
-        tv = t.tv;
-    }
-    bool tile_ok = false;
-    for (const auto &t : kTiles) tile_ok |= (t.tu == tu && t.tv == tv);
-    if (!tile_ok) return set_error(RICK_ERR_INVALID, "unsupported tile %d x %d", tu, tv);
-    if (tu < d.w_support || tv < d.w_support)
-        return set_error(RICK_ERR_INVALID, "tile %d x %d smaller than support %d", tu, tv,
-                         d.w_support);
     GridGeom &g = p->geom;
-    g.planes = d.num_w_planes;
-    g.nx = d.grid_size_x;
-    g.ny = d.grid_size_y;
-    g.support = d.w_support;
-    g.kl = (d.w_support - 1) / 2;
-    g.kind = d.kernel;
-    g.dx = d.dx;
-    g.dw = d.dw;
-    g.inv_dx = exact_inverse(d.dx);
-    g.inv_dw = exact_inverse(d.dw);
-    g.tu = tu;
-    g.tv = tv;
-    g.tu_shift = __builtin_ctz((unsigned)tu);
-    g.tv_shift = __builtin_ctz((unsigned)tv);
-    g.tiles_u = (g.nx + tu - 1) / tu;
-    g.tiles_v = (g.ny + tv - 1) / tv;
-    const uint64_t nb = (uint64_t)g.planes * g.tiles_u * g.tiles_v;
-    if (nb >= (1ull << 31)) return set_error(RICK_ERR_INVALID, "too many grid tiles");
-    g.nb = (uint32_t)nb;
-    g.cshift = counter_shift(g.nb);
-    g.ntable = kTableOversample * d.w_support;
-    // ~64-128 KB of grid per zero task measured best (LOFAR-like grid).
-    g.zrun = d.precision == RICK_FP64 ? 2 : 4;
-    // Unrolled footprint loops of the tile kernel: the instantiated lengths.
-    {
-        const int unrolls[] = {7, 9, 11, 15};
-        g.smax = 0;
-        for (int u : unrolls)
-            if (u >= d.w_support && (d.footprint_unroll == 0 ? g.smax == 0 : u == d.footprint_unroll))
-                g.smax = u;
-        if (g.smax == 0)
-            return set_error(RICK_ERR_INVALID,
-                             "footprint_unroll %d: must be 0 or one of 7, 9, 11, 15 and >= "
-                             "w_support %d", d.footprint_unroll, d.w_support);
-    }
-    g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
-                                 : default_rows_per_task(d, tu, tv, g.smax);
-    if ((uint64_t)d.max_points * 4ull >= (1ull << 32))
-        return set_error(RICK_ERR_INVALID, "max_points %u too large (limit 2^30)", d.max_points);
-
-    p->grid_ok = d.max_points > 0;
-    if (p->grid_ok) {
-        if (const char *why = grid_launch_limit(g, d.max_points))
-            return set_error(RICK_ERR_INVALID, "%d x %d x %d grid, %d x %d tiles, %u points: %s",
-                             g.nx, g.ny, g.planes, tu, tv, d.max_points, why);
-    }
-    p->fft_ok = is_pow2(g.nx) && is_pow2(g.ny) && g.nx >= 16 && g.ny >= 16 && g.nx <= 8192 &&
-                g.ny <= 8192;
-    if (!p->fft_ok) p->gen_ok = gen_fft_prepare(g.nx, g.ny, d.precision, &p->gen);
-
-    // Device memory: [table | twiddles x | twiddles y | l table | m table |
-    //                 tmp plane | gridding workspace].
-    const size_t csz = d.precision == RICK_FP64 ? 16 : 8;
-    auto al = [](size_t x) { return (x + 255) / 256 * 256; };
-    size_t off = 0;
-    const size_t o_table = off; off += al(sizeof(double) * kMaxTable);
-    const size_t o_twx = off; off += al(csz * (size_t)g.nx);
-    const size_t o_twy = off; off += al(csz * (size_t)g.ny);
-    const size_t o_l = off; off += al(sizeof(double) * (size_t)g.nx);
-    const size_t o_m = off; off += al(sizeof(double) * (size_t)g.ny);
-    const size_t o_tmp = off;
-    if (p->fft_ok && fft_needs_tmp(d.precision, g.ny)) off += al(csz * (size_t)g.nx * g.ny);
-    const size_t o_gen_tab = off;
-    if (p->gen_ok) off += al(p->gen.table_bytes);
-    const size_t o_gen_work = off;
-    if (p->gen_ok) off += al(p->gen.work_bytes);
-    const size_t o_work = off;
-    if (p->grid_ok) off += grid_work_bytes(g, d.max_points, d.precision);
+    const int st = plan_geometry(d, g);
+    if (st != RICK_OK) return st;
+    const PlanLayout L = plan_layout(d, g);
+    p->grid_ok = L.grid_ok;
+    p->fft_ok = L.fft_ok;
+    p->gen_ok = L.gen_ok;
+    p->gen = L.gen;
 
     int prev = 0;
     hipGetDevice(&prev);
     RICK_HIP(hipSetDevice(d.device));
-    hipError_t e = hipMalloc(&p->dmem, off);
+    hipError_t e = hipMalloc(&p->dmem, L.bytes);
     if (e != hipSuccess) {
         hipSetDevice(prev);
-        return set_error(RICK_ERR_NOMEM, "hipMalloc(%zu) failed: %s", off, hipGetErrorString(e));
+        return set_error(RICK_ERR_NOMEM, "hipMalloc(%zu) failed: %s", L.bytes, hipGetErrorString(e));
     }
-    p->dbytes = off;
+    p->dbytes = L.bytes;
     char *base = static_cast<char *>(p->dmem);
-    p->table_d = reinterpret_cast<double *>(base + o_table);
-    if (p->fft_ok && fft_needs_tmp(d.precision, g.ny)) p->tmp_plane = base + o_tmp;
-    if (p->grid_ok) grid_work_carve(g, d.max_points, d.precision, base + o_work, &p->work);
+    p->table_d = reinterpret_cast<double *>(base + L.table);
+    if (p->fft_ok && fft_needs_tmp(d.precision, g.ny)) p->tmp_plane = base + L.tmp;
+    if (p->grid_ok) grid_work_carve(g, d.max_points, d.precision, base + L.work, &p->work);
     // The FP32 split-bucket accumulators and tickets start at zero (the
     // gridder leaves them zero after every call).
-    if (p->grid_ok) e = hipMemset(base + o_work, 0, grid_work_bytes(g, d.max_points, d.precision));
+    if (p->grid_ok) e = hipMemset(base + L.work, 0, grid_work_bytes(g, d.max_points, d.precision));
     if (e != hipSuccess) {
         hipFree(p->dmem);
         hipSetDevice(prev);
@@ -332,23 +362,23 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
         std::vector<float> f(tw.begin(), tw.end());
         return hipMemcpy(base + o, f.data(), 8 * (size_t)n, hipMemcpyHostToDevice);
     };
-    if (e == hipSuccess) e = put_tw(g.nx, o_twx);
-    if (e == hipSuccess) e = put_tw(g.ny, o_twy);
+    if (e == hipSuccess) e = put_tw(g.nx, L.twx);
+    if (e == hipSuccess) e = put_tw(g.ny, L.twy);
     std::vector<double> lt(g.nx), mt(g.ny);
     pixel_sines(g.nx, d.xaxistot > 0 ? d.xaxistot : g.nx, d.resolution, lt.data());
     pixel_sines(g.ny, d.yaxistot > 0 ? d.yaxistot : g.ny, d.resolution, mt.data());
     if (e == hipSuccess)
-        e = hipMemcpy(base + o_l, lt.data(), sizeof(double) * g.nx, hipMemcpyHostToDevice);
+        e = hipMemcpy(base + L.l, lt.data(), sizeof(double) * g.nx, hipMemcpyHostToDevice);
     if (e == hipSuccess)
-        e = hipMemcpy(base + o_m, mt.data(), sizeof(double) * g.ny, hipMemcpyHostToDevice);
+        e = hipMemcpy(base + L.m, mt.data(), sizeof(double) * g.ny, hipMemcpyHostToDevice);
     if (e == hipSuccess && p->gen_ok)
-        e = gen_fft_upload(&p->gen, d.precision, base + o_gen_tab, base + o_gen_work);
+        e = gen_fft_upload(&p->gen, d.precision, base + L.gen_tab, base + L.gen_work);
     hipSetDevice(prev);
     if (e != hipSuccess) {
         hipFree(p->dmem);
         return set_error(RICK_ERR_DEVICE, "table upload failed: %s", hipGetErrorString(e));
     }
-    p->fft = FftPlan{g.planes, g.nx, g.ny, base + o_twx, base + o_twy};
+    p->fft = FftPlan{g.planes, g.nx, g.ny, base + L.twx, base + L.twy};
     PhaseGeom &ph = p->phase;
     ph.planes = g.planes;
     ph.nx = g.nx;
@@ -358,9 +388,28 @@ int rick_plan_create(rick_plan *out, const rick_plan_desc *desc)
     ph.dw = (d.wmax - d.wmin) / (double)d.num_w_planes;
     ph.dwnorm = ph.dw / (d.wmax - d.wmin);
     ph.phase_on = d.phase_on;
-    ph.ltab = reinterpret_cast<const double *>(base + o_l);
-    ph.mtab = reinterpret_cast<const double *>(base + o_m);
+    ph.ltab = reinterpret_cast<const double *>(base + L.l);
+    ph.mtab = reinterpret_cast<const double *>(base + L.m);
     *out = p.release();
+    return RICK_OK;
+}
+
+int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points, rick_plan_shape *shape)
+{
+    clear_error();
+    if (!desc || !shape) return set_error(RICK_ERR_INVALID, "null argument");
+    *shape = rick_plan_shape{};
+    GridGeom g{};
+    const int st = plan_geometry(*desc, g);
+    if (st != RICK_OK) return st;
+    if (num_points > desc->max_points)
+        return set_error(RICK_ERR_INVALID, "num_points %u exceeds plan capacity %u", num_points,
+                         desc->max_points);
+    shape->tile_u = g.tu;
+    shape->tile_v = g.tv;
+    shape->rows_per_task = (int)g.rmax;
+    shape->footprint_unroll = g.smax;
+    shape->device_bytes = plan_layout(*desc, g).bytes;
     return RICK_OK;
 }
 

@@ -141,6 +141,10 @@ class Plan:
             _lib._lib.rick_plan_destroy(h)
             self._h = ctypes.c_void_p()
 
+    def shape(self, num_points=None) -> dict:
+        """Launch shape of a call of ``num_points`` rows (default: the plan's capacity)."""
+        return describe(self.desc, num_points)
+
     @property
     def device_bytes(self) -> int:
         return lib().rick_plan_device_bytes(self._h)
@@ -264,6 +268,15 @@ class Plan:
             self._ptr(image_real, torch.float64, npix, "image_real"),
             self._ptr(image_imag, torch.float64, npix, "image_imag"), self._stream(stream)))
         return image_real, image_imag, grid
+
+
+def describe(desc, num_points=None) -> dict:
+    """Launch shape and device bytes of a plan description (no GPU needed)."""
+    s = _lib.PlanShape()
+    n = desc.max_points if num_points is None else int(num_points)
+    check(lib().rick_plan_describe(ctypes.byref(desc), n, ctypes.byref(s)))
+    return {"tile": (s.tile_u, s.tile_v), "rows_per_task": s.rows_per_task,
+            "unroll": s.footprint_unroll, "device_bytes": s.device_bytes}
 
 
 def plan_for(ds, precision=FP64, **kw) -> Plan:

@@ -1,0 +1,57 @@
+"""Launch shapes and memory of plan descriptions, on the CPU: the built-in choices as
+rick_plan_describe() tells them, and the benchmark's record of them."""
+import pytest
+
+import bench
+from rick_amd import FP32, FP64, KAISERBESSEL, _lib
+from rick_amd.imaging import describe
+
+
+def desc(nx, planes, rows, precision=FP64, support=7, kernel=KAISERBESSEL, **kw):
+    d = _lib.PlanDesc(num_w_planes=planes, grid_size_x=nx, grid_size_y=nx, kernel=kernel,
+                      w_support=support, dx=1.0 / nx, dw=1.0 / planes, precision=precision,
+                      max_points=rows)
+    for k, v in kw.items():
+        setattr(d, k, v)
+    return d
+
+
+@pytest.mark.parametrize("nx,planes,rows,tile", [
+    (256, 4, 50_000, (64, 32)), (512, 16, 100_000, (64, 32)), (512, 17, 100_000, (64, 64)),
+    (4096, 32, 7_745_536, (64, 64)), (8192, 64, 2_900_000, (128, 32))])
+def test_builtin_tiles(nx, planes, rows, tile):
+    assert describe(desc(nx, planes, rows))["tile"] == tile
+
+
+def test_named_shapes_stay():
+    d = desc(8192, 8, 100_000, tile_u=32, tile_v=64, rows_per_task=777, footprint_unroll=11)
+    s = describe(d)
+    assert (s["tile"], s["rows_per_task"], s["unroll"]) == ((32, 64), 777, 11)
+
+
+@pytest.mark.parametrize("bad", [{"w_support": 8}, {"tile_u": 48, "tile_v": 48},
+                                 {"max_points": 2 ** 31}])
+def test_what_no_plan_takes_has_no_shape(bad):
+    with pytest.raises(_lib.RickError):
+        describe(desc(256, 4, 1000, **bad))
+    with pytest.raises(_lib.RickError):
+        describe(desc(256, 4, 1000), 1001)
+
+
+def test_benchmark_records_the_shapes_that_run():
+    rows = 2_900_000
+    plain, named = desc(8192, 64, rows, FP32), desc(8192, 64, rows, FP32, tile_u=64, tile_v=64,
+                                                    rows_per_task=1024)
+    got = bench.launch_shapes(plain, named, rows)
+    assert got["tile"] == [128, 32] and got["image_tile"] == [64, 64]
+    assert got["rows_per_task"] == describe(plain)["rows_per_task"] != 4096
+    assert got["image_rows_per_task"] == 1024 and got["footprint_unroll"] == 7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,planes,rows,precision", [
+    (256, 4, 50_000, FP32), (300, 3, 1000, FP64), (1024, 8, 0, FP32), (2048, 2, 100_000, FP64)])
+def test_described_bytes_are_the_plans(nx, planes, rows, precision):
+    from rick_amd import Plan
+    plan = Plan(nx, nx, planes, precision=precision, max_points=rows)
+    assert plan.shape()["device_bytes"] == plan.device_bytes
