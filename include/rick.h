@@ -144,6 +144,8 @@ typedef struct {
     int tile_u, tile_v;
     int rows_per_task;      /* records per gridding task */
     int footprint_unroll;
+    int by_class;           /* long tasks accumulate by footprint class */
+    int long_tasks_first;   /* order of a dense overwrite; else bucket order */
     size_t device_bytes;    /* rick_plan_device_bytes() of the plan */
 } rick_plan_shape;
 int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points,

@@ -37,7 +37,8 @@ class PlanDesc(ctypes.Structure):
 class PlanShape(ctypes.Structure):
     """rick_plan_shape (include/rick.h)."""
     _fields_ = [("tile_u", _c_int), ("tile_v", _c_int), ("rows_per_task", _c_int),
-                ("footprint_unroll", _c_int), ("device_bytes", _c_size)]
+                ("footprint_unroll", _c_int), ("by_class", _c_int), ("long_tasks_first", _c_int),
+                ("device_bytes", _c_size)]
 
 
 class BinmsMeta(ctypes.Structure):

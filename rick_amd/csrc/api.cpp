@@ -106,15 +106,15 @@ TileShape default_tile(const rick_plan_desc &d)
 // 833 us at 2048, 780 at 8192 and 16384; dense FP32 gridding of 7.7 M rows 1.36 ms at
 // 4096, 1.27 at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us
 // at 512, 98 at 4096.
-uint32_t default_rows_per_task(const rick_plan_desc &d, int tu, int tv, int smax)
+uint32_t default_rows_per_task(const GridGeom &g, uint32_t rows)
 {
     auto from = [](uint32_t share, uint32_t most) {
         uint32_t r = 512;
         while (r < most && r < share) r *= 2;
         return r;
     };
-    const uint32_t r = from(d.max_points / 512u, 16384);
-    return tile_by_class(d, tu, tv, smax) ? std::max(r, from(d.max_points / 192u, 8192)) : r;
+    const uint32_t r = from(rows / 512u, 16384);
+    return tile_by_class(g) ? std::max(r, from(rows / 192u, 8192)) : r;
 }
 
 }  // namespace
@@ -205,7 +205,7 @@ int plan_geometry(const rick_plan_desc &d, GridGeom &g)
                              "w_support %d", d.footprint_unroll, d.w_support);
     }
     g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
-                                 : default_rows_per_task(d, tu, tv, g.smax);
+                                 : default_rows_per_task(g, d.max_points);
     if ((uint64_t)d.max_points * 4ull >= (1ull << 32))
         return set_error(RICK_ERR_INVALID, "max_points %u too large (limit 2^30)", d.max_points);
 
@@ -409,6 +409,8 @@ int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points, rick
     shape->tile_v = g.tv;
     shape->rows_per_task = (int)g.rmax;
     shape->footprint_unroll = g.smax;
+    shape->by_class = tile_by_class(g);
+    shape->long_tasks_first = long_tasks_first(g);
     shape->device_bytes = plan_layout(*desc, g).bytes;
     return RICK_OK;
 }

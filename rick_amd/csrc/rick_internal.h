@@ -169,9 +169,10 @@ struct BatchJob {
     int plane0, planes;     // the job's planes in the group's plane stack
     double dw, inv_dw;      // inv_dw: exact_inverse(dw)
 };
-// Whether the tile kernel of a plan with this tile and footprint unroll takes
-// long tasks by footprint class.
-bool tile_by_class(const rick_plan_desc &d, int tu, int tv, int smax);
+// Whether the tile kernel of this geometry takes long tasks by footprint class.
+bool tile_by_class(const GridGeom &g);
+// Whether a dense overwrite runs its long tasks first, or all of them in bucket order.
+bool long_tasks_first(const GridGeom &g);
 // log2 of the words between the counters of consecutive buckets.
 int counter_shift(uint32_t nb);
 // Rows per block of the count kernel: batch jobs start at multiples of it.

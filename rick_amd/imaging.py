@@ -276,7 +276,8 @@ def describe(desc, num_points=None) -> dict:
     n = desc.max_points if num_points is None else int(num_points)
     check(lib().rick_plan_describe(ctypes.byref(desc), n, ctypes.byref(s)))
     return {"tile": (s.tile_u, s.tile_v), "rows_per_task": s.rows_per_task,
-            "unroll": s.footprint_unroll, "device_bytes": s.device_bytes}
+            "unroll": s.footprint_unroll, "by_class": bool(s.by_class),
+            "long_tasks_first": bool(s.long_tasks_first), "device_bytes": s.device_bytes}
 
 
 def plan_for(ds, precision=FP64, **kw) -> Plan:

@@ -3,7 +3,7 @@ rick_plan_describe() tells them, and the benchmark's record of them."""
 import pytest
 
 import bench
-from rick_amd import FP32, FP64, KAISERBESSEL, _lib
+from rick_amd import FP32, FP64, GAUSS, GAUSS_HI_PRECISION, KAISERBESSEL, _lib
 from rick_amd.imaging import describe
 
 
@@ -27,6 +27,21 @@ def test_named_shapes_stay():
     d = desc(8192, 8, 100_000, tile_u=32, tile_v=64, rows_per_task=777, footprint_unroll=11)
     s = describe(d)
     assert (s["tile"], s["rows_per_task"], s["unroll"]) == ((32, 64), 777, 11)
+
+
+# Large tiles filled record by record keep the bucket order; those by class, and the
+# tiles that take one workgroup per task, run their long tasks first.
+@pytest.mark.parametrize("kernel,support,unroll,tile,by_class,first", [
+    (KAISERBESSEL, 7, 0, (64, 64), True, True), (KAISERBESSEL, 11, 0, (64, 64), True, True),
+    (KAISERBESSEL, 5, 0, (64, 64), False, False), (GAUSS, 3, 0, (64, 64), False, False),
+    (KAISERBESSEL, 7, 9, (64, 64), False, False), (KAISERBESSEL, 15, 0, (64, 64), False, False),
+    (GAUSS_HI_PRECISION, 7, 0, (64, 64), False, False),
+    (KAISERBESSEL, 7, 0, (128, 32), False, False), (KAISERBESSEL, 5, 0, (64, 32), False, True),
+    (GAUSS_HI_PRECISION, 7, 0, (32, 32), False, True)])
+def test_task_order_follows_the_accumulation(kernel, support, unroll, tile, by_class, first):
+    s = describe(desc(1024, 8, 1_000_000, support=support, kernel=kernel, tile_u=tile[0],
+                      tile_v=tile[1], footprint_unroll=unroll))
+    assert (s["by_class"], s["long_tasks_first"]) == (by_class, first)
 
 
 @pytest.mark.parametrize("bad", [{"w_support": 8}, {"tile_u": 48, "tile_v": 48},
