@@ -94,29 +94,6 @@ TileShape default_tile(const rick_plan_desc &d)
     return nb <= 1024 && fits ? TileShape{64, 32} : TileShape{64, 64};
 }
 
-// Built-in records per task: the power of two from the share of one of 512
-// workgroups up (two per CU).  Where the tile kernel takes full tasks by footprint
-// class, whose fixed cost wants long tasks, from the share of one of 192, but over
-// 8192 no longer than the first: a hot tile's tasks would outlast all others (2.8 M
-// rows about the centre of 1024^2 x 23 FP32: tile kernel 170 us at 4096, 145 at 8192,
-// 297 at 16384).  Shorter tasks split more buckets, whose parts meet in atomics;
-// longer ones leave the last workgroups running alone.  Image by records per task:
-// 516 k rows on 512^2 x 8 FP64 137 us at 1024, 119 at 4096, 143 at 8192; 1 M rows on
-// 1024^2 x 16 464 us at 2048, 444 at 8192, 482 at 16384; 3 M rows on 2048^2 x 12 FP32
-// 833 us at 2048, 780 at 8192 and 16384; dense FP32 gridding of 7.7 M rows 1.36 ms at
-// 4096, 1.27 at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us
-// at 512, 98 at 4096.
-uint32_t default_rows_per_task(const GridGeom &g, uint32_t rows)
-{
-    auto from = [](uint32_t share, uint32_t most) {
-        uint32_t r = 512;
-        while (r < most && r < share) r *= 2;
-        return r;
-    };
-    const uint32_t r = from(rows / 512u, 16384);
-    return tile_by_class(g) ? std::max(r, from(rows / 192u, 8192)) : r;
-}
-
 }  // namespace
 
 struct rick_plan_s {
@@ -204,12 +181,18 @@ int plan_geometry(const rick_plan_desc &d, GridGeom &g)
                              "footprint_unroll %d: must be 0 or one of 7, 9, 11, 15 and >= "
                              "w_support %d", d.footprint_unroll, d.w_support);
     }
-    g.rmax = d.rows_per_task > 0 ? (uint32_t)d.rows_per_task
-                                 : default_rows_per_task(g, d.max_points);
+    const bool builtin = d.rows_per_task <= 0;
+    g.rmax = builtin ? default_rows_per_task(g, d.max_points) : (uint32_t)d.rows_per_task;
+    g.rmin = builtin ? kShortestTask : g.rmax;
     if ((uint64_t)d.max_points * 4ull >= (1ull << 32))
         return set_error(RICK_ERR_INVALID, "max_points %u too large (limit 2^30)", d.max_points);
 
     if (d.max_points > 0) {
+        // Built-in tasks are made longer before a plan is refused for their number.
+        while (builtin && g.rmin < 4096 && grid_launch_limit(g, d.max_points)) {
+            g.rmin *= 2;
+            g.rmax = std::max(g.rmax, g.rmin);
+        }
         if (const char *why = grid_launch_limit(g, d.max_points))
             return set_error(RICK_ERR_INVALID, "%d x %d x %d grid, %d x %d tiles, %u points: %s",
                              g.nx, g.ny, g.planes, tu, tv, d.max_points, why);
@@ -407,7 +390,7 @@ int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points, rick
                          desc->max_points);
     shape->tile_u = g.tu;
     shape->tile_v = g.tv;
-    shape->rows_per_task = (int)g.rmax;
+    shape->rows_per_task = (int)call_rows_per_task(g, num_points);
     shape->footprint_unroll = g.smax;
     shape->by_class = tile_by_class(g);
     shape->long_tasks_first = long_tasks_first(g);

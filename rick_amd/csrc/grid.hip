@@ -1672,19 +1672,68 @@ hipError_t launch_tile(const GridGeom &g, const GridWork &w, const double *table
     }
 }
 
+// Most rows for which built-in tasks hold r records or fewer (see
+// default_rows_per_task()).
+uint64_t rows_of_length(const GridGeom &g, uint32_t r)
+{
+    const uint64_t share = tile_by_class(g) && r < 8192 ? 192 : 512;
+    return share * (r + 1ull) - 1;
+}
+
+}  // namespace
+
+// As k_tile decides it, apart from the length of the task.
+bool tile_by_class(const GridGeom &g)
+{
+    return g.kind != RICK_GAUSS_HI_PRECISION && g.support == g.smax &&
+           class_tile(g.tu, g.tv, g.smax);
+}
+
+// Built-in records per task: the power of two from the share of one of 512
+// workgroups up (two per CU).  Where the tile kernel takes full tasks by footprint
+// class, whose fixed cost wants long tasks, from the share of one of 192, but over
+// 8192 no longer than the first: a hot tile's tasks would outlast all others (2.8 M
+// rows about the centre of 1024^2 x 23 FP32: tile kernel 170 us at 4096, 145 at 8192,
+// 297 at 16384).  Shorter tasks split more buckets, whose parts meet in atomics;
+// longer ones leave the last workgroups running alone.  Image by records per task:
+// 516 k rows on 512^2 x 8 FP64 137 us at 1024, 119 at 4096, 143 at 8192; 1 M rows on
+// 1024^2 x 16 464 us at 2048, 444 at 8192, 482 at 16384; 3 M rows on 2048^2 x 12 FP32
+// 833 us at 2048, 780 at 8192 and 16384; dense FP32 gridding of 7.7 M rows 1.36 ms at
+// 4096, 1.27 at 16384, 1.43 at 32768.  Without classes 50 k rows on 256^2 x 4 75 us
+// at 512, 98 at 4096; from support 11 on, where a record adds to 121 cells and more, no
+// task over 4096 (tile kernel of 7.7 M rows at 4096 and 16384 records: support 15 FP64
+// 3.50 and 3.83 ms, FP32 2.30 and 2.34; GAUSS_HI_PRECISION support 11 FP64 2.55 and
+// 2.71, support 7 1.61 and 1.59).
+uint32_t default_rows_per_task(const GridGeom &g, uint32_t rows)
+{
+    const uint32_t most = tile_by_class(g) || g.support < 11 ? 16384 : 4096;
+    uint32_t r = kShortestTask;
+    while (r < most && rows > rows_of_length(g, r)) r *= 2;
+    return r;
+}
+
+namespace {
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Capacities: a footprint (support <= tile size) touches at most 2 tiles per
-// axis, so a row lands in at most 4 buckets; a split bucket holds more than
-// rmax records, so there are at most 4*rows/(rmax+1) of them; tasks number at
-// most nb + 4*rows/rmax.
+// axis, so a row lands in at most 4 buckets; with tasks of r records a split
+// bucket holds more than r, so there are at most 4*rows/(r+1) of them, and tasks
+// number at most nb + 4*rows/r.  r is g.rmax for a call that fills the plan, and
+// a power of two from g.rmin up for one of fewer rows.
 void capacities(const GridGeom &g, uint32_t max_points, uint32_t *rec_cap, uint32_t *split_cap,
                 uint32_t *task_cap, uint32_t *nscan)
 {
     const uint64_t recs = 4ull * (uint64_t)max_points;
+    uint64_t split = recs / ((uint64_t)g.rmax + 1), tasks = recs / g.rmax;
+    for (uint64_t r = g.rmin; r < g.rmax; r *= 2) {
+        const uint64_t n4 = 4ull * std::min<uint64_t>(max_points, rows_of_length(g, (uint32_t)r));
+        split = std::max(split, n4 / (r + 1));
+        tasks = std::max(tasks, n4 / r);
+    }
     *rec_cap = (uint32_t)(recs > 0 ? recs : 1);
-    *split_cap = (uint32_t)(recs / ((uint64_t)g.rmax + 1) + 1);
-    *task_cap = (uint32_t)((uint64_t)g.nb + recs / g.rmax + 1);
+    *split_cap = (uint32_t)(split + 1);
+    *task_cap = (uint32_t)((uint64_t)g.nb + tasks + 1);
     *nscan = (g.nb + kScanBlock - 1) / kScanBlock;
 }
 
@@ -1701,19 +1750,20 @@ int count_rows_per_thread(uint32_t n)
     return n >= 128u * 4 * kBinThreads ? 4 : 1;
 }
 
-// As k_tile decides it, apart from the length of the task.
-bool tile_by_class(const GridGeom &g)
-{
-    return g.kind != RICK_GAUSS_HI_PRECISION && g.support == g.smax &&
-           class_tile(g.tu, g.tv, g.smax);
-}
-
 // See kZeroSpread: large tiles filled record by record keep the bucket order, also
 // those of a shape that goes by class at another support or unroll (64 x 64, the same
 // rows, long tasks first against bucket order: support 5 FP64 1.47 -> 1.34 ms, support
 // 7 with unroll 9 FP64 1.60 -> 1.43 and FP32 0.91 -> 0.88, GAUSS_HI_PRECISION support
 // 7 FP64 1.63 -> 1.53).
 bool long_tasks_first(const GridGeom &g) { return !tile_persistent(g.tu, g.tv) || tile_by_class(g); }
+
+// The length follows the rows of the call, not of the plan (images of 50 k rows on 256^2 x
+// 4 by a plan for 8 M rows, the plan's length against the call's: support 7 FP64 158 ->
+// 74 us, support 15 FP64 731 -> 102; 1 M rows on 1024^2 x 16 FP32 463 -> 279).
+uint32_t call_rows_per_task(const GridGeom &g, uint32_t n)
+{
+    return std::clamp(default_rows_per_task(g, n), g.rmin, g.rmax);
+}
 
 int counter_shift(uint32_t nb)
 {
@@ -1796,7 +1846,7 @@ void grid_work_carve(const GridGeom &g, uint32_t max_points, int precision, void
     w->nscan = nscan;
 }
 
-hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
+hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precision,
                        const double *table_d, uint32_t n, uint32_t F, uint32_t P,
                        const double *uu, const double *vv, const double *ww, const float *vr,
                        const float *vi, const float *wt, void *grid, int accumulate,
@@ -1805,6 +1855,8 @@ hipError_t launch_grid(const GridGeom &g, const GridWork &w, int precision,
 {
     Timing off;
     if (tm == nullptr) tm = &off;
+    GridGeom g = plan_geom;
+    g.rmax = call_rows_per_task(plan_geom, n);
     const uint32_t nblk = (n + kRowsPerBlock - 1) / kRowsPerBlock;
     const int rpt = count_rows_per_thread(n);
     const uint32_t cblk = (uint32_t)(((uint64_t)n + (uint64_t)rpt * kBinThreads - 1) /

@@ -110,6 +110,7 @@ struct GridGeom {
     uint32_t nb;            // buckets = planes*tiles_u*tiles_v
     int cshift;             // log2 words between consecutive buckets' counters
     uint32_t rmax;          // rows per task
+    uint32_t rmin;          // a call's tasks may be this short: call_rows_per_task()
     int ntable;
     double cmax;            // largest per-cell convolution weight (a bound)
     // Power of two <= cmax / (largest table entry): sums of S * K[jKer] scaled by
@@ -169,6 +170,11 @@ struct BatchJob {
     int plane0, planes;     // the job's planes in the group's plane stack
     double dw, inv_dw;      // inv_dw: exact_inverse(dw)
 };
+// Built-in records per task for this many rows, from kShortestTask up.
+constexpr uint32_t kShortestTask = 512;
+uint32_t default_rows_per_task(const GridGeom &g, uint32_t rows);
+// Records per task of a call of n rows.
+uint32_t call_rows_per_task(const GridGeom &g, uint32_t n);
 // Whether the tile kernel of this geometry takes long tasks by footprint class.
 bool tile_by_class(const GridGeom &g);
 // Whether a dense overwrite runs its long tasks first, or all of them in bucket order.

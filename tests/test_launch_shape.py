@@ -44,6 +44,25 @@ def test_task_order_follows_the_accumulation(kernel, support, unroll, tile, by_c
     assert (s["by_class"], s["long_tasks_first"]) == (by_class, first)
 
 
+# A call takes the task length of its own rows, whatever the plan was made for.
+@pytest.mark.parametrize("precision", [FP64, FP32])
+@pytest.mark.parametrize("support,kernel", [(7, KAISERBESSEL), (5, KAISERBESSEL),
+                                            (15, KAISERBESSEL), (7, GAUSS_HI_PRECISION)])
+@pytest.mark.parametrize("rows", [1, 50_000, 516_000, 1_500_000])
+def test_task_length_follows_the_call(rows, support, kernel, precision):
+    own = describe(desc(1024, 8, rows, precision, support, kernel, tile_u=64, tile_v=64))
+    big = describe(desc(1024, 8, 8_000_000, precision, support, kernel, tile_u=64, tile_v=64), rows)
+    assert big["rows_per_task"] == own["rows_per_task"]
+    assert describe(desc(1024, 8, 8_000_000, rows_per_task=3000), rows)["rows_per_task"] == 3000
+
+
+def test_tasks_are_longer_before_a_plan_is_refused():
+    # 8,387,600 tiles of one workgroup each leave slots for 1000 tasks of records.
+    few = describe(desc(32, 8, 500_000, support=5, tile_u=32, tile_v=32))
+    many = describe(desc(32, 8_387_600, 500_000, support=5, tile_u=32, tile_v=32))
+    assert (few["rows_per_task"], many["rows_per_task"]) == (1024, 2048)
+
+
 @pytest.mark.parametrize("bad", [{"w_support": 8}, {"tile_u": 48, "tile_v": 48},
                                  {"max_points": 2 ** 31}])
 def test_what_no_plan_takes_has_no_shape(bad):
