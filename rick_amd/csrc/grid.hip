@@ -309,8 +309,8 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
 }
 
 // Scan of the histogram: grids of up to 1024 buckets in one workgroup, larger
-// ones in two kernels, per-block sums and the downsweep that emits offsets and
-// tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
+// ones in three kernels, per-block sums, their scan and the downsweep that emits
+// offsets and tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
 // the accumulation tasks of three lengths.  The task array holds the long tasks
 // first (more than g.rmax / 2 records), then the middle ones (more than
 // g.rmax / 8), then the short ones, so that no long task starts when the others
@@ -396,6 +396,48 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
     }
 }
 
+// Exclusive scan of each quantity's block sums in place, its total behind them all: one
+// workgroup per quantity.
+constexpr int kTopThreads = 1024;
+__global__ void __launch_bounds__(kTopThreads)
+k_scan_top(uint32_t *__restrict__ blocksum, uint32_t nscan)
+{
+    constexpr uint32_t CHUNK = 4 * kTopThreads;
+    __shared__ uint32_t wsum[kTopThreads / 64];
+    uint32_t *s = blocksum + (size_t)blockIdx.x * nscan;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint32_t i0 = 0; i0 < nscan; i0 += CHUNK) {
+        uint32_t v[4], own = 0;
+        const uint32_t i = i0 + 4 * threadIdx.x;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = i + k < nscan ? s[i + k] : 0u;
+            own += v[k];
+        }
+        uint32_t x = own;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d);
+            if (lane >= d) x += y;
+        }
+        if (lane == 63) wsum[wave] = x;
+        __syncthreads();
+        uint32_t run = carry + x - own;
+        for (int w = 0; w < kTopThreads / 64; ++w) {
+            const uint32_t t = wsum[w];
+            run += w < wave ? t : 0u;
+            carry += t;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i + k < nscan) s[i + k] = run;
+            run += v[k];
+        }
+        __syncthreads();   // wsum is read
+    }
+    if (threadIdx.x == 0) blocksum[(size_t)kScanQ * nscan + blockIdx.x] = carry;
+}
+
 // Tasks first, first + stride, ... of the nt equal parts of split bucket b with
 // c records from ro; they start at slot t.
 __device__ __forceinline__ void split_tasks(uint4 *__restrict__ tasks, uint32_t task_cap,
@@ -413,9 +455,10 @@ __device__ __forceinline__ void split_tasks(uint4 *__restrict__ tasks, uint32_t 
 // Offsets, cursors, tasks and split list of 1024 buckets per workgroup.  The
 // counters it has read and the row flags are cleared on the way: the counters
 // for the next call's count, the flags for this call's tile kernel.  With nscan == 1
-// this is the whole scan; otherwise each workgroup sums the block sums before
-// it (and all of them, for the totals) itself, which for at most a few
-// thousand blocks is less than a launch between the two kernels costs.
+// this is the whole scan; otherwise k_scan_top has scanned the block sums.  (Each
+// workgroup adding up all of them itself saves that launch, but its reads grow with the
+// square of the buckets: scan of 16 M buckets 1114 us against 157, of 1 M 34 and 27, of
+// 16384 18.4 and 17.5.)
 __global__ void __launch_bounds__(kThreads)
 k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restrict__ blocksum,
             uint32_t nscan, uint32_t *__restrict__ offsets, uint32_t *__restrict__ cursor,
@@ -455,32 +498,19 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
         if (lane == 63) wtot[a][wave] = x[a];
     }
     if (threadIdx.x == 0) nbig = 0u;
-    if (threadIdx.x < kScanQ) before[threadIdx.x] = total[threadIdx.x] = 0u;
-    __syncthreads();
-    if (nscan > 1) {
-#pragma unroll
-        for (int a = 0; a < kScanQ; ++a) {
-            uint32_t pre = 0, all = 0;
-            for (uint32_t i = threadIdx.x; i < nscan; i += NT) {
-                const uint32_t y = blocksum[a * nscan + i];
-                all += y;
-                if (i < blockIdx.x) pre += y;
-            }
-            for (int d = 32; d > 0; d >>= 1) {
-                pre += __shfl_xor(pre, d);
-                all += __shfl_xor(all, d);
-            }
-            if (lane == 0) {
-                atomicAdd(&before[a], pre);
-                atomicAdd(&total[a], all);
-            }
-        }
-    } else if (threadIdx.x < kScanQ) {
-        uint32_t all = 0;
-        for (int i = 0; i < NW; ++i) all += wtot[threadIdx.x][i];
-        total[threadIdx.x] = all;
+    if (threadIdx.x < kScanQ) {
+        before[threadIdx.x] = nscan > 1 ? blocksum[(size_t)threadIdx.x * nscan + blockIdx.x] : 0u;
+        if (nscan > 1) total[threadIdx.x] = blocksum[(size_t)kScanQ * nscan + threadIdx.x];
     }
     __syncthreads();
+    if (nscan == 1) {
+        if (threadIdx.x < kScanQ) {
+            uint32_t all = 0;
+            for (int i = 0; i < NW; ++i) all += wtot[threadIdx.x][i];
+            total[threadIdx.x] = all;
+        }
+        __syncthreads();
+    }
     uint32_t ex[kScanQ];
 #pragma unroll
     for (int a = 0; a < kScanQ; ++a) {
@@ -1800,7 +1830,7 @@ size_t grid_work_bytes(const GridGeom &g, uint32_t max_points, int precision)
     b += align_up((size_t)g.planes * g.ny, 256);           // rowlive (after the counts)
     b += align_up((sizeof(uint32_t) * g.nb) << g.cshift, 256);   // cursor
     b += align_up(sizeof(uint32_t) * (g.nb + 1), 256);     // offsets
-    b += align_up(sizeof(uint32_t) * kScanQ * nscan, 256); // blocksum
+    b += align_up(sizeof(uint32_t) * kScanQ * (nscan + 1), 256); // blocksum, totals
     b += align_up(sizeof(uint4) * task_cap, 256);          // tasks
     b += align_up(sizeof(uint32_t) * split_cap, 256);      // split_list
     b += align_up(sizeof(uint32_t) * 8, 256);              // meta
@@ -1828,7 +1858,7 @@ void grid_work_carve(const GridGeom &g, uint32_t max_points, int precision, void
     w->rowlive = reinterpret_cast<unsigned char *>(take((size_t)g.planes * g.ny));
     w->cursor = reinterpret_cast<uint32_t *>(take((sizeof(uint32_t) * g.nb) << g.cshift));
     w->offsets = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * (g.nb + 1)));
-    w->blocksum = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * kScanQ * nscan));
+    w->blocksum = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * kScanQ * (nscan + 1)));
     w->tasks = reinterpret_cast<uint4 *>(take(sizeof(uint4) * task_cap));
     w->split_list = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * split_cap));
     w->meta = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t) * 8));
@@ -1895,6 +1925,8 @@ hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precisi
     } else {
         hipLaunchKernelGGL(k_scan_reduce, dim3(w.nscan), dim3(kThreads), 0, s, g, w.counts,
                            w.blocksum, w.nscan, zero);
+        hipLaunchKernelGGL(k_scan_top, dim3(kScanQ), dim3(kTopThreads), 0, s, w.blocksum,
+                           w.nscan);
         hipLaunchKernelGGL(k_scan_down, dim3(w.nscan), dim3(kThreads), 0, s, g,
                            w.counts, w.blocksum, w.nscan, w.offsets, w.cursor, w.tasks,
                            w.task_cap, w.split_list, w.split_cap, w.meta, rl, rl_words, zero);

@@ -137,7 +137,7 @@ struct GridWork {
     uint32_t *counts;       // [nb << cshift] records per bucket; zero between calls
     uint32_t *cursor;       // [nb << cshift] scatter cursor (starts at the bucket offset)
     uint32_t *offsets;      // [nb+1] exclusive scan of counts
-    uint32_t *blocksum;     // [7*nscan] per scan block: records, split and non-empty buckets,
+    uint32_t *blocksum;     // [7*(nscan+1)] per scan block: records, split and non-empty buckets,
                             //   zero tasks, accumulation tasks by length
     uint4 *tasks;           // [task_cap] (bucket, first record, end record, split)
     uint32_t *split_list;   // [split_cap] buckets handled by more than one task
