@@ -750,6 +750,7 @@ int gen_phase_lines(const GenPassDesc &gp, int nl, int sets)
 {
     if (gp.np == 0) return 0;
     const int G = gen_lines(gp, nl, gen_elems<double>(), true, kPhaseValues);
+    if (!gen_threads(gp, G, kPhaseValues)) return 0;   // radix 6 or 7 of a line above 3072
     return (long long)((nl + G - 1) / G) * sets >= 1024 ? G : 0;
 }
 
