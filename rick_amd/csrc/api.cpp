@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -776,10 +777,11 @@ struct Ctx {
 constexpr size_t kPiece = 4ull << 20;   // bytes of a staging piece
 constexpr size_t kPieces = 4;           // pieces in flight
 constexpr size_t kCopyShare = 256 << 10;   // least bytes of a copy per thread
-constexpr int kCopyThreads = 8;         // most threads of a copy below kLarge
-// Copies of kLarge bytes and more take twice as many threads and pieces four times
-// as long.
-constexpr size_t kLarge = 256ull << 20;
+// Looks (and yields) of an idle thread before it sleeps: short copies are over before a
+// thread that sleeps would be back.
+constexpr int kCopySpins = 4000, kLargeCopySpins = 100;
+constexpr int kCopyThreads = 8;         // most threads of a copy
+constexpr size_t kLarge = 256ull << 20;    // copies from here on take pieces of 32 MB
 
 Ctx *context_for(int rank)
 {
@@ -843,15 +845,19 @@ enum class Copy { to_device, to_host, add_to_host };
 // device and 64 MB pieces back: wstack() 2.86 / 2.02 / 1.87 -> 2.37 / 1.39 / 1.43
 // ms with 1 / 4 / 8 threads, phase_correction() 1.50 / 1.39 / 1.56 -> 1.50 / 0.96
 // / 1.01, rick_fft_planes() 3.21 -> 1.74; more than 8 threads cost more to start
-// than they add (16: 1.60 and 1.18 ms).  Large copies hide that, and want longer
-// pieces: wstack() into a grid of 8.6 GB 214 ms with 8 threads, 209 with 16, 193 with
-// those and 16 MB pieces.
+// than they add (16: 1.60 and 1.18 ms).  Large copies want longer pieces: wstack()
+// into a grid of 8.6 GB 0.179 s (0.1790 .. 0.1792 in 12 calls with 4, 8 and 16 threads),
+// with 16 MB pieces 0.183, with two of 64 MB 0.177.  Few pieces also make few commands:
+// after some 500 on a stream the runtime moves it to another copy engine, and where
+// that one is busy (just after gigabytes of device memory were freed) a call takes twice
+// as long (0.32 s at 16 MB in every other call, 0.179 in 26 of 26 at 32 MB).  Idle
+// threads sleep: 0.8 s of CPU time a call, 2.9 s while 16 of them spun.
 int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthreads)
 {
     std::vector<HostCopy> pieces;
     size_t total = 0;
     for (const HostCopy &a : arrays) total += a.bytes;
-    const size_t piece = total >= kLarge ? 4 * kPiece : kPiece;
+    const size_t piece = total >= kLarge ? 8 * kPiece : kPiece;
     for (const HostCopy &a : arrays)
         for (size_t o = 0; o < a.bytes; o += piece)
             pieces.push_back(HostCopy{a.dev + o, a.host + o, std::min(piece, a.bytes - o)});
@@ -886,8 +892,25 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
     std::atomic<size_t> open{how == Copy::to_device ? kPieces : 0};
     std::vector<std::atomic<int>> done(n);
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
-    std::atomic<int> team{1};       // threads at work, final before `start`
-    std::atomic<bool> start{false}, stop{false};
+    std::atomic<int> team{0};       // threads at work, 0 until all have been started
+    std::atomic<bool> stop{false};
+    // A thread that has nothing to do looks again a few times, then sleeps until a
+    // piece opens (helpers) or is finished (the calling thread).
+    std::mutex mu;
+    std::condition_variable changed;
+    const int spins = total >= kLarge ? kLargeCopySpins : kCopySpins;
+    auto wait_for = [&](auto &&ready) {
+        for (int k = 0; k < spins; ++k) {
+            if (ready()) return;
+            std::this_thread::yield();
+        }
+        std::unique_lock<std::mutex> lk(mu);
+        changed.wait(lk, ready);
+    };
+    auto tell = [&] {
+        { std::lock_guard<std::mutex> lk(mu); }   // no waiter is between its test and its sleep
+        changed.notify_all();
+    };
     auto part = [&](size_t i, int t, int nt) {
         const HostCopy &p = pieces[i];
         const size_t per = ((p.bytes + nt - 1) / nt + 63) / 64 * 64;
@@ -902,21 +925,18 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             const double *src = reinterpret_cast<const double *>(buf + a);
             for (size_t q = 0; q < (b - a) / sizeof(double); ++q) dst[q] += src[q];
         }
-        done[i].fetch_add(1, std::memory_order_release);
+        if (done[i].fetch_add(1, std::memory_order_acq_rel) + 1 == nt) tell();
     };
     auto helper = [&](int t) {
-        while (!start.load(std::memory_order_acquire)) std::this_thread::yield();
+        wait_for([&] { return team.load(std::memory_order_acquire) > 0; });
         const int nt = team.load();
         for (size_t i = 0; i < n; ++i) {
-            while (open.load(std::memory_order_acquire) <= i) {
-                if (stop.load()) return;
-                std::this_thread::yield();
-            }
+            wait_for([&] { return open.load(std::memory_order_acquire) > i || stop.load(); });
+            if (open.load(std::memory_order_acquire) <= i) return;
             part(i, t, nt);
         }
     };
-    const int most = total >= kLarge ? 2 * kCopyThreads : kCopyThreads;
-    const int want = (int)std::min<size_t>(std::max(1, std::min(nthreads, most)),
+    const int want = (int)std::min<size_t>(std::max(1, std::min(nthreads, kCopyThreads)),
                                            std::max<size_t>(1, total / kCopyShare));
     std::vector<std::thread> th;
     try {
@@ -925,8 +945,8 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
         // The threads that did start share the work.
     }
     const int nt = 1 + (int)th.size();
-    team.store(nt);
-    start.store(true, std::memory_order_release);
+    team.store(nt, std::memory_order_release);
+    tell();
     auto queue = [&](size_t i) {
         const HostCopy &p = pieces[i];
         char *buf = c.pinned + (i % kPieces) * piece;
@@ -937,7 +957,11 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
         return e != hipSuccess ? e : hipEventRecord(c.staged[i % kPieces], c.stream);
     };
     auto all_done = [&](size_t i) {
-        while (done[i].load(std::memory_order_acquire) < nt) std::this_thread::yield();
+        wait_for([&] { return done[i].load(std::memory_order_acquire) >= nt; });
+    };
+    auto open_to = [&](size_t count) {
+        open.store(count, std::memory_order_release);
+        tell();
     };
     hipError_t e = hipSuccess;
     if (how != Copy::to_device)
@@ -950,17 +974,20 @@ int copy_arrays(Ctx &c, const std::vector<HostCopy> &arrays, Copy how, int nthre
             // The next piece to open takes the buffer of the one kPieces before it.
             if (e == hipSuccess && i + 1 >= kPieces && i + 1 < n)
                 e = hipEventSynchronize(c.staged[(i + 1) % kPieces]);
-            if (e == hipSuccess) open.store(std::max(kPieces, i + 2), std::memory_order_release);
+            if (e == hipSuccess) open_to(std::max(kPieces, i + 2));
         } else {
             e = hipEventSynchronize(c.staged[i % kPieces]);
             if (e != hipSuccess) break;
-            open.store(i + 1, std::memory_order_release);
+            open_to(i + 1);
             part(i, 0, nt);
             all_done(i);
             if (i + kPieces < n) e = queue(i + kPieces);
         }
     }
-    stop.store(e != hipSuccess);
+    if (e != hipSuccess) {
+        stop.store(true);
+        tell();
+    }
     for (auto &x : th) x.join();
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(c.stream);
