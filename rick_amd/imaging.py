@@ -102,6 +102,32 @@ def _torch():
     return torch
 
 
+def plan_desc(grid_x, grid_y, planes, kernel=KAISERBESSEL, support=7, dx=None, dw=None,
+              precision=FP64, max_points=0, resolution=1.0, wmin=0.0, wmax=1.0, phase_on=True,
+              tile=(0, 0), rows_per_task=0, device=0, xaxistot=0, yaxistot=0, unroll=0):
+    """The rick_plan_desc of these arguments."""
+    d = _lib.PlanDesc()
+    d.num_w_planes = planes
+    d.grid_size_x = grid_x
+    d.grid_size_y = grid_y
+    d.kernel = KERNELS.get(kernel, kernel) if isinstance(kernel, str) else kernel
+    d.w_support = support
+    d.dx = 1.0 / grid_x if dx is None else dx      # init.c:11
+    d.dw = 1.0 / planes if dw is None else dw      # init.c:12
+    d.precision = precision
+    d.max_points = max_points
+    d.resolution = resolution
+    d.wmin = wmin
+    d.wmax = wmax
+    d.phase_on = int(bool(phase_on))
+    d.tile_u, d.tile_v = tile
+    d.rows_per_task = rows_per_task
+    d.device = device
+    d.xaxistot, d.yaxistot = xaxistot, yaxistot   # a rank's slab of the image
+    d.footprint_unroll = unroll                    # 0: smallest of 7, 9, 11, 15 >= support
+    return d
+
+
 class Plan:
     """A rick_plan: device tables and gridding workspace for one problem shape."""
 
@@ -109,26 +135,9 @@ class Plan:
                  dw=None, precision=FP64, max_points=0, resolution=1.0, wmin=0.0, wmax=1.0,
                  phase_on=True, tile=(0, 0), rows_per_task=0, device=0, xaxistot=0,
                  yaxistot=0, unroll=0):
-        d = _lib.PlanDesc()
-        d.num_w_planes = planes
-        d.grid_size_x = grid_x
-        d.grid_size_y = grid_y
-        d.kernel = KERNELS.get(kernel, kernel) if isinstance(kernel, str) else kernel
-        d.w_support = support
-        d.dx = 1.0 / grid_x if dx is None else dx      # init.c:11
-        d.dw = 1.0 / planes if dw is None else dw      # init.c:12
-        d.precision = precision
-        d.max_points = max_points
-        d.resolution = resolution
-        d.wmin = wmin
-        d.wmax = wmax
-        d.phase_on = int(bool(phase_on))
-        d.tile_u, d.tile_v = tile
-        d.rows_per_task = rows_per_task
-        d.device = device
-        d.xaxistot, d.yaxistot = xaxistot, yaxistot   # a rank's slab of the image
-        d.footprint_unroll = unroll                    # 0: smallest of 7, 9, 11, 15 >= support
-        self.desc = d
+        self.desc = d = plan_desc(grid_x, grid_y, planes, kernel, support, dx, dw, precision,
+                                  max_points, resolution, wmin, wmax, phase_on, tile,
+                                  rows_per_task, device, xaxistot, yaxistot, unroll)
         self._h = ctypes.c_void_p()
         check(lib().rick_plan_create(ctypes.byref(self._h), ctypes.byref(d)))
         self.nx, self.ny, self.planes = grid_x, grid_y, planes

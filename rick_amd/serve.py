@@ -5,7 +5,7 @@ arrive over time.  The scheduler keeps up to `slots` jobs on the device at
 once, each on its own stream, and admits queued requests in arrival order as
 soon as a slot and enough HBM are free: a job's footprint (its grid, images and
 plan workspace, bytes computed from planes x grid^2 x element size and the
-gridder's capacities) is charged against `hbm_budget`.  Plans and buffers are
+library's count of the plan's memory) is charged against `hbm_budget`.  Plans and buffers are
 pooled per job signature, so after warm-up no request allocates; idle pooled
 buffers stay charged to the budget too, and when a job would not fit, idle
 entries of other signatures are freed, least recently used first.
@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import argparse
 import collections
+import functools
 import json
 import sys
 import time
@@ -30,7 +31,8 @@ from dataclasses import dataclass, field
 import numpy as np
 
 from . import synth
-from ._lib import FP32, FP64
+from ._lib import FP32, FP64, RickError
+from .imaging import describe, plan_desc
 
 
 @dataclass
@@ -53,10 +55,19 @@ def grid_footprint(cfg, precision) -> int:
     cb = 16 if precision == FP64 else 8
     grid = cfg.planes * cfg.grid * cfg.grid * cb
     images = 2 * 8 * cfg.grid * cfg.grid
-    rec = (32 if precision == FP64 else 24) * 4 * cfg.n_rows
-    tiles = cfg.planes * max(1, cfg.grid // 32) ** 2
-    work = rec + 48 * tiles + (cfg.grid * cfg.grid * cb if cfg.grid > 512 else 0)
-    return grid + images + work
+    return grid + images + _plan_bytes(cfg.grid, cfg.planes, cfg.kernel, cfg.support, cfg.n_rows,
+                                       precision)
+
+
+@functools.lru_cache(maxsize=1024)
+def _plan_bytes(grid, planes, kernel, support, rows, precision) -> int:
+    """Device bytes of the job's plan, as the library counts them; 0 for a job no
+    plan takes (it fails when it is started, by itself)."""
+    try:
+        return describe(plan_desc(grid, grid, planes, kernel=kernel, support=support,
+                                  precision=precision, max_points=rows))["device_bytes"]
+    except RickError:
+        return 0
 
 
 class PlanPool:

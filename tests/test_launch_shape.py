@@ -3,7 +3,7 @@ rick_plan_describe() tells them, and the benchmark's record of them."""
 import pytest
 
 import bench
-from rick_amd import FP32, FP64, GAUSS, GAUSS_HI_PRECISION, KAISERBESSEL, _lib
+from rick_amd import FP32, FP64, GAUSS, GAUSS_HI_PRECISION, KAISERBESSEL, _lib, serve
 from rick_amd.imaging import describe
 
 
@@ -80,6 +80,21 @@ def test_benchmark_records_the_shapes_that_run():
     assert got["tile"] == [128, 32] and got["image_tile"] == [64, 64]
     assert got["rows_per_task"] == describe(plain)["rows_per_task"] != 4096
     assert got["image_rows_per_task"] == 1024 and got["footprint_unroll"] == 7
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32])
+@pytest.mark.parametrize("grid,planes,rows", [(256, 4, 50_000), (1024, 16, 1_000_000),
+                                              (2048, 12, 3_000_000), (300, 4, 20_000)])
+def test_service_charges_the_whole_plan(grid, planes, rows, precision):
+    class Cfg:
+        kernel, support, n_rows = KAISERBESSEL, 7, rows
+    Cfg.grid, Cfg.planes = grid, planes
+    cell = 16 if precision == FP64 else 8
+    held = (planes * cell + 2 * 8) * grid * grid
+    held += describe(desc(grid, planes, rows, precision))["device_bytes"]
+    assert serve.grid_footprint(Cfg, precision) == held
+    Cfg.support = 8         # refused: the job fails by itself, the service goes on
+    assert 0 < serve.grid_footprint(Cfg, precision) < held
 
 
 @pytest.mark.gpu
