@@ -394,7 +394,7 @@ int rick_plan_describe(const rick_plan_desc *desc, unsigned int num_points, rick
     shape->rows_per_task = (int)call_rows_per_task(g, num_points);
     shape->footprint_unroll = g.smax;
     shape->by_class = tile_by_class(g);
-    shape->long_tasks_first = long_tasks_first(g);
+    shape->long_tasks_first = long_tasks_first(g, desc->precision, num_points);
     shape->device_bytes = plan_layout(*desc, g).bytes;
     return RICK_OK;
 }

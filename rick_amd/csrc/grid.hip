@@ -1780,12 +1780,20 @@ int count_rows_per_thread(uint32_t n)
     return n >= 128u * 4 * kBinThreads ? 4 : 1;
 }
 
-// See kZeroSpread: large tiles filled record by record keep the bucket order, also
-// those of a shape that goes by class at another support or unroll (64 x 64, the same
-// rows, long tasks first against bucket order: support 5 FP64 1.47 -> 1.34 ms, support
-// 7 with unroll 9 FP64 1.60 -> 1.43 and FP32 0.91 -> 0.88, GAUSS_HI_PRECISION support
-// 7 FP64 1.63 -> 1.53).
-bool long_tasks_first(const GridGeom &g) { return !tile_persistent(g.tu, g.tv) || tile_by_class(g); }
+// See kZeroSpread: FP64 tiles filled record by record keep the bucket order where the
+// grid is large beside the records' adds, 20 bytes and more for each cell of each row's
+// footprint.  Tasks in bucket order against long ones first, dense gridding: 4096^2 x 32,
+// 7.7 M rows, unroll 9 (support 7, 23 bytes) 1920 -> 1751 us, support 5 (44) 1749 -> 1655;
+// 2048^2 x 8, 0.5 M rows, support 5 (44) 170 -> 156; but support 9 of
+// GAUSS_HI_PRECISION (13.7) 2159 -> 2229, 2048^2 x 16 with 7.7 M rows, support 7 (2.8)
+// 1003 -> 1161.  FP32 grids write half the bytes and lose or gain nothing: 4096^2 x 32
+// support 7 1177 -> 1159, support 5 1034 both, 2048^2 x 8 with 0.5 M rows 150 -> 169.
+bool long_tasks_first(const GridGeom &g, int precision, uint32_t n)
+{
+    if (!tile_persistent(g.tu, g.tv) || tile_by_class(g) || precision == RICK_FP32) return true;
+    const double bytes = 16.0 * g.planes * g.nx * g.ny;
+    return bytes < 20.0 * n * g.support * g.support;
+}
 
 // The length follows the rows of the call, not of the plan (images of 50 k rows on 256^2 x
 // 4 by a plan for 8 M rows, the plan's length against the call's: support 7 FP64 158 ->
@@ -1893,8 +1901,8 @@ hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precisi
                                      ((uint64_t)rpt * kBinThreads));
     // Overwrite of a dense grid: runs of empty buckets get zero tasks.
     const int zero = accumulate || !clear_empty ? kZeroNone
-                     : long_tasks_first(g)      ? kZeroLong
-                                                : kZeroSpread;
+                     : long_tasks_first(g, precision, n) ? kZeroLong
+                                                         : kZeroSpread;
     // Overwrite of a sparse grid: the tile kernel flags the rows it writes
     // non-zero cells to, for the image chain.
     unsigned char *rowlive = (!accumulate && !clear_empty) ? w.rowlive : nullptr;

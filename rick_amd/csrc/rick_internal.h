@@ -177,8 +177,9 @@ uint32_t default_rows_per_task(const GridGeom &g, uint32_t rows);
 uint32_t call_rows_per_task(const GridGeom &g, uint32_t n);
 // Whether the tile kernel of this geometry takes long tasks by footprint class.
 bool tile_by_class(const GridGeom &g);
-// Whether a dense overwrite runs its long tasks first, or all of them in bucket order.
-bool long_tasks_first(const GridGeom &g);
+// Whether a dense overwrite of n rows runs its long tasks first, or all of them in
+// bucket order.
+bool long_tasks_first(const GridGeom &g, int precision, uint32_t n);
 // log2 of the words between the counters of consecutive buckets.
 int counter_shift(uint32_t nb);
 // Rows per block of the count kernel: batch jobs start at multiples of it.

@@ -29,19 +29,23 @@ def test_named_shapes_stay():
     assert (s["tile"], s["rows_per_task"], s["unroll"]) == ((32, 64), 777, 11)
 
 
-# Large tiles filled record by record keep the bucket order; those by class, and the
-# tiles that take one workgroup per task, run their long tasks first.
-@pytest.mark.parametrize("kernel,support,unroll,tile,by_class,first", [
-    (KAISERBESSEL, 7, 0, (64, 64), True, True), (KAISERBESSEL, 11, 0, (64, 64), True, True),
-    (KAISERBESSEL, 5, 0, (64, 64), False, False), (GAUSS, 3, 0, (64, 64), False, False),
-    (KAISERBESSEL, 7, 9, (64, 64), False, False), (KAISERBESSEL, 15, 0, (64, 64), False, False),
-    (GAUSS_HI_PRECISION, 7, 0, (64, 64), False, False),
-    (KAISERBESSEL, 7, 0, (128, 32), False, False), (KAISERBESSEL, 5, 0, (64, 32), False, True),
-    (GAUSS_HI_PRECISION, 7, 0, (32, 32), False, True)])
-def test_task_order_follows_the_accumulation(kernel, support, unroll, tile, by_class, first):
-    s = describe(desc(1024, 8, 1_000_000, support=support, kernel=kernel, tile_u=tile[0],
-                      tile_v=tile[1], footprint_unroll=unroll))
-    assert (s["by_class"], s["long_tasks_first"]) == (by_class, first)
+# Large FP64 tiles filled record by record keep the bucket order where the grid is large
+# beside the rows; those by class, smaller ones and FP32 run their long tasks first.
+@pytest.mark.parametrize("kernel,support,unroll,tile,by_class,bucket_order", [
+    (KAISERBESSEL, 7, 0, (64, 64), True, False), (KAISERBESSEL, 11, 0, (64, 64), True, False),
+    (KAISERBESSEL, 5, 0, (64, 64), False, True), (GAUSS, 3, 0, (64, 64), False, True),
+    (KAISERBESSEL, 7, 9, (64, 64), False, True), (KAISERBESSEL, 15, 0, (64, 64), False, True),
+    (GAUSS_HI_PRECISION, 7, 0, (64, 64), False, True),
+    (KAISERBESSEL, 7, 0, (128, 32), False, True), (KAISERBESSEL, 5, 0, (64, 32), False, False),
+    (GAUSS_HI_PRECISION, 7, 0, (32, 32), False, False)])
+def test_task_order_follows_the_accumulation(kernel, support, unroll, tile, by_class, bucket_order):
+    shape = dict(support=support, kernel=kernel, tile_u=tile[0], tile_v=tile[1],
+                 footprint_unroll=unroll)
+    most = 16 * 8 * 1024 * 1024 // (20 * support * support)      # 20 bytes a footprint cell
+    for rows, order in ((most, bucket_order), (most + 1, False)):
+        s = describe(desc(1024, 8, 1_000_000, **shape), rows)
+        assert (s["by_class"], s["long_tasks_first"]) == (by_class, not order)
+        assert describe(desc(1024, 8, 1_000_000, FP32, **shape), rows)["long_tasks_first"]
 
 
 # A call takes the task length of its own rows, whatever the plan was made for.
