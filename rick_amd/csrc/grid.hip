@@ -1134,7 +1134,18 @@ __device__ __forceinline__ uint32_t odd_owner(double pu, double pv, int c, uint3
 
 // Tiles that LDS holds to two workgroups per CU keep within the registers of
 // four waves per SIMD.
-template <int PREC, int TU, int TV, int SMAX, bool HIPREC>
+// KIND: how the records are accumulated; kTileClasses takes short tasks, and supports
+// below SMAX, record by record too.
+enum { kTileRecords, kTileClasses, kTileHiPrec };
+// Whether accumulation record by record alone has an instance of its own: F and the
+// queues leave three workgroups of a 64 x 32 tile to a CU (43.6 KB of LDS), the tile alone
+// four (36.9 KB; tile kernel of 7.7 M rows added to 4096^2 x 32: support 3 FP64 435 ->
+// 365 us and FP32 434 -> 374, support 5 618 -> 534 and 535 -> 478).
+__host__ __device__ constexpr bool own_records(int tu, int tv, int smax)
+{
+    return tu == 64 && tv == 32 && class_tile(tu, tv, smax);
+}
+template <int PREC, int TU, int TV, int SMAX, int KIND>
 __global__ void __launch_bounds__(kTileThreads, tile_persistent(TU, TV) ? 4 : 1)
 k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
        const typename RecOf<PREC>::type *__restrict__ rec, const double *__restrict__ table,
@@ -1145,7 +1156,7 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
     using T = typename std::conditional<PREC == RICK_FP64, double, float>::type;
     using T2 = typename std::conditional<PREC == RICK_FP64, double2, float2>::type;
     constexpr int LDU = TU + kPadU;
-    constexpr bool CLS = !HIPREC && class_tile(TU, TV, SMAX);
+    constexpr bool CLS = KIND == kTileClasses && class_tile(TU, TV, SMAX);
     constexpr int RF = TV + SMAX - 1;   // rows of F
     __shared__ double lds[CLS && RF * TU > TV * LDU ? 2 * RF * TU : 2 * TV * LDU];
     __shared__ double stab[kMaxTable];
@@ -1294,7 +1305,7 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
         const int S = g.support, KL = g.kl;
         // Per-cell Gaussian (GAUSS_HI_PRECISION) or table product: a template
         // parameter, so each instantiation carries only its own cell arithmetic.
-        constexpr bool hiprec = HIPREC;
+        constexpr bool hiprec = KIND == kTileHiPrec;
         // gauss_kernel_norm constants (w-stacking.cu:254-256).
         const double std22 = 1.0 / (2.0 * 1.0 * 1.0);
         const double gnorm = std22 / kRefPi;
@@ -1632,11 +1643,11 @@ k_tile(GridGeom g, const uint4 *__restrict__ tasks, uint32_t *__restrict__ meta,
 // per device and kernel).  Smaller launches keep one workgroup per slot: they
 // often run beside other jobs on other streams, which persistent workgroups
 // would hold off the CUs.
-template <int PREC, int TU, int TV, int SMAX, bool HIPREC>
+template <int PREC, int TU, int TV, int SMAX, int KIND>
 uint32_t tile_grid(uint32_t task_cap)
 {
     if (!tile_persistent(TU, TV)) return task_cap;
-    const void *kernel = reinterpret_cast<const void *>(&k_tile<PREC, TU, TV, SMAX, HIPREC>);
+    const void *kernel = reinterpret_cast<const void *>(&k_tile<PREC, TU, TV, SMAX, KIND>);
     static std::atomic<uint32_t> resident[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return task_cap;
@@ -1662,18 +1673,20 @@ hipError_t launch_tile_s(const GridGeom &g, const GridWork &w, const double *tab
     using Rec = typename RecOf<PREC>::type;
     const Rec *rec = static_cast<const Rec *>(w.records);
     const dim3 blk(kTileThreads);
-#define RICK_TILE_LAUNCH(A, B, HI)                                                          \
-    hipLaunchKernelGGL((k_tile<PREC, A, B, SMAX, HI>),                                      \
-                       dim3(tile_grid<PREC, A, B, SMAX, HI>(w.task_cap)), blk, 0, s,        \
+#define RICK_TILE_LAUNCH(A, B, KIND)                                                        \
+    hipLaunchKernelGGL((k_tile<PREC, A, B, SMAX, KIND>),                                    \
+                       dim3(tile_grid<PREC, A, B, SMAX, KIND>(w.task_cap)), blk, 0, s,      \
                        g, w.tasks, w.meta, rec, table, grid, accumulate, w.offsets,        \
                        w.split_ticket, w.split_acc, rowlive)
 #define RICK_TILE_CASE(A, B)                                                                \
     if (g.tu == A && g.tv == B) {                                                           \
         tm->begin(RICK_STAGE_TILE, s);                                                      \
         if (g.kind == RICK_GAUSS_HI_PRECISION)                                              \
-            RICK_TILE_LAUNCH(A, B, true);                                                   \
+            RICK_TILE_LAUNCH(A, B, kTileHiPrec);                                            \
+        else if (own_records(A, B, SMAX) && !tile_by_class(g))                              \
+            RICK_TILE_LAUNCH(A, B, (own_records(A, B, SMAX) ? kTileRecords : kTileClasses)); \
         else                                                                                \
-            RICK_TILE_LAUNCH(A, B, false);                                                  \
+            RICK_TILE_LAUNCH(A, B, kTileClasses);                                           \
         tm->end(RICK_STAGE_TILE, s);                                                        \
         return hipGetLastError();                                                           \
     }
