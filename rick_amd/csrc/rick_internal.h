@@ -110,7 +110,6 @@ struct GridGeom {
     uint32_t nb;            // buckets = planes*tiles_u*tiles_v
     int cshift;             // log2 words between consecutive buckets' counters
     uint32_t rmax;          // rows per task
-    uint32_t rmin;          // a call's tasks may be this short: call_rows_per_task()
     int ntable;
     double cmax;            // largest per-cell convolution weight (a bound)
     // Power of two <= cmax / (largest table entry): sums of S * K[jKer] scaled by
@@ -121,6 +120,7 @@ struct GridGeom {
     // 1/dx and 1/dw when dx / dw are powers of two (then x * inv is exactly
     // the IEEE quotient x / d), else 0 (divide).
     double inv_dx, inv_dw;
+    uint32_t rmin;          // a call's tasks may be this short: call_rows_per_task()
 };
 
 // 1/d if d is a power of two whose reciprocal is exact, else 0.
