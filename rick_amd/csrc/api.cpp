@@ -82,12 +82,18 @@ const TileShape kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {128, 32}, {32, 64}};
 // more workgroups (512^2 x 8 planes, 516 k rows: image 171 -> 165 us, 256^2 x 4
 // 81 -> 77 us; 1024^2 x 16 with 4096 tiles: 670 -> 677 us), and rows above 4096
 // cells 128 x 32, which keeps them at 64 tiles, the row transform's occupancy
-// mask (8192^2 x 64 planes: image 23.1 -> 22.6 ms).
+// mask (8192^2 x 64 planes: image 23.1 -> 22.6 ms).  GAUSS_HI_PRECISION of support 9 and
+// more, whose records cost most, takes 64 x 32 only for tiles that are few and full:
+// gridding with 64 x 32 and 64 x 64 tiles, support 9 FP64, 693 rows on 256 x 128 x 2 60
+// and 46 us, 50 k rows on 512^2 x 8 84 and 65, on 256^2 x 4 50 and 55.
 TileShape default_tile(const rick_plan_desc &d)
 {
     if (d.grid_size_x > 4096) return {128, 32};
     const uint64_t nb = (uint64_t)d.num_w_planes * ((d.grid_size_x + 63) / 64) *
                         ((d.grid_size_y + 63) / 64);
+    if (d.kernel == RICK_GAUSS_HI_PRECISION && d.w_support >= 9 &&
+        (nb > 256 || d.max_points < 128 * nb))
+        return {64, 64};
     // 64 x 32 tiles take one workgroup per task, of which a launch holds fewer
     // than 2^32 threads; the larger tiles' workgroups stay and take many.
     const uint64_t rows = d.rows_per_task > 0 ? d.rows_per_task : 512;

@@ -23,6 +23,14 @@ def test_builtin_tiles(nx, planes, rows, tile):
     assert describe(desc(nx, planes, rows))["tile"] == tile
 
 
+@pytest.mark.parametrize("kernel,support,planes,rows,tile", [
+    (GAUSS_HI_PRECISION, 9, 2, 4095, (64, 64)), (GAUSS_HI_PRECISION, 9, 2, 4096, (64, 32)),
+    (GAUSS_HI_PRECISION, 15, 17, 10 ** 6, (64, 64)), (GAUSS_HI_PRECISION, 15, 16, 10 ** 6, (64, 32)),
+    (GAUSS_HI_PRECISION, 7, 2, 700, (64, 32)), (KAISERBESSEL, 9, 2, 700, (64, 32))])
+def test_builtin_tile_of_a_dear_footprint(kernel, support, planes, rows, tile):
+    assert describe(desc(256, planes, rows, support=support, kernel=kernel))["tile"] == tile
+
+
 def test_named_shapes_stay():
     d = desc(8192, 8, 100_000, tile_u=32, tile_v=64, rows_per_task=777, footprint_unroll=11)
     s = describe(d)
