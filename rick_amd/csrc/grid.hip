@@ -309,8 +309,8 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
 }
 
 // Scan of the histogram: grids of up to 1024 buckets in one workgroup, larger
-// ones in three kernels, per-block sums, their scan and the downsweep that emits
-// offsets and tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
+// ones in two or three kernels, per-block sums, their scan from 16384 buckets on, and
+// the downsweep that emits offsets and tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
 // the accumulation tasks of three lengths.  The task array holds the long tasks
 // first (more than g.rmax / 2 records), then the middle ones (more than
 // g.rmax / 8), then the short ones, so that no long task starts when the others
@@ -398,6 +398,7 @@ k_scan_reduce(GridGeom g, const uint32_t *__restrict__ counts, uint32_t *__restr
 
 // Exclusive scan of each quantity's block sums in place, its total behind them all: one
 // workgroup per quantity.
+constexpr uint32_t kOwnSums = 16;     // block sums that a workgroup of k_scan_down adds up
 constexpr int kTopThreads = 1024;
 __global__ void __launch_bounds__(kTopThreads)
 k_scan_top(uint32_t *__restrict__ blocksum, uint32_t nscan)
@@ -455,10 +456,13 @@ __device__ __forceinline__ void split_tasks(uint4 *__restrict__ tasks, uint32_t 
 // Offsets, cursors, tasks and split list of 1024 buckets per workgroup.  The
 // counters it has read and the row flags are cleared on the way: the counters
 // for the next call's count, the flags for this call's tile kernel.  With nscan == 1
-// this is the whole scan; otherwise k_scan_top has scanned the block sums.  (Each
-// workgroup adding up all of them itself saves that launch, but its reads grow with the
-// square of the buckets: scan of 16 M buckets 1114 us against 157, of 1 M 34 and 27, of
-// 16384 18.4 and 17.5.)
+// this is the whole scan; with up to kOwnSums each workgroup adds up the block sums
+// itself, which saves a launch (3.5 us of the 26 that 100 rows take where the host is the
+// slower side; 0.9 us more on the GPU); with more, k_scan_top has scanned them: the reads
+// of adding them up grow with the square of the buckets (scan of 16 M buckets 1114 us
+// against 157, of 1 M 34 and 27).
+// ONE: nscan == 1.
+template <bool ONE>
 __global__ void __launch_bounds__(kThreads)
 k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restrict__ blocksum,
             uint32_t nscan, uint32_t *__restrict__ offsets, uint32_t *__restrict__ cursor,
@@ -498,12 +502,32 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
         if (lane == 63) wtot[a][wave] = x[a];
     }
     if (threadIdx.x == 0) nbig = 0u;
-    if (threadIdx.x < kScanQ) {
-        before[threadIdx.x] = nscan > 1 ? blocksum[(size_t)threadIdx.x * nscan + blockIdx.x] : 0u;
-        if (nscan > 1) total[threadIdx.x] = blocksum[(size_t)kScanQ * nscan + threadIdx.x];
+    if constexpr (ONE) {
+        (void)blocksum;
+    } else if (nscan > kOwnSums) {
+        if (threadIdx.x < kScanQ) {
+            before[threadIdx.x] = blocksum[(size_t)threadIdx.x * nscan + blockIdx.x];
+            total[threadIdx.x] = blocksum[(size_t)kScanQ * nscan + threadIdx.x];
+        }
+    } else {
+        // kOwnSums lanes per quantity.
+        static_assert(kOwnSums == 16 && kScanQ * kOwnSums <= NT, "lanes of the block sums");
+        const uint32_t a = threadIdx.x / kOwnSums, i = threadIdx.x % kOwnSums;
+        if (a < kScanQ) {
+            uint32_t all = i < nscan ? blocksum[a * nscan + i] : 0u;
+            uint32_t pre = i < blockIdx.x ? all : 0u;
+            for (int d = kOwnSums / 2; d > 0; d >>= 1) {
+                pre += __shfl_xor(pre, d);
+                all += __shfl_xor(all, d);
+            }
+            if (i == 0) {
+                before[a] = pre;
+                total[a] = all;
+            }
+        }
     }
     __syncthreads();
-    if (nscan == 1) {
+    if constexpr (ONE) {
         if (threadIdx.x < kScanQ) {
             uint32_t all = 0;
             for (int i = 0; i < NW; ++i) all += wtot[threadIdx.x][i];
@@ -514,7 +538,7 @@ k_scan_down(GridGeom g, uint32_t *__restrict__ counts, const uint32_t *__restric
     uint32_t ex[kScanQ];
 #pragma unroll
     for (int a = 0; a < kScanQ; ++a) {
-        ex[a] = before[a] + x[a] - v[a];
+        ex[a] = (ONE ? 0u : before[a]) + x[a] - v[a];
         for (int i = 0; i < wave; ++i) ex[a] += wtot[a][i];
     }
     uint32_t ro = ex[kQRecords], so = ex[kQSplit], to[kLengths];
@@ -1940,15 +1964,16 @@ hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precisi
     const uint32_t rl_words = (uint32_t)(align_up((size_t)g.planes * g.ny, 256) / sizeof(uint32_t));
     uint32_t *rl = reinterpret_cast<uint32_t *>(w.rowlive);
     if (w.nscan == 1) {
-        hipLaunchKernelGGL(k_scan_down, dim3(1), dim3(kThreads), 0, s, g, w.counts, w.blocksum,
+        hipLaunchKernelGGL(k_scan_down<true>, dim3(1), dim3(kThreads), 0, s, g, w.counts, w.blocksum,
                            1u, w.offsets, w.cursor, w.tasks, w.task_cap, w.split_list,
                            w.split_cap, w.meta, rl, rl_words, zero);
     } else {
         hipLaunchKernelGGL(k_scan_reduce, dim3(w.nscan), dim3(kThreads), 0, s, g, w.counts,
                            w.blocksum, w.nscan, zero);
-        hipLaunchKernelGGL(k_scan_top, dim3(kScanQ), dim3(kTopThreads), 0, s, w.blocksum,
-                           w.nscan);
-        hipLaunchKernelGGL(k_scan_down, dim3(w.nscan), dim3(kThreads), 0, s, g,
+        if (w.nscan > kOwnSums)
+            hipLaunchKernelGGL(k_scan_top, dim3(kScanQ), dim3(kTopThreads), 0, s, w.blocksum,
+                               w.nscan);
+        hipLaunchKernelGGL(k_scan_down<false>, dim3(w.nscan), dim3(kThreads), 0, s, g,
                            w.counts, w.blocksum, w.nscan, w.offsets, w.cursor, w.tasks,
                            w.task_cap, w.split_list, w.split_cap, w.meta, rl, rl_words, zero);
     }

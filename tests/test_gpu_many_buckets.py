@@ -1,5 +1,6 @@
-"""Grids of very many tiles: the scan's block sums at the edges of k_scan_top's chunks
-(4096 blocks of 1024 buckets), against the CPU oracle at the suite's 1e-6 for FP32."""
+"""Grids of very many tiles: the scan's block sums on either side of 16 blocks, from which
+on a kernel scans them, and at the edges of that kernel's chunks (4096 blocks of 1024
+buckets), against the CPU oracle at the suite's 1e-6 for FP32."""
 import numpy as np
 import pytest
 import torch
@@ -11,8 +12,8 @@ from rick_amd import FP32, KAISERBESSEL, Plan
 pytestmark = pytest.mark.gpu
 
 
-# Planes of 4 x 4 cells are one tile each: 2, 3, 4096, 4097 and 8193 scan blocks.
-@pytest.mark.parametrize("planes", [1025, 2049, 4096 * 1024, 4096 * 1024 + 1, 8192 * 1024 + 3])
+# Planes of 4 x 4 cells are one tile each: 2, 3, 16, 17, 4096, 4097 and 8193 scan blocks.
+@pytest.mark.parametrize("planes", [1025, 2049, 16 * 1024, 16 * 1024 + 1, 4096 * 1024, 4096 * 1024 + 1, 8192 * 1024 + 3])
 def test_grids_of_many_tiles_match_oracle(planes):
     nx, n = 4, 30_000
     print(f"case many tiles planes={planes}", flush=True)
