@@ -792,11 +792,13 @@ __device__ __forceinline__ void zero_split_tiles(const GridGeom &g, uint32_t fir
 
 // VMODE: 0 = per-row scalar reads, 1 = one 16-byte read per row (F*P = 4),
 // 2 or 4 = wave-cooperative reads with VMODE lanes per row (F*P = 8 or 16),
-// 3 or 5 = wave-cooperative reads of any larger multiple of 4, 5 (from 24 values on)
-// ranking a wave's few rows inside the grid and with the registers of one workgroup
-// per CU; the 16-byte modes need 16-byte aligned visibility arrays.  3 and 5: 2.9 M
-// rows of 64 values 474 and 420 us, 2.8 M rows of 24 values, 84 % outside the grid,
-// 51 and 37; 1.2 M rows of 12 values, one round of loads a row, 47 and 55.
+// 5 = wave-cooperative reads of any other multiple of 4 above 8, ranking a wave's few
+// rows inside the grid and with the registers of one workgroup per CU, 3 = the same
+// without the rank and with two workgroups per CU, for the FP64 records of 12 values, whose
+// one round of loads a row leaves room for them; the 16-byte modes need 16-byte aligned
+// visibility arrays.  3 and 5, 1.2 M rows: 12 values FP64 97 and 111 us (a fifth of them
+// inside the grid 23 and 20), FP32, whose registers spill in 3, 117 and 114; 20 values FP64
+// 208 and 156, FP32 229 and 159; 2.9 M rows of 64 values 474 and 420.
 template <int PREC, int VMODE, bool BATCH>
 __global__ void __launch_bounds__(kScatterThreads, VMODE == 5 ? 4 : 8)
 k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__restrict__ uu_all,
@@ -1984,7 +1986,12 @@ hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precisi
         const bool vec4 = (FP % 4u) == 0u &&
                           ((reinterpret_cast<uintptr_t>(vr) | reinterpret_cast<uintptr_t>(vi)) &
                            15u) == 0u;   // batch: vr = vi = null, the caller checked the jobs
-        const int mode = !vec4 ? 0 : FP == 4u ? 1 : FP == 8u ? 2 : FP == 16u ? 4 : FP < 24u ? 3 : 5;
+        const int mode = !vec4       ? 0
+                         : FP == 4u  ? 1
+                         : FP == 8u  ? 2
+                         : FP == 16u ? 4
+                         : FP == 12u && precision == RICK_FP64 ? 3
+                                                               : 5;
         // Overwritten grids: the split buckets' tiles start at zero (FP32: for
         // the non-finite fallback; its finite sums go through integer tiles).
         const uint32_t zblk = accumulate ? 0u : std::min(w.split_cap, kZeroBlocks);
@@ -2002,7 +2009,7 @@ hipError_t launch_grid(const GridGeom &plan_geom, const GridWork &w, int precisi
     switch (mode) {                                                                           \
     case 5: RICK_SCATTER(PR, 5); break;                                                       \
     case 4: RICK_SCATTER(PR, 4); break;                                                       \
-    case 3: RICK_SCATTER(PR, 3); break;                                                       \
+    case 3: RICK_SCATTER(PR, PR == RICK_FP64 ? 3 : 5); break;                                 \
     case 2: RICK_SCATTER(PR, 2); break;                                                       \
     case 1: RICK_SCATTER(PR, 1); break;                                                       \
     default: RICK_SCATTER(PR, 0); break;                                                      \
