@@ -220,7 +220,7 @@ def cpu_baseline(ds_host_fn, cfg, target_s, host_grid_fn):
     t_grid_all = cfg.n_vis / rate
     return {"value": rate, "unit": "vis/s", "cores": threads, "kind": kind,
             "sample": f"{n} of {cfg.n_rows} rows ({n * FP} vis, time-major block from the middle "
-                      f"of the observation) gridded by the reference's wstack() (KAISERBESSEL, "
+                      f"of the observation) gridded by the {'reference' if kind == 'reference' else 'oracle'}'s wstack() (KAISERBESSEL, "
                       f"support {cfg.support}) into the full {nx}^2 x {cfg.planes}-plane FP64 "
                       f"grid with {threads} OpenMP threads in {t:.2f} s; {n1} rows with 1 thread "
                       f"in {t1:.2f} s; FFT and phase timed on {k} of {cfg.planes} planes and "

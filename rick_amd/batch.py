@@ -143,8 +143,8 @@ class FusedBatch:
     one fused column/phase pass writing every job's image.  Groups are dealt
     to `n_streams` streams, largest first, so one group's LDS-bound
     accumulation overlaps another's memory-bound transforms (96-job mix,
-    FP32: 28.5 ms on one stream, 23.1 ms on four; eight are no better, the
-    device exposing four hardware queues per process), and the whole batch
+    FP32: 20.3 ms on one stream, 18.6 ms on four, 18.5 on eight, the device
+    exposing four hardware queues per process), and the whole batch
     is one HIP graph replay after capture()."""
 
     def __init__(self, datasets, precision, device="cuda:0", n_streams=4, tile=(0, 0),

@@ -35,14 +35,13 @@ namespace {
 using namespace fftk;
 
 constexpr int kGenThreads = 512;      // most threads of a workgroup
-constexpr int kGenValues = 16;        // most complex values a thread holds
+constexpr int kGenValues = 16;        // most complex values a thread holds (its largest radix)
+constexpr int kPhaseValues = 10;      // ... in the fused phase pass
 constexpr int kGenElems = 4096;       // longest line of one pass
 constexpr int kGenDirectCols = 256;   // longest column transform done in one pass
 constexpr size_t kBlueChunk = size_t(1) << 25;   // Bluestein scratch: elements per chunk
 
 constexpr int kGenLdsBytes = 80 * 1024;          // dynamic LDS of a workgroup, at most
-
-constexpr int kPhaseValues = 10;      // the same in the fused phase pass (its largest radix)
 
 // Butterflies of radix R a thread of V values takes in one pass.
 __host__ __device__ constexpr int gen_bpt(int R, int V) { return V / R > 1 ? V / R : 1; }
@@ -423,7 +422,7 @@ __device__ __forceinline__ void gen_lines_of(const GenCtx<T> &c, const GenPassDe
 // 243 and 2 when each thread held up to 4096 / R / 256 butterflies), and all
 // index divisions are by constants formed on the host.  Bound by memory now:
 // column pass A of 8 planes of 3000^2 FP64 moves 2.3 GB in 0.51 ms where half
-// its rows are live, rows 0.35 ms over the live ones (before, dense: 2.0 ms the
+// its rows are live, rows 0.37 ms over the live ones (before, dense: 2.0 ms the
 // columns, 1.33 ms the rows).  HARD: the instance with radices 11 and 13, whose
 // registers the lengths without them do not pay for.
 template <typename T, bool HARD>
@@ -482,8 +481,8 @@ k_fft_gen(GenPassDesc gp, GenAddr a, const C2<T> *__restrict__ tw, const C2<T> *
 // one: each plane is read once, and not written and read again.  A thread holds 10
 // values (with 16, and their sums, 776 registers spill), so radices above 10 are not
 // used here.  Bound by the vector units now, half of it the sines, at 2 waves per
-// SIMD: both passes of 8 planes of 3000^2 736 -> 650 us, of 10 of 1920 x 2560 459 ->
-// 370, of 16 of 960 x 3000 473 -> 383, of 30 of 2400 x 1280 793 -> 800.
+// SIMD: last pass and phase of 8 planes of 3000^2 752 -> 663 us, of 10 of 1920 x 2560
+// 462 -> 370, of 16 of 960 x 3000 480 -> 400, of 30 of 2400 x 1280 819 -> 811.
 __global__ void __launch_bounds__(kGenThreads)
 k_fft_gen_phase(GenPassDesc gp, GenAddr a, const C2<double> *__restrict__ tw,
                 const C2<double> *in, PhaseGeom pg, double *ore, double *oim)
@@ -743,9 +742,10 @@ constexpr int gen_elems() { return sizeof(T) == 8 ? 4096 : 8192; }
 
 // Lines of a workgroup of the fused last column pass, or 0 where the pass is not
 // used: it walks the planes one after another, so images that fill the chip less
-// than four times over are faster apart (1000^2 x 8 85 us, fused 111; 1500^2 x 8 197
-// and 189; 2000^2 x 8 331 and 281).  FP32 is too, the plain pass having six waves per
-// SIMD (3000^2 x 8: 375 us, fused 463).
+// than four times over are faster apart (1000^2 x 8 88 us, fused 119; 1500^2 x 8 200
+// and 218), the larger among them not always (2000^2 x 8 347 and 291).  FP32 is faster
+// apart too, the plain pass having six waves per SIMD (3000^2 x 8, before every twiddle
+// came from the table: 375 us, fused 463; apart now 411).
 int gen_phase_lines(const GenPassDesc &gp, int nl, int sets)
 {
     if (gp.np == 0) return 0;

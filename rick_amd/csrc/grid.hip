@@ -8,25 +8,30 @@
 //
 //   k_count      rows -> buckets (bucket = w-plane x TUxTV grid tile whose core
 //                the row's footprint touches; at most 4 per row).  Each
-//                workgroup aggregates the keys of its 16384 rows in an LDS hash
-//                table and adds one count per distinct key to the global
-//                histogram: device-scope atomics are slow on this chip (its
-//                eight L2 slices are not coherent with each other), and 16384
-//                consecutive rows touch a few thousand distinct buckets.
-//   k_scan_*     exclusive scans of the histogram -> bucket offsets, the task list (a task is <= rmax records of one
-//                bucket, or a zero task), the list of split buckets.
+//                workgroup aggregates the keys of its 1024, 4096 or 16384 rows
+//                in an LDS hash table and adds one count per distinct key to
+//                the global histogram: device-scope atomics are slow on this
+//                chip (its eight L2 slices are not coherent with each other),
+//                and 16384 consecutive rows touch a few thousand distinct
+//                buckets.
+//   k_scan_*     exclusive scans of the histogram -> bucket offsets, the task
+//                list (a task is <= rmax records of one bucket, or a zero
+//                task), the list of split buckets; they leave the counters at
+//                zero for the next call.
 //   k_scatter    forms per row S = sum_{f,p} fl32(weight*vis) (NaN real parts
-//                skipped, w-stacking.cu:517) and writes a record {pos_u,
+//                skipped, w-stacking.cu:517; rows of 12 and of more than 16
+//                values in four partial sums) and writes a record {pos_u,
 //                pos_v, S} to each of its buckets; slots come from one
 //                returning global atomic per distinct key per 2048-row block.
 //                Its last workgroups clear the tiles of split buckets
 //                (overwrite mode).
 //   k_tile       one workgroup per task: accumulates its records into an FP64
-//                LDS tile (one lane per record, LDS atomics), then writes
+//                LDS tile (one lane per record, LDS atomics; long tasks by
+//                footprint class), then writes
 //                the tile once with plain, coalesced stores; tasks of split
 //                buckets flush with HBM atomics instead.  In overwrite mode
 //                each empty bucket gets a zero task that clears its tile; zero
-//                tasks sit between the accumulation tasks in bucket order, so
+//                tasks sit between the accumulation tasks, so
 //                the bandwidth-bound clearing shares the launch with the
 //                LDS-bound accumulation.  Every grid cell is written exactly
 //                once, so no memset of the grid is needed.  For the image
@@ -34,9 +39,10 @@
 //                flags each grid row it writes a non-zero cell to, so the FFT
 //                skips the rest.
 //
-// The per-cell weight K[jKer]*K[kKer] is bitwise the reference's; the per-cell
-// value S*c differs from the reference's sum_{f,p} fl(fl32(w*v)*c) only by
-// rounding order (identical when F*P == 1).
+// Record by record the per-cell weight K[jKer]*K[kKer] is bitwise the reference's
+// and the per-cell value S*c differs from the reference's sum_{f,p}
+// fl(fl32(w*v)*c) only by rounding order (identical when F*P == 1).  By class the
+// table entries are the same, but the sum of S*K[jKer] is multiplied by K[kKer].
 #include "rick_internal.h"
 
 #include <algorithm>
@@ -309,9 +315,10 @@ k_count(GridGeom g, uint32_t n_all, const double *__restrict__ uu_all,
 }
 
 // Scan of the histogram: grids of up to 1024 buckets in one workgroup, larger
-// ones in two or three kernels, per-block sums, their scan from 16384 buckets on, and
-// the downsweep that emits offsets and tasks.  Scanned are records, split buckets, non-empty buckets, zero tasks and
-// the accumulation tasks of three lengths.  The task array holds the long tasks
+// ones in two or three kernels, per-block sums, their scan above 16384 buckets, and
+// the downsweep that emits offsets and tasks.  Scanned are records, split buckets,
+// non-empty buckets, zero tasks and the accumulation tasks of three lengths.  The
+// task array holds the long tasks
 // first (more than g.rmax / 2 records), then the middle ones (more than
 // g.rmax / 8), then the short ones, so that no long task starts when the others
 // are done, and the zero tasks last; the tile kernel interleaves accumulation
@@ -796,9 +803,9 @@ __device__ __forceinline__ void zero_split_tiles(const GridGeom &g, uint32_t fir
 // rows inside the grid and with the registers of one workgroup per CU, 3 = the same
 // without the rank and with two workgroups per CU, for the FP64 records of 12 values, whose
 // one round of loads a row leaves room for them; the 16-byte modes need 16-byte aligned
-// visibility arrays.  3 and 5, 1.2 M rows: 12 values FP64 97 and 111 us (a fifth of them
-// inside the grid 23 and 20), FP32, whose registers spill in 3, 117 and 114; 20 values FP64
-// 208 and 156, FP32 229 and 159; 2.9 M rows of 64 values 474 and 420.
+// visibility arrays.  3 (its registers spill, 84 and 100 bytes a lane) and 5, 1.2 M rows: 12
+// values FP64 97 and 111 us (0.2 M, a fifth of them inside the grid: 23 and 20), FP32 117
+// and 114; 20 values FP64 208 and 156, FP32 229 and 159; 2.9 M rows of 64 values 474 and 420.
 template <int PREC, int VMODE, bool BATCH>
 __global__ void __launch_bounds__(kScatterThreads, VMODE == 5 ? 4 : 8)
 k_scatter(GridGeom g, uint32_t n_all, uint32_t F, uint32_t P, const double *__restrict__ uu_all,
